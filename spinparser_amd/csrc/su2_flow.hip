@@ -185,8 +185,10 @@ struct FlowDev {
   float2 *G32;  // FP32 shadow of G (mixed precision), null otherwise
   double *v2, *dv2;
   const double *mesh;
-  const int *site_rid, *inv_rid, *ovl_off, *ovl_rid1, *ovl_rid2, *range_fwd, *range_inv, *corr_rid;
+  const int *site_rid, *inv_rid, *ovl_off, *range_fwd, *range_inv, *corr_rid;
   const unsigned short *ovl_idx;  // per overlap entry: rid1 * Lp + rid2 (Lp = L rounded up to a multiple of 4)
+  const unsigned *plan_ent;       // overlap lists merged and dealt to the lanes of k_t (OverlapPlan)
+  const int *plan_lane, *plan_count;
   double *Wwp, *Wc;
   int *Wn;
   double *Cwp, *Cw;
@@ -197,7 +199,9 @@ struct FlowDev {
                // binary exponent of G written since the last plan, [6] planned S
   int nw, L, R, B, Rb, emax, nb, slots, precision, euler;
   int nt;  // threads per workgroup of the dGamma kernel
+  int asym;  // some bond is not equivalent to its reverse (site_rid != inv_rid)
   long long nf, item_base, nv;
+  long long su_base, t_base;  // first workgroup of the flow in its launch of k_su / k_t
   unsigned g_bytes, g32_bytes;
   double spin, cut, step;
   int pad_index;  // host bookkeeping: position of the flow in the caller's array
@@ -218,11 +222,18 @@ __device__ __forceinline__ int flow_of(const FlowDev *__restrict__ fl, int nflow
 // W tables: workgroup x < nw -> channel list with propagators; x == nw ->
 // plain correlation list (corr_only: that one alone, launched as workgroup 0).
 // flags[1] is raised if a list overflows its capacity.  Dynamic LDS: the mesh.
+// Workgroups past x == nw clear dG for the kernels that add to it (k_su), so
+// that this needs no launch of its own.
 __global__ __launch_bounds__(64) void k_weights(const FlowDev *__restrict__ fl, int corr_only) {
   extern __shared__ double s_wmesh[];
   const FlowDev &F = fl[blockIdx.y];
   const int x = corr_only ? F.nw : (int)blockIdx.x;
-  if (x > F.nw) return;
+  if (x > F.nw) {
+    if (!F.plan_ent || F.precision != SP_PRECISION_FP64) return;
+    const size_t n = (size_t)F.nv, stride = (size_t)(gridDim.x - F.nw - 1) * 64;
+    for (size_t i = (size_t)(x - F.nw - 1) * 64 + threadIdx.x; i < n; i += stride) F.dG[i] = make_double2(0.0, 0.0);
+    return;
+  }
   weight_tables_wave(x, F.mesh, F.nw, F.cut, F.v2, F.dv2, F.Wwp, F.Wc, F.Wn, F.Cwp, F.Cw, F.Cn, F.emax, F.flags + 1,
                      s_wmesh);
 }
@@ -269,8 +280,11 @@ __global__ __launch_bounds__(256) void k_dsigma(const FlowDev *__restrict__ fl) 
   }
 }
 
+#include "su2_rhs.h"
+
 // ---------------------------------------------------------------------------
-// dGamma/dLambda
+// dGamma/dLambda, general kernel: the mixed form, and lattices of more than
+// kMaxRhsL sites
 // ---------------------------------------------------------------------------
 // LDS carve-up (bytes), computed identically on host and device.  Lp = L
 // rounded up to a multiple of 4 (register tiles of the lattice-bubble update); vs =
@@ -1245,13 +1259,22 @@ size_t lds_of(const FlowDev &f) {
 // the occupancy of a larger one.  Launch class = precision x workgroup size x
 // LDS level (within 160 KB / resident_blocks, within kLdsBudget, above); a
 // batch issues one launch per class.
-constexpr int kLaunchClasses = 12;
+// FP64 flows of up to kMaxRhsL sites run the wave kernels of su2_rhs.h, whose
+// class is the compiled lane shapes of k_su and k_t.
+constexpr int kLdsClasses = 12;
+constexpr int kLaunchClasses = kLdsClasses + 3 * 4 * 2;
+int t_index(const TShape &t) { return t.ft == 2 ? 3 : (t.ft == 0 ? 0 : 1 + t.ht); }
+bool wave_form(const FlowDev &f) { return f.precision == SP_PRECISION_FP64 && f.plan_ent; }
 int lds_level(const FlowDev &f) {
   const int vs = f.precision == SP_PRECISION_MIXED ? 4 : 8;
   const size_t lds = lds_of(f);
   return lds <= (size_t)160 * 1024 / resident_blocks(vs, f.nt) ? 0 : (lds <= kLdsBudget ? 1 : 2);
 }
 int launch_class(const FlowDev &f) {
+  if (wave_form(f)) {
+    const TShape t = t_shape(f.L);
+    return kLdsClasses + ((su_shape(f.L).rho - 1) * 4 + t_index(t)) * 2 + f.asym;
+  }
   return ((f.precision == SP_PRECISION_MIXED ? 2 : 0) + (f.nt == kSmallThreads ? 1 : 0)) * 3 + lds_level(f);
 }
 
@@ -1271,6 +1294,48 @@ Geometry geometry(const FlowDev *h, int n) {
   return g;
 }
 
+// workgroups of a flow in the wave kernels
+long long su_flow_blocks(const FlowDev &f) { return (su_units(f.nw) + kRhsWaves - 1) / kRhsWaves; }
+long long t_flow_blocks(const FlowDev &f) { return (f.nf + kRhsWaves - 1) / kRhsWaves; }
+
+template <int RHO>
+void launch_su(bool asym, dim3 grid, size_t lds, hipStream_t st, const FlowDev *d, int n, long long blocks) {
+  if (asym) hipLaunchKernelGGL((k_su<RHO, true>), grid, dim3(64 * kRhsWaves), lds, st, d, n, blocks);
+  else hipLaunchKernelGGL((k_su<RHO, false>), grid, dim3(64 * kRhsWaves), lds, st, d, n, blocks);
+}
+template <int FT, int HT>
+void launch_t(bool asym, dim3 grid, size_t lds, hipStream_t st, const FlowDev *d, int n, long long blocks) {
+  if (asym) hipLaunchKernelGGL((k_t<FT, HT, true>), grid, dim3(64 * kRhsWaves), lds, st, d, n, blocks);
+  else hipLaunchKernelGGL((k_t<FT, HT, false>), grid, dim3(64 * kRhsWaves), lds, st, d, n, blocks);
+}
+
+// dGamma of n flows of one wave class
+hipError_t launch_wave_form(hipStream_t st, const FlowDev *d, const FlowDev *h, int n, long long su_blocks,
+                            long long t_blocks) {
+  size_t su_lds = 0, t_lds = 0;
+  for (int i = 0; i < n; ++i) {
+    const size_t mesh = (size_t)(h[i].nw * 8 + 15) & ~size_t(15);
+    su_lds = std::max(su_lds, mesh + (size_t)kRhsWaves * kSuWaveBytes);
+    t_lds = std::max(t_lds, mesh + (size_t)kRhsWaves * t_wave_bytes(h[i].L));
+  }
+  auto grid = [](long long blocks) {
+    return dim3((unsigned)((blocks + 8 * kChunk - 1) / (8 * kChunk) * 8 * kChunk));
+  };
+  const bool asym = h[0].asym != 0;
+  switch (su_shape(h[0].L).rho) {
+    case 1: launch_su<1>(asym, grid(su_blocks), su_lds, st, d, n, su_blocks); break;
+    case 2: launch_su<2>(asym, grid(su_blocks), su_lds, st, d, n, su_blocks); break;
+    default: launch_su<3>(asym, grid(su_blocks), su_lds, st, d, n, su_blocks); break;
+  }
+  switch (t_index(t_shape(h[0].L))) {
+    case 0: launch_t<0, 1>(asym, grid(t_blocks), t_lds, st, d, n, t_blocks); break;
+    case 1: launch_t<1, 0>(asym, grid(t_blocks), t_lds, st, d, n, t_blocks); break;
+    case 2: launch_t<1, 1>(asym, grid(t_blocks), t_lds, st, d, n, t_blocks); break;
+    default: launch_t<2, 0>(asym, grid(t_blocks), t_lds, st, d, n, t_blocks); break;
+  }
+  return hipGetLastError();
+}
+
 // dSigma, weight tables and dGamma for n flows; the flows come ordered by
 // launch_class and h[i].item_base is relative to the first flow of its class.
 hipError_t launch_compute(hipStream_t st, const FlowDev *d, const FlowDev *h, int n, sp_ctx *prof) {
@@ -1281,7 +1346,10 @@ hipError_t launch_compute(hipStream_t st, const FlowDev *d, const FlowDev *h, in
   }
   {
     ProfScope ps(prof, 2);
-    hipLaunchKernelGGL(k_weights, dim3(geo.maxnw + 1, n), dim3(64), geo.maxnw * sizeof(double), st, d, 0);
+    bool clear = false;
+    for (int i = 0; i < n; ++i) clear = clear || wave_form(h[i]);
+    const int clear_blocks = clear ? (int)std::min<long long>((geo.maxnv + 255) / 256, 4096) : 0;
+    hipLaunchKernelGGL(k_weights, dim3(geo.maxnw + 1 + clear_blocks, n), dim3(64), geo.maxnw * sizeof(double), st, d, 0);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -1293,10 +1361,19 @@ hipError_t launch_compute(hipStream_t st, const FlowDev *d, const FlowDev *h, in
     int i1 = i0;
     long long total = 0;
     size_t lds = 0;
+    long long su_blocks = 0, t_blocks = 0;
     while (i1 < n && launch_class(h[i1]) == cls) {
       total += h[i1].nf;
       lds = std::max(lds, lds_of(h[i1]));
+      su_blocks += su_flow_blocks(h[i1]);
+      t_blocks += t_flow_blocks(h[i1]);
       ++i1;
+    }
+    if (wave_form(h[i0])) {
+      e = launch_wave_form(st, d + i0, h + i0, i1 - i0, su_blocks, t_blocks);
+      if (e != hipSuccess) return e;
+      i0 = i1;
+      continue;
     }
     {
       const long long per_xcd = 0;  // unused by the chunked mapping
@@ -1314,9 +1391,6 @@ hipError_t launch_compute(hipStream_t st, const FlowDev *d, const FlowDev *h, in
                            i1 - i0, total, per_xcd);
       else if (mixed)
         hipLaunchKernelGGL((k_dgamma<true, kThreads, SPFRG_MIN_BLOCKS>), dim3(grid), dim3(nt), lds, st, d + i0,
-                           i1 - i0, total, per_xcd);
-      else if (nt == kSmallThreads)
-        hipLaunchKernelGGL((k_dgamma<false, kSmallThreads, SPFRG_MIN_BLOCKS>), dim3(grid), dim3(nt), lds, st, d + i0,
                            i1 - i0, total, per_xcd);
       else
         hipLaunchKernelGGL((k_dgamma<false, kThreads, SPFRG_MIN_BLOCKS>), dim3(grid), dim3(nt), lds, st, d + i0,
@@ -1387,8 +1461,10 @@ int sp_ctx_footprint(const sp_su2_problem *p, long long *bytes) {
   b += 3LL * p->nw * 8;                                          // Sigma, dSigma, mesh
   b += 2 * (long long)p->nw * emax * 8 + 2 * emax * 8 + (p->nw + 1) * 4;  // weight tables
   b += emax * p->L * 16 + 2LL * p->B * p->Rb * 8 + 32;                   // correlation scratch / output, flags
-  b += 4LL * (3 * p->L + 1 + 2 * (p->ovl_off ? p->ovl_off[p->L] : 0) + 2 * p->R + p->B * p->Rb);
+  b += 4LL * (3 * p->L + 1 + 2 * p->R + p->B * p->Rb);
   b += 2LL * (p->ovl_off ? p->ovl_off[p->L] : 0);                         // packed overlap indices
+  if (p->L <= kMaxRhsL)  // overlap plan of k_t: at most two places per entry, and the lane tables
+    b += 8LL * (p->ovl_off ? p->ovl_off[p->L] : 0) + 4LL * (64 + 64 + p->L + 1);
   b += (long long)sizeof(FlowDev);
   *bytes = b;
   return SP_OK;
@@ -1435,12 +1511,12 @@ int sp_ctx_create(const sp_su2_problem *p, sp_ctx **out) {
   const size_t nv = (size_t)f.nv;
   const int emax = f.emax;
   double *mesh = nullptr;
-  int *site = nullptr, *inv = nullptr, *ooff = nullptr, *o1 = nullptr, *o2 = nullptr, *rf = nullptr, *ri = nullptr,
+  int *site = nullptr, *inv = nullptr, *ooff = nullptr, *rf = nullptr, *ri = nullptr,
       *corr = nullptr;
   unsigned short *oidx = nullptr;
   if ((rc = dalloc(ctx, &oidx, O))) return rc;
   if ((rc = dalloc(ctx, &mesh, f.nw)) || (rc = dalloc(ctx, &site, f.L)) || (rc = dalloc(ctx, &inv, f.L)) ||
-      (rc = dalloc(ctx, &ooff, f.L + 1)) || (rc = dalloc(ctx, &o1, O)) || (rc = dalloc(ctx, &o2, O)) ||
+      (rc = dalloc(ctx, &ooff, f.L + 1)) ||
       (rc = dalloc(ctx, &rf, f.R)) || (rc = dalloc(ctx, &ri, f.R)) || (rc = dalloc(ctx, &corr, (size_t)f.B * f.Rb)) ||
       (rc = dalloc(ctx, &f.G, nv)) || (rc = dalloc(ctx, &f.dG, nv)) || (rc = dalloc(ctx, &f.v2, f.nw)) ||
       (rc = dalloc(ctx, &f.dv2, f.nw)) || (rc = dalloc(ctx, &f.Wwp, (size_t)f.nw * emax)) ||
@@ -1467,8 +1543,6 @@ int sp_ctx_create(const sp_su2_problem *p, sp_ctx **out) {
   f.site_rid = site;
   f.inv_rid = inv;
   f.ovl_off = ooff;
-  f.ovl_rid1 = o1;
-  f.ovl_rid2 = o2;
   f.ovl_idx = oidx;
   f.range_fwd = rf;
   f.range_inv = ri;
@@ -1482,14 +1556,34 @@ int sp_ctx_create(const sp_su2_problem *p, sp_ctx **out) {
   SP_HIP(hipMemcpy(inv, p->inv_rid, f.L * 4, hipMemcpyHostToDevice));
   SP_HIP(hipMemcpy(ooff, p->ovl_off, (f.L + 1) * 4, hipMemcpyHostToDevice));
   if (O > 0) {
-    SP_HIP(hipMemcpy(o1, p->ovl_rid1, (size_t)O * 4, hipMemcpyHostToDevice));
-    SP_HIP(hipMemcpy(o2, p->ovl_rid2, (size_t)O * 4, hipMemcpyHostToDevice));
     // packed C-matrix index of every overlap entry (rid < L <= 64, so it fits 16 bits)
     const int Lp = (f.L + 3) & ~3;
     std::vector<unsigned short> idx(O);
     for (int i = 0; i < O; ++i) idx[i] = (unsigned short)(p->ovl_rid1[i] * Lp + p->ovl_rid2[i]);
     SP_HIP(hipMemcpy(oidx, idx.data(), (size_t)O * 2, hipMemcpyHostToDevice));
   }
+  if (f.L <= kMaxRhsL) {
+    OverlapPlan plan;
+    try { plan.build(f.L, p->ovl_off, p->ovl_rid1, p->ovl_rid2); } catch (...) { return fail(ctx, SP_ENOMEM, "host buffer"); }
+    // one table: lane_of (L + 1), count (64), entries
+    const size_t head = plan.lane_of.size() + plan.count.size();
+    std::vector<unsigned> table;
+    try {
+      table.assign(plan.lane_of.begin(), plan.lane_of.end());
+      table.insert(table.end(), plan.count.begin(), plan.count.end());
+      table.insert(table.end(), plan.ent.begin(), plan.ent.end());
+    } catch (...) { return fail(ctx, SP_ENOMEM, "host buffer"); }
+    unsigned *tab = nullptr;
+    if ((rc = dalloc(ctx, &tab, table.size()))) return rc;
+    SP_HIP(hipMemcpy(tab, table.data(), table.size() * 4, hipMemcpyHostToDevice));
+    const unsigned *ent = tab + head;
+    const int *lane = reinterpret_cast<const int *>(tab), *count = lane + plan.lane_of.size();
+    f.plan_ent = ent;
+    f.plan_lane = lane;
+    f.plan_count = count;
+  }
+  for (int r = 0; r < f.L; ++r)
+    if (p->site_rid[r] != p->inv_rid[r]) f.asym = 1;
   SP_HIP(hipMemcpy(rf, p->range_fwd, (size_t)f.R * 4, hipMemcpyHostToDevice));
   SP_HIP(hipMemcpy(ri, p->range_inv, (size_t)f.R * 4, hipMemcpyHostToDevice));
   SP_HIP(hipMemcpy(corr, p->corr_rid, (size_t)f.B * f.Rb * 4, hipMemcpyHostToDevice));
@@ -1506,8 +1600,6 @@ int sp_ctx_create(const sp_su2_problem *p, sp_ctx **out) {
   SP_HIP(hipFuncSetAttribute((const void *)k_dgamma<true, kThreads, SPFRG_MIN_BLOCKS>,
                              hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
   SP_HIP(hipFuncSetAttribute((const void *)k_dgamma<true, kThreads, SPFRG_MIN_BLOCKS_MIXED>,
-                             hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
-  SP_HIP(hipFuncSetAttribute((const void *)k_dgamma<false, kSmallThreads, SPFRG_MIN_BLOCKS>,
                              hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
   SP_HIP(hipFuncSetAttribute((const void *)k_dgamma<true, kSmallThreads, SPFRG_MIN_BLOCKS>,
                              hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
@@ -1826,16 +1918,20 @@ static int group_prepare(sp_group *grp, sp_ctx *const *ctxs, int n, size_t *out_
     grp->h_out = static_cast<double *>(q);
     grp->out_cap = need;
   }
-  long long base = 0;
+  long long base = 0, su_base = 0, t_base = 0;
   int prev = -1;
   for (int j = 0; j < n; ++j) {
     sp_ctx *c = ctxs[order[j]];
     SP_GHIP(hipStreamSynchronize(c->stream));
     c->list_cut = -1.0;  // the group's launches rebuild the flow's point lists
     FlowDev f = c->fd;
-    if (launch_class(f) != prev) { base = 0; prev = launch_class(f); }
+    if (launch_class(f) != prev) { base = su_base = t_base = 0; prev = launch_class(f); }
     f.item_base = base;
+    f.su_base = su_base;
+    f.t_base = t_base;
     base += f.nf;
+    su_base += su_flow_blocks(f);
+    t_base += t_flow_blocks(f);
     f.cut = c->cutoff;
     f.euler = 0;
     f.corr_out = grp->d_out + out_off[order[j]];
@@ -1933,13 +2029,16 @@ constexpr int kNoAllocDevices = 64;
 std::mutex g_noalloc_mu;
 unsigned char *g_noalloc_ptr[kNoAllocDevices] = {};  // device address of scratch, per device
 int g_noalloc_lds[kNoAllocDevices] = {};            // LDS limit per workgroup, per device
+OverlapPlan g_noalloc_overlap;                      // keeps its host buffers from call to call
 unsigned char g_noalloc_image[SP_NOALLOC_SCRATCH_BYTES];  // host image of the scratch contents
 
 struct NoAllocPlan {
-  size_t fd, flags, mesh, site, inv, ooff, o1, o2, oidx, rf, ri, wwp, wc, wn, cwp, cw, cn, total;
+  size_t fd, flags, mesh, site, inv, ooff, o1, o2, oidx, pent, plane, pcount, rf, ri, wwp, wc, wn, cwp, cw, cn, total;
 };
 
-NoAllocPlan noalloc_plan(const sp_su2_problem *p) {
+// contents of the scratch for the general dGamma kernel (wave null; its size
+// is what the documented limit is held against) or for the wave kernels
+NoAllocPlan noalloc_plan(const sp_su2_problem *p, const OverlapPlan *wave) {
   NoAllocPlan q{};
   size_t o = 0;
   auto take = [&](size_t bytes) {
@@ -1955,9 +2054,15 @@ NoAllocPlan noalloc_plan(const sp_su2_problem *p) {
   q.site = take((size_t)p->L * 4);
   q.inv = take((size_t)p->L * 4);
   q.ooff = take(((size_t)p->L + 1) * 4);
-  q.o1 = take(O * 4);
-  q.o2 = take(O * 4);
-  q.oidx = take(O * 2);
+  if (wave) {
+    q.pent = take(wave->ent.size() * 4);
+    q.plane = take(wave->lane_of.size() * 4);
+    q.pcount = take(wave->count.size() * 4);
+  } else {
+    q.o1 = take(O * 4);
+    q.o2 = take(O * 4);
+    q.oidx = take(O * 2);
+  }
   q.rf = take((size_t)p->R * 4);
   q.ri = take((size_t)p->R * 4);
   q.wwp = take((size_t)p->nw * emax * 8);
@@ -1980,8 +2085,6 @@ int noalloc_scratch(int dev, unsigned char **base, int *max_lds) {
     int lds = 0;
     if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) return SP_EHIP;
     if (hipFuncSetAttribute((const void *)k_dgamma<false, kThreads, SPFRG_MIN_BLOCKS>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess ||
-        hipFuncSetAttribute((const void *)k_dgamma<false, kSmallThreads, SPFRG_MIN_BLOCKS>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
       return SP_EHIP;
     g_noalloc_lds[dev] = lds;
@@ -2000,7 +2103,7 @@ extern "C" int sp_compute_step_noalloc(const sp_su2_problem *p, double cutoff, c
   if (check_problem(nullptr, p) != SP_OK) return SP_EARG;
   if (p->precision != SP_PRECISION_FP64) return SP_EARG;
   if (!d_v2 || !d_v4 || !d_dv2 || !d_dv4 || !std::isfinite(cutoff) || cutoff <= 0.0) return SP_EARG;
-  const NoAllocPlan q = noalloc_plan(p);
+  NoAllocPlan q = noalloc_plan(p, nullptr);
   if (q.total > (size_t)SP_NOALLOC_SCRATCH_BYTES) return SP_EARG;
   FlowDev f{};
   f.nw = p->nw;
@@ -2017,7 +2120,7 @@ extern "C" int sp_compute_step_noalloc(const sp_su2_problem *p, double cutoff, c
   f.g_bytes = (unsigned)(f.nv * 16);
   f.cut = cutoff;
   size_t lds = 0;
-  f.nt = dgamma_threads(f.L);
+  f.nt = kThreads;
   launch_shape(f.nw, f.L, 8, f.nt, f.slots, f.nb, lds);
   double mesh_d[256];
   for (int i = 0; i < f.nw; ++i) mesh_d[i] = (double)p->mesh[i];
@@ -2032,6 +2135,21 @@ extern "C" int sp_compute_step_noalloc(const sp_su2_problem *p, double cutoff, c
   int rc = noalloc_scratch(dev, &base, &max_lds);
   if (rc != SP_OK) return rc;
   if (lds > (size_t)max_lds) return SP_EARG;
+  // the wave kernels add to d_dv4 with FP64 atomics of the memory side, which
+  // ordinary device memory takes; any other buffer runs the general kernel
+  OverlapPlan &plan = g_noalloc_overlap;
+  bool wave = false;
+  if (f.L <= kMaxRhsL) {
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, d_dv4) == hipSuccess) wave = at.type == hipMemoryTypeDevice && !at.isManaged;
+    else (void)hipGetLastError();
+  }
+  if (wave) {
+    try { plan.build(f.L, p->ovl_off, p->ovl_rid1, p->ovl_rid2); } catch (...) { return SP_ENOMEM; }
+    const NoAllocPlan qw = noalloc_plan(p, &plan);
+    wave = qw.total <= (size_t)SP_NOALLOC_SCRATCH_BYTES;
+    if (wave) q = qw;
+  }
   // an earlier call on this stream may still read the scratch
   if (hipStreamSynchronize(st) != hipSuccess) return SP_EHIP;
 
@@ -2043,12 +2161,19 @@ extern "C" int sp_compute_step_noalloc(const sp_su2_problem *p, double cutoff, c
   std::memcpy(h + q.site, p->site_rid, (size_t)f.L * 4);
   std::memcpy(h + q.inv, p->inv_rid, (size_t)f.L * 4);
   std::memcpy(h + q.ooff, p->ovl_off, ((size_t)f.L + 1) * 4);
-  if (O > 0) {
-    std::memcpy(h + q.o1, p->ovl_rid1, (size_t)O * 4);
-    std::memcpy(h + q.o2, p->ovl_rid2, (size_t)O * 4);
+  if (wave) {
+    std::memcpy(h + q.pent, plan.ent.data(), plan.ent.size() * 4);
+    std::memcpy(h + q.plane, plan.lane_of.data(), plan.lane_of.size() * 4);
+    std::memcpy(h + q.pcount, plan.count.data(), plan.count.size() * 4);
+    f.plan_ent = reinterpret_cast<const unsigned *>(base + q.pent);
+    f.plan_lane = reinterpret_cast<const int *>(base + q.plane);
+    f.plan_count = reinterpret_cast<const int *>(base + q.pcount);
+  } else if (O > 0) {
     unsigned short *idx = reinterpret_cast<unsigned short *>(h + q.oidx);
     for (int i = 0; i < O; ++i) idx[i] = (unsigned short)(p->ovl_rid1[i] * Lp + p->ovl_rid2[i]);
   }
+  for (int r = 0; r < f.L; ++r)
+    if (p->site_rid[r] != p->inv_rid[r]) f.asym = 1;
   std::memcpy(h + q.rf, p->range_fwd, (size_t)f.R * 4);
   std::memcpy(h + q.ri, p->range_inv, (size_t)f.R * 4);
   f.G = reinterpret_cast<double2 *>(const_cast<double *>(d_v4));
@@ -2060,9 +2185,7 @@ extern "C" int sp_compute_step_noalloc(const sp_su2_problem *p, double cutoff, c
   f.site_rid = reinterpret_cast<const int *>(base + q.site);
   f.inv_rid = reinterpret_cast<const int *>(base + q.inv);
   f.ovl_off = reinterpret_cast<const int *>(base + q.ooff);
-  f.ovl_rid1 = reinterpret_cast<const int *>(base + q.o1);
-  f.ovl_rid2 = reinterpret_cast<const int *>(base + q.o2);
-  f.ovl_idx = reinterpret_cast<const unsigned short *>(base + q.oidx);
+  f.ovl_idx = wave ? nullptr : reinterpret_cast<const unsigned short *>(base + q.oidx);
   f.range_fwd = reinterpret_cast<const int *>(base + q.rf);
   f.range_inv = reinterpret_cast<const int *>(base + q.ri);
   f.corr_rid = nullptr;
