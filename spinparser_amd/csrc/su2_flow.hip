@@ -67,6 +67,7 @@
 
 #include "spfrg.h"
 #include "frg_common.h"
+#include "wave_rhs.h"
 
 namespace {
 
@@ -187,7 +188,7 @@ struct FlowDev {
   const double *mesh;
   const int *site_rid, *inv_rid, *ovl_off, *range_fwd, *range_inv, *corr_rid;
   const unsigned short *ovl_idx;  // per overlap entry: rid1 * Lp + rid2 (Lp = L rounded up to a multiple of 4)
-  const unsigned *plan_ent;       // overlap lists merged and dealt to the lanes of k_t (OverlapPlan)
+  const unsigned *plan_ent;       // overlap lists merged and dealt to the lanes of k_t (LanePlan)
   const int *plan_lane, *plan_count;
   double *Wwp, *Wc;
   int *Wn;
@@ -1464,7 +1465,7 @@ int sp_ctx_footprint(const sp_su2_problem *p, long long *bytes) {
   b += 4LL * (3 * p->L + 1 + 2 * p->R + p->B * p->Rb);
   b += 2LL * (p->ovl_off ? p->ovl_off[p->L] : 0);                         // packed overlap indices
   if (p->L <= kMaxRhsL)  // overlap plan of k_t: at most two places per entry, and the lane tables
-    b += 8LL * (p->ovl_off ? p->ovl_off[p->L] : 0) + 4LL * (64 + 64 + p->L + 1);
+    b += 8LL * (p->ovl_off ? p->ovl_off[p->L] : 0) + 4LL * (4 * 64 + 64 + p->L + 4);
   b += (long long)sizeof(FlowDev);
   *bytes = b;
   return SP_OK;
@@ -1563,14 +1564,15 @@ int sp_ctx_create(const sp_su2_problem *p, sp_ctx **out) {
     SP_HIP(hipMemcpy(oidx, idx.data(), (size_t)O * 2, hipMemcpyHostToDevice));
   }
   if (f.L <= kMaxRhsL) {
-    OverlapPlan plan;
-    try { plan.build(f.L, p->ovl_off, p->ovl_rid1, p->ovl_rid2); } catch (...) { return fail(ctx, SP_ENOMEM, "host buffer"); }
-    // one table: lane_of (L + 1), count (64), entries
-    const size_t head = plan.lane_of.size() + plan.count.size();
+    LanePlan plan;
+    try { build_overlap_plan(plan, f.L, p->ovl_off, p->ovl_rid1, p->ovl_rid2); } catch (...) { return fail(ctx, SP_ENOMEM, "host buffer"); }
+    // one table: lane_of (L + 1), count (64), entries (16-byte aligned)
+    const size_t head = (plan.lane_of.size() + plan.count.size() + 3) & ~size_t(3);
     std::vector<unsigned> table;
     try {
       table.assign(plan.lane_of.begin(), plan.lane_of.end());
       table.insert(table.end(), plan.count.begin(), plan.count.end());
+      table.resize(head, 0);
       table.insert(table.end(), plan.ent.begin(), plan.ent.end());
     } catch (...) { return fail(ctx, SP_ENOMEM, "host buffer"); }
     unsigned *tab = nullptr;
@@ -2029,7 +2031,7 @@ constexpr int kNoAllocDevices = 64;
 std::mutex g_noalloc_mu;
 unsigned char *g_noalloc_ptr[kNoAllocDevices] = {};  // device address of scratch, per device
 int g_noalloc_lds[kNoAllocDevices] = {};            // LDS limit per workgroup, per device
-OverlapPlan g_noalloc_overlap;                      // keeps its host buffers from call to call
+LanePlan g_noalloc_overlap;                         // keeps its host buffers from call to call
 unsigned char g_noalloc_image[SP_NOALLOC_SCRATCH_BYTES];  // host image of the scratch contents
 
 struct NoAllocPlan {
@@ -2038,7 +2040,7 @@ struct NoAllocPlan {
 
 // contents of the scratch for the general dGamma kernel (wave null; its size
 // is what the documented limit is held against) or for the wave kernels
-NoAllocPlan noalloc_plan(const sp_su2_problem *p, const OverlapPlan *wave) {
+NoAllocPlan noalloc_plan(const sp_su2_problem *p, const LanePlan *wave) {
   NoAllocPlan q{};
   size_t o = 0;
   auto take = [&](size_t bytes) {
@@ -2137,7 +2139,7 @@ extern "C" int sp_compute_step_noalloc(const sp_su2_problem *p, double cutoff, c
   if (lds > (size_t)max_lds) return SP_EARG;
   // the wave kernels add to d_dv4 with FP64 atomics of the memory side, which
   // ordinary device memory takes; any other buffer runs the general kernel
-  OverlapPlan &plan = g_noalloc_overlap;
+  LanePlan &plan = g_noalloc_overlap;
   bool wave = false;
   if (f.L <= kMaxRhsL) {
     hipPointerAttribute_t at{};
@@ -2145,7 +2147,7 @@ extern "C" int sp_compute_step_noalloc(const sp_su2_problem *p, double cutoff, c
     else (void)hipGetLastError();
   }
   if (wave) {
-    try { plan.build(f.L, p->ovl_off, p->ovl_rid1, p->ovl_rid2); } catch (...) { return SP_ENOMEM; }
+    try { build_overlap_plan(plan, f.L, p->ovl_off, p->ovl_rid1, p->ovl_rid2); } catch (...) { return SP_ENOMEM; }
     const NoAllocPlan qw = noalloc_plan(p, &plan);
     wave = qw.total <= (size_t)SP_NOALLOC_SCRATCH_BYTES;
     if (wave) q = qw;

@@ -43,53 +43,7 @@
 // 0.05: 3.0 -> 1.5 ms; square, 9 sites, 32 frequencies, whole flow 142 -> 87 ms.
 #pragma once
 
-constexpr int kRhsWaves = 4;    // waves (independent work units) per workgroup
-constexpr int kRhsPoints = 16;  // points described per production pass: 64 lanes, four per point
 constexpr int kMaxRhsL = 32;    // largest lattice of the T kernel's register tiles
-// byte offsets past every vertex (smaller than 2 GiB): buffer loads return 0.
-// Rows of points past the list, and sites past L; their sum stays below 2^32
-constexpr unsigned kNoRow = 0x80000000u, kNoSite = 0x7ffffff0u;
-
-// value of the other lane of an even/odd lane pair
-__device__ __forceinline__ int pair_swap(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true); }
-__device__ __forceinline__ double pair_swap(double v) {
-  int2 q;
-  __builtin_memcpy(&q, &v, 8);
-  q.x = pair_swap(q.x);
-  q.y = pair_swap(q.y);
-  __builtin_memcpy(&v, &q, 8);
-  return v;
-}
-// lanes i and i ^ 8 of every row of 16 exchanged
-__device__ __forceinline__ double half_row_swap(double v) {
-  int2 q;
-  __builtin_memcpy(&q, &v, 8);
-  q.x = __builtin_amdgcn_mov_dpp(q.x, 0x128, 0xf, 0xf, true);  // row_ror:8
-  q.y = __builtin_amdgcn_mov_dpp(q.y, 0x128, 0xf, 0xf, true);
-  __builtin_memcpy(&v, &q, 8);
-  return v;
-}
-// orders a wave's LDS writes before its later reads of other lanes' data (the
-// LDS executes one wave's accesses in order; this keeps the compiler from
-// moving them)
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
-// keeps the descriptors of a point out of registers between its uses: tiles
-// and sites of one point read them again from LDS (broadcast reads, cheap
-// next to the gathers) where the compiler would otherwise hold some 50
-// registers of them
-__device__ __forceinline__ void reread_lds() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-// computes a and b here: the compiler would otherwise sink their sums to the
-// last use, across the branches between, and hold the gathered supports until
-// then (more than 100 spilled registers)
-__device__ __forceinline__ void settle(double &a, double &b) { asm volatile("" : "+v"(a), "+v"(b)); }
 
 // the four supports of an access buffer at one site: (t lo, t hi) of the first
 // and of the second o index
@@ -115,24 +69,6 @@ __device__ __forceinline__ double density_sum(double2 wa, double2 wb, const Quad
 // the part of density_sum on diagonal supports (flag bits 2 and 3)
 __device__ __forceinline__ double diagonal_sum(int flags, double2 wa, double2 wb, const Quad &q) {
   return ((flags & 4) ? fma(wa.y, q.v1.y, wa.x * q.v0.y) : 0.0) + ((flags & 8) ? fma(wb.y, q.v3.y, wb.x * q.v2.y) : 0.0);
-}
-
-struct Bracket {
-  int lo, step;  // support indices lo and lo + step (step 0: clamped, weight 0)
-  double b;
-};
-__device__ __forceinline__ Bracket bracket_of(const double *m, int nw, double w, int geo, float ga, float gb) {
-  int lo, hi;
-  double b;
-  interp_sel(m, nw, w, geo, ga, gb, lo, hi, b);
-  return Bracket{lo, hi - lo, b};
-}
-
-__device__ __forceinline__ int tri_decode(int q) {
-  int s = (int)((sqrt(8.0 * q + 1.0) - 1.0) * 0.5);
-  while ((s + 1) * (s + 2) / 2 <= q) ++s;
-  while (s * (s + 1) / 2 > q) --s;
-  return s;
 }
 
 // ---------------------------------------------------------------------------
@@ -161,10 +97,6 @@ inline SuShape su_shape(int L) {
   }
   return best;
 }
-// units of a flow: (X, a >= b), and per (X, t) the second result of the
-// diagonal item (X, t, X)
-inline long long su_units(long long nw) { return nw * (nw * (nw + 1) / 2 + nw); }
-
 constexpr int kSuWaveBytes = 64 * 16 + 64 * 32 + kRhsPoints * 8;
 
 // adds the S and U integrals of all items to dG (zeroed before): every item
@@ -172,8 +104,7 @@ constexpr int kSuWaveBytes = 64 * 16 + 64 * 32 + kRhsPoints * 8;
 template <int RHO, bool ASYM>
 __global__ __launch_bounds__(64 * kRhsWaves, 4) void k_su(const FlowDev *__restrict__ fl, int nflows, long long total) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  const long long j0 = blockIdx.x >> 3;
-  const long long blk = ((j0 / kChunk) * 8 + (blockIdx.x & 7)) * kChunk + (j0 % kChunk);
+  const long long blk = xcd_position(blockIdx.x, kChunk);
   if (blk >= total) return;
   int f = 0;
   {
@@ -192,23 +123,10 @@ __global__ __launch_bounds__(64 * kRhsWaves, 4) void k_su(const FlowDev *__restr
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   for (int i = tid; i < nw; i += 64 * kRhsWaves) s_mesh[i] = F.mesh[i];
   __syncthreads();
-  const int npair = nw * (nw + 1) / 2, per = npair + nw;
   const int unit = (int)(blk - F.su_base) * kRhsWaves + wave;
-  if (unit >= nw * per) return;
-  const int X = unit / per, q = unit - X * per;
-  int a, b, kind, outs;  // kind 0: S rule for both results, 1: U rule for both, 2: first U, second S
-  if (q < npair) {
-    a = __builtin_amdgcn_readfirstlane(tri_decode(q));
-    b = q - a * (a + 1) / 2;
-    kind = a <= X ? 0 : (b >= X ? 1 : 2);
-    outs = a == b ? 1 : 3;
-  } else {
-    const int t = q - npair;
-    a = t <= X ? X : t;
-    b = t <= X ? t : X;
-    kind = t <= X ? 1 : 0;
-    outs = t <= X ? 1 : 2;
-  }
+  if (unit >= nw * (nw * (nw + 1) / 2 + nw)) return;
+  const SuUnit un = su_unit(unit, nw);
+  const int X = un.X, a = un.a, b = un.b, kind = un.kind, outs = un.outs;
   unsigned char *wl = lds_raw + ((nw * 8 + 15) & ~15) + wave * kSuWaveBytes;
   int4 *s_off = reinterpret_cast<int4 *>(wl);
   double2 *s_wa = reinterpret_cast<double2 *>(wl + 64 * 16);
@@ -263,23 +181,17 @@ __global__ __launch_bounds__(64 * kRhsWaves, 4) void k_su(const FlowDev *__restr
         int4 d = make_int4((int)kNoRow, (int)kNoRow, 0, 0);
         double2 wa = make_double2(0.0, 0.0), wb = wa;
         if (ok) {
-          const int ol = o.lo, oh = o.lo + o.step;
-          const int rl = ol > X ? tri(ol, X) : tri(X, ol), rh = oh > X ? tri(oh, X) : tri(X, oh);
-          d.x = (rl * nw + t.lo) * rowbytes;
-          d.y = (rh * nw + t.lo) * rowbytes;
-          d.z = t.step * rowbytes;
-          // bits 2, 3: the support's outer indices are equal (first / second o index)
-          d.w = (ol == X ? 4 : 0) | (oh == X ? 8 : 0);
+          // bits 2, 3 of w: the support's outer indices are equal
+          const SuBuffer sb = su_buffer(t, o, X, nw, rowbytes, rule);
+          d = make_int4(sb.x, sb.y, sb.z, sb.diag);
+          wa = sb.wa;
+          wb = sb.wb;
           if (ASYM) {
             const double vo = pair_swap(v);
             const bool pos = vo > 0, neg = vo < 0;
             d.w |= (pj ? neg : pos) ? 1 : 0;
             d.w |= (pj ? pos : neg) ? 2 : 0;  // the exchange of the second result's V0 / V2
           }
-          const bool nl = rule ? ol >= X : ol > X, nh = rule ? oh >= X : oh > X;
-          const double bl = nl ? -(1.0 - o.b) : 1.0 - o.b, bh = nh ? -o.b : o.b;
-          wa = make_double2((1.0 - t.b) * bl, t.b * bl);
-          wb = make_double2((1.0 - t.b) * bh, t.b * bh);
         }
         wave_lds_fence();
         s_off[lane] = d;
@@ -384,9 +296,8 @@ __global__ __launch_bounds__(64 * kRhsWaves, 4) void k_su(const FlowDev *__restr
             r ? make_double2(a2s[i], a2d[i]) : make_double2(a1s[i], a1d[i]);
     }
     wave_lds_fence();
-    const int t = r ? a : b, o = r ? b : a;
-    const bool urule = kind == 1 || (kind == 2 && r == 0);  // item (o, t, X), else (X, t, o)
-    const int item = (urule ? tri(o, X) : tri(X, o)) * nw + t;
+    const bool urule = un.u_rule(r);
+    const int item = un.item(r, nw);
     double *out = reinterpret_cast<double *>(F.dG + (size_t)item * L);
     for (int k = lane; k < 2 * L; k += 64) {
       double v = 0.0;
@@ -399,8 +310,6 @@ __global__ __launch_bounds__(64 * kRhsWaves, 4) void k_su(const FlowDev *__restr
 // ---------------------------------------------------------------------------
 // T channel and the final sum
 // ---------------------------------------------------------------------------
-using d4 = __attribute__((ext_vector_type(4))) double;
-
 // A wave evaluates the T channel of an item, eight points at a time, its lanes
 // in the operand layout of the 16 x 16 x 4 FP64 matrix instruction (lane l =
 // row l % 16 of point l / 16): the gathered values are the operands of the
@@ -428,68 +337,24 @@ __host__ __device__ inline int t_wave_bytes(int L) {
   return c > kTDescBytes ? c : kTDescBytes;
 }
 
-// Overlap lists for the contraction of a bubble matrix: the distinct (rid1,
-// rid2) pairs of every site with their multiplicities, dealt to the 64 lanes
-// (lane_of[r] .. lane_of[r + 1] sum site r), entry k of lane l at [k * 64 + l]
-// = index | multiplicity << 16.
-struct OverlapPlan {
-  int rows = 0;
-  std::vector<unsigned> ent;
-  std::vector<int> lane_of, count;
-
-  // capacity the entries need at most: rows * 64 <= 2 * distinct + 64 (L <= 32)
-  void build(int L, const int *off, const int *rid1, const int *rid2) {
-    const int lp = t_shape(L).lp;
-    std::vector<unsigned> item, mult((size_t)lp * lp, 0);
-    std::vector<int> first(L + 1, 0);
-    for (int r = 0; r < L; ++r) {
-      first[r] = (int)item.size();
-      for (int i = off[r]; i < off[r + 1]; ++i) {
-        const unsigned k = (unsigned)(rid1[i] * lp + rid2[i]);
-        if (mult[k]++ == 0) item.push_back(k);
-      }
-      // an entry holds multiplicities up to 0xffff; larger ones take several
-      const size_t end = item.size();
-      for (size_t j = first[r]; j < end; ++j) {
-        const unsigned k = item[j];
-        unsigned left = mult[k];
-        mult[k] = 0;
-        for (; left > 0xffffu; left -= 0xffffu) item.push_back(k | 0xffff0000u);
-        item[j] = k | left << 16;
-      }
-    }
-    first[L] = (int)item.size();
-    auto lanes_at = [&](int r, int rws) { return std::max(1, (first[r + 1] - first[r] + rws - 1) / rws); };
-    rows = std::max(1, ((int)item.size() + 63) / 64);
-    for (;; ++rows) {
-      int lanes = 0;
-      for (int r = 0; r < L; ++r) lanes += lanes_at(r, rows);
-      if (lanes <= 64) break;
-    }
-    ent.assign((size_t)rows * 64, 0);
-    count.assign(64, 0);
-    lane_of.assign(L + 1, 0);
-    int lane = 0;
-    for (int r = 0; r < L; ++r) {
-      lane_of[r] = lane;
-      for (int k = 0; k < first[r + 1] - first[r]; ++k) {
-        const int l = lane + k / rows;
-        ent[(size_t)(k % rows) * 64 + l] = item[first[r] + k];
-        count[l] = k % rows + 1;
-      }
-      lane += lanes_at(r, rows);
-    }
-    lane_of[L] = lane;
+// distinct (rid1, rid2) pairs of every site's overlap list, with their
+// multiplicities, dealt to the lanes of a wave
+inline void build_overlap_plan(LanePlan &plan, int L, const int *off, const int *rid1, const int *rid2) {
+  const int lp = t_shape(L).lp;
+  plan.begin((size_t)lp * lp);
+  for (int r = 0; r < L; ++r) {
+    for (int i = off[r]; i < off[r + 1]; ++i) plan.add((unsigned)(rid1[i] * lp + rid2[i]));
+    plan.end_output();
   }
-};
+  plan.deal(64);
+}
 
 template <int FT, int HT, bool ASYM>
 __global__ __launch_bounds__(64 * kRhsWaves, FT + HT == 1 ? 4 : 3) void k_t(const FlowDev *__restrict__ fl, int nflows, long long total) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   constexpr int LP = 16 * FT + 8 * HT;
   constexpr int NT = FT + HT;
-  const long long j0 = blockIdx.x >> 3;
-  const long long blk = ((j0 / kChunk) * 8 + (blockIdx.x & 7)) * kChunk + (j0 % kChunk);
+  const long long blk = xcd_position(blockIdx.x, kChunk);
   if (blk >= total) return;
   int f = 0;
   {
@@ -754,12 +619,7 @@ __global__ __launch_bounds__(64 * kRhsWaves, FT + HT == 1 ? 4 : 3) void k_t(cons
         }
       }
     wave_lds_fence();
-    double sum = 0.0;
-    for (int k = 0; k < cnt; ++k) {
-      const unsigned en = F.plan_ent[k * 64 + lane];
-      sum = fma((double)(en >> 16), s_C[en & 0xffff], sum);
-    }
-    s_part[lane] = sum;
+    s_part[lane] = plan_sum(reinterpret_cast<const uint4 *>(F.plan_ent) + lane, 64, cnt, s_C);
     wave_lds_fence();
     if (lane < L) {
       const int l1 = F.plan_lane[lane + 1];

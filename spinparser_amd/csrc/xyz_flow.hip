@@ -12,11 +12,14 @@
 //   src/XYZ/XYZMeasurementCorrelation.cpp:98-212    static susceptibility, 4 outputs
 //
 // Device memory (per flow):
-//   Gamma, dGamma  FP64, components interleaved: the element of (row, site) is
-//                  {X, Y, Z, D} at ((row * L) + rid) * 4, row = (s(s+1)/2 + u) * N_w + t,
-//                  so one support of one site is two 16-byte loads.  The C ABI
-//                  converts from / to the reference's four planes
-//                  (_dataXX ... _dataDD) on upload and download.
+//   Gamma, dGamma  FP64, rows of 4 L values, row = (s(s+1)/2 + u) * N_w + t: {X, Y}
+//                  of all sites, then {Z, D} of all sites, so one support of one
+//                  site is two 16-byte loads and a wave's load reads adjacent sites
+//                  without gaps (elements {X, Y, Z, D} at a stride of 32 bytes cost
+//                  the gathers of k_xyz_su 24 instead of 17 cycles each).  Sites are
+//                  numbered so that the lanes of a point hold consecutive ones
+//                  (site_order); the C ABI converts from / to the reference's four
+//                  planes (_dataXX ... _dataDD) on upload and download.
 //   Sigma, dSigma  FP64 [N_w]
 //   weight tables  per exact index x: evaluation points and weights at the cutoff
 //
@@ -39,16 +42,19 @@
 // evaluates the bubble per point from the overlap lists instead.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
 #include "frg_common.h"
 #include "spfrg.h"
+#include "wave_rhs.h"
 
 namespace {
 
@@ -96,10 +102,17 @@ struct XyzDev {
   long long nf;
   long long np;  // N_f * L
   unsigned g_bytes;
+  // wave kernels (xyz_rhs.h): lanes of a point, bubble tiles, plan of the overlap sums
+  int lps, ntiles;
+  const struct XyzLane *lanes;
+  const int *tiles, *plan;
   double cut, step;
   int geo;  // geometric mesh: bracket guess from the logarithm (count_le_geo)
   float ga, gb;
 };
+
+// position of component c of a site within a row of 4 L values
+__host__ __device__ __forceinline__ int xyz_el(int L, int site, int c) { return (c >> 1) * 2 * L + 2 * site + (c & 1); }
 
 __device__ __forceinline__ double gload(__amdgpu_buffer_rsrc_t r, int byte_off) {
   auto v = __builtin_amdgcn_raw_buffer_load_b64(r, byte_off, 0, 0);
@@ -108,10 +121,19 @@ __device__ __forceinline__ double gload(__amdgpu_buffer_rsrc_t r, int byte_off) 
   return d;
 }
 
-// weight tables of one flow (the SU(2) core's definition)
+#include "xyz_rhs.h"
+
+// weight tables of one flow (the SU(2) core's definition); workgroups past
+// x == nw clear dG for k_xyz_su
 __global__ __launch_bounds__(64) void k_xyz_weights(XyzDev F, int corr_only) {
   extern __shared__ double s_wmesh[];
   const int x = corr_only ? F.nw : (int)blockIdx.x;
+  if (x > F.nw) {
+    double2 *g = reinterpret_cast<double2 *>(F.dG);
+    const size_t n = 2 * (size_t)F.np, stride = (size_t)(gridDim.x - F.nw - 1) * 64;
+    for (size_t i = (size_t)(x - F.nw - 1) * 64 + threadIdx.x; i < n; i += stride) g[i] = make_double2(0.0, 0.0);
+    return;
+  }
   weight_tables_wave(x, F.mesh, F.nw, F.cut, F.v2, F.dv2, F.Wwp, F.Wc, F.Wn, F.Cwp, F.Cw, F.Cn, F.emax, F.flags + 1,
                      s_wmesh);
 }
@@ -132,7 +154,7 @@ __device__ double xyz_value_none(const double *G, const double *m, int nw, int L
   interp(m, nw, s, lS, uS, bS);
   interp(m, nw, t, lT, uT, bT);
   interp(m, nw, u, lU, uU, bU);
-  const double *P = G + (size_t)rid * 4 + c;
+  const double *P = G + xyz_el(L, rid, c);
   const size_t rs = (size_t)L * 4;
   auto A = [&](int so, int to, int uo) {
     if (so < uo) {
@@ -290,8 +312,8 @@ __global__ __launch_bounds__(kXyzPW, SPFRG_XYZ_MIN_BLOCKS) void k_xyz_dgamma(Xyz
   // permutations (2 bits per component) of getSites / getInvertedSites
   int sr_fwd = 0, sr_inv = 0, pf = 0, pi = 0;
   if (active) {
-    sr_fwd = F.site_rid[rid] * 32;
-    sr_inv = F.inv_rid[rid] * 32;
+    sr_fwd = F.site_rid[rid] * 16;
+    sr_inv = F.inv_rid[rid] * 16;
     pf = F.site_perm[3 * rid] | (F.site_perm[3 * rid + 1] << 2) | (F.site_perm[3 * rid + 2] << 4);
     pi = F.inv_perm[3 * rid] | (F.inv_perm[3 * rid + 1] << 2) | (F.inv_perm[3 * rid + 2] << 4);
   }
@@ -382,7 +404,7 @@ __global__ __launch_bounds__(kXyzPW, SPFRG_XYZ_MIN_BLOCKS) void k_xyz_dgamma(Xyz
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const double2 v01 = buf_load<double2>(rG, d.off[r]);
-              const double2 v23 = buf_load<double2>(rG, d.off[r] + 16);
+              const double2 v23 = buf_load<double2>(rG, d.off[r] + 16 * L);
               l[kX] = fma(d.ws[r], v01.x, l[kX]);
               l[kY] = fma(d.ws[r], v01.y, l[kY]);
               l[kZ] = fma(d.ws[r], v23.x, l[kZ]);
@@ -422,7 +444,7 @@ __global__ __launch_bounds__(kXyzPW, SPFRG_XYZ_MIN_BLOCKS) void k_xyz_dgamma(Xyz
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const double2 v01 = buf_load<double2>(rG, oo[r] + sr);
-            const double2 v23 = buf_load<double2>(rG, oo[r] + sr + 16);
+            const double2 v23 = buf_load<double2>(rG, oo[r] + sr + 16 * L);
             const double ws = s_ws[sk * 4 + r];
             const double wd = (exw >> (1 + r)) & 1 ? -ws : ws;
             u0 = fma(ws, v01.x, u0);
@@ -542,7 +564,7 @@ __global__ __launch_bounds__(kXyzPW, SPFRG_XYZ_MIN_BLOCKS) void k_xyz_dgamma(Xyz
     double v = s_rpa[q];
     for (int sl = 0; sl < slots; ++sl) v += s_red[(sl * L + r) * 4 + k];
     v *= (1.0 / kTwoPi);
-    F.dG[(size_t)item * 4 * L + q] = v;
+    F.dG[(size_t)item * 4 * L + xyz_el(L, r, k)] = v;
     if (isnan(v)) atomicOr(&F.flags[0], 1);
   }
 }
@@ -646,8 +668,8 @@ __global__ __launch_bounds__(kXyzThreads) void k_xyz_dgamma_direct(XyzDev F) {
   for (int q = tid; q < 4 * L; q += kXyzThreads) {
     const int c = q / L, j = q - (q / L) * L;
     const int pf = c < 3 ? F.site_perm[3 * j + c] : kD, pi = c < 3 ? F.inv_perm[3 * j + c] : kD;
-    s_cf[q] = F.site_rid[j] * 4 + pf;
-    s_ci[q] = F.inv_rid[j] * 4 + pi;
+    s_cf[q] = xyz_el(L, F.site_rid[j], pf);
+    s_ci[q] = xyz_el(L, F.inv_rid[j], pi);
   }
   __syncthreads();
 
@@ -713,7 +735,7 @@ __global__ __launch_bounds__(kXyzThreads) void k_xyz_dgamma_direct(XyzDev F) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               const double sg = (cc == kD && ((fl >> (2 + q)) & 1)) ? -w[q] : w[q];
-              v = fma(sg, gload(rG, (off[q] + cc) * 8), v);
+              v = fma(sg, gload(rG, (off[q] + xyz_el(L, 0, cc)) * 8), v);
             }
             s_loc[(e * 4 + (k - 4)) * 4 + cc] = v;
           }
@@ -794,7 +816,7 @@ __global__ __launch_bounds__(kXyzThreads) void k_xyz_dgamma_direct(XyzDev F) {
     for (int g = 0; g < ng; ++g) v += red[(size_t)g * 4 * L + q];
     v *= (1.0 / kTwoPi);
     const int c = q / L, j = q - (q / L) * L;
-    F.dG[((size_t)item * L + j) * 4 + c] = v;
+    F.dG[(size_t)item * 4 * L + xyz_el(L, j, c)] = v;
     if (isnan(v)) atomicOr(&F.flags[0], 1);
   }
 }
@@ -849,14 +871,15 @@ __global__ __launch_bounds__(kXyzThreads) void k_xyz_corr_partial(XyzDev F) {
         interp(m, nw, c, lU, uU, bU);
         const int srid = exch ? F.inv_rid[rid] : F.site_rid[rid];
         const int *perm = exch ? F.inv_perm + 3 * rid : F.site_perm + 3 * rid;
-        const int comp[4] = {perm[0], perm[1], perm[2], kD};
+        const int comp[4] = {xyz_el(L, srid, perm[0]), xyz_el(L, srid, perm[1]), xyz_el(L, srid, perm[2]),
+                             xyz_el(L, srid, kD)};
         double v[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int S = (i & 1) ? uS : lS, T = (i & 2) ? uT : lT, U = (i & 4) ? uU : lU;
           const double wi = ((i & 2) ? bT : (1 - bT)) * ((i & 1) ? bS : (1 - bS)) * ((i & 4) ? bU : (1 - bU));
           const bool fx = S < U;
-          const double *el = G + (((size_t)(fx ? tri(U, S) : tri(S, U)) * nw + T) * L + srid) * 4;
+          const double *el = G + ((size_t)(fx ? tri(U, S) : tri(S, U)) * nw + T) * 4 * L;
 #pragma unroll
           for (int k = 0; k < 4; ++k) v[k] = fma((k == kD && fx) ? -wi : wi, el[comp[k]], v[k]);
         }
@@ -930,10 +953,12 @@ struct sp_xyz_ctx {
   XyzDev fd{};
   double cutoff = 0.0;
   bool have_flow = false;
+  bool waves = false;   // dGamma by the wave kernels (xyz_rhs.h)
   bool direct = false;  // bubble summed per point (k_xyz_dgamma_direct)
   size_t lds = 0;
   std::vector<void *> allocs;
-  std::vector<double> host;  // plane <-> interleaved staging of the state
+  std::vector<double> host;  // staging of the state between the planes and the device layout
+  std::vector<int> place;    // position of (rid, component) within a device row
   bool prof = false;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> pending[4];
   double prof_ms[4] = {0, 0, 0, 0};
@@ -1021,28 +1046,210 @@ hipError_t xyz_launch_compute(sp_xyz_ctx *ctx) {
   }
   {
     XyzProf ps(ctx, 2);
-    hipLaunchKernelGGL(k_xyz_weights, dim3(F.nw + 1), dim3(64), F.nw * sizeof(double), ctx->stream, F, 0);
+    const unsigned clear = ctx->waves ? (unsigned)std::min<long long>((2 * F.np + 255) / 256, 4096) : 0;
+    hipLaunchKernelGGL(k_xyz_weights, dim3(F.nw + 1 + clear), dim3(64), F.nw * sizeof(double), ctx->stream, F, 0);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   XyzProf ps(ctx, 0);
   const long long rounds = (F.nf + 8 * kXyzChunk - 1) / (8 * kXyzChunk);
   const dim3 grid((unsigned)(rounds * 8 * kXyzChunk));
-  if (ctx->direct)
+  if (ctx->waves) {
+    const long long units = (su_units(F.nw) + kRhsWaves - 1) / kRhsWaves;
+    auto padded = [](long long blocks) { return dim3((unsigned)((blocks + 8 * kXyzChunk - 1) / (8 * kXyzChunk) * 8 * kXyzChunk)); };
+    const size_t mesh = (size_t)(F.nw * 8 + 15) & ~size_t(15);
+    hipLaunchKernelGGL(k_xyz_su, padded(units), dim3(64 * kRhsWaves), mesh + kRhsWaves * kXyzSuWaveBytes, ctx->stream, F, units);
+    const size_t lds = xyz_t_lds(F.nw, F.L, F.lps);
+    const dim3 tg = padded(F.nf);
+    if (F.ntiles <= 4 * kRhsWaves) hipLaunchKernelGGL(k_xyz_t<4>, tg, dim3(64 * kRhsWaves), lds, ctx->stream, F);
+    else if (F.ntiles <= 7 * kRhsWaves) hipLaunchKernelGGL(k_xyz_t<7>, tg, dim3(64 * kRhsWaves), lds, ctx->stream, F);
+    else hipLaunchKernelGGL(k_xyz_t<kXyzMaxTiles>, tg, dim3(64 * kRhsWaves), lds, ctx->stream, F);
+  } else if (ctx->direct)
     hipLaunchKernelGGL(k_xyz_dgamma_direct, grid, dim3(kXyzThreads), ctx->lds, ctx->stream, F);
   else
     hipLaunchKernelGGL(k_xyz_dgamma, grid, dim3(kXyzPW), ctx->lds, ctx->stream, F);
   return hipGetLastError();
 }
 
-// the reference's four planes X, Y, Z, D <-> the interleaved device layout
-void planes_to_interleaved(const double *planes, double *out, size_t np) {
-  for (size_t i = 0; i < np; ++i)
-    for (int c = 0; c < 4; ++c) out[4 * i + c] = planes[c * np + i];
+// The device's numbering of the sites (order[rid] = device site).  Lattices of
+// the form the wave kernels need (site_rid the identity, inv_rid an
+// involution) are numbered by the lanes of a point: first the lanes' first
+// sites, then their second ones, a site and its inverse in one lane, the
+// self-inverse ones in pairs; site 0 stays first.  Others keep their order.
+struct XyzOrder {
+  bool waves = false;
+  std::vector<int> order;
+  std::vector<int> first, second;  // sites of the lanes, device numbering (-1: none)
+};
+XyzOrder xyz_order(const sp_xyz_problem *p) {
+  XyzOrder o;
+  const int L = p->L;
+  o.order.resize(L);
+  for (int r = 0; r < L; ++r) o.order[r] = r;
+  if (L > kMaxXyzRhsL || p->inv_rid[0] != 0) return o;
+  for (int r = 0; r < L; ++r)
+    if (p->site_rid[r] != r || p->inv_rid[p->inv_rid[r]] != r) return o;
+  o.waves = true;
+  std::vector<int> self, a, b;
+  for (int r = 0; r < L; ++r)
+    if (p->inv_rid[r] == r) self.push_back(r);
+  size_t k = 0;
+  if (self.size() & 1) { a.push_back(self[k++]); b.push_back(-1); }
+  for (; k < self.size(); k += 2) { a.push_back(self[k]); b.push_back(self[k + 1]); }
+  for (int r = 0; r < L; ++r)
+    if (p->inv_rid[r] > r) { a.push_back(r); b.push_back(p->inv_rid[r]); }
+  int next = 0;
+  for (int r : a) { o.first.push_back(next); o.order[r] = next++; }
+  for (int r : b) {
+    o.second.push_back(r < 0 ? -1 : next);
+    if (r >= 0) o.order[r] = next++;
+  }
+  return o;
 }
-void interleaved_to_planes(const double *in, double *planes, size_t np) {
-  for (size_t i = 0; i < np; ++i)
-    for (int c = 0; c < 4; ++c) planes[c * np + i] = in[4 * i + c];
+
+// Tables of the wave kernels, if the lattice has the form they need: lanes of
+// a point, the tiles of the bubble product matrix that the overlap lists refer
+// to, and the plan of their sums.
+int xyz_wave_tables(sp_xyz_ctx *ctx, const sp_xyz_problem *p, const XyzOrder &order, int max_lds) {
+  XyzDev &f = ctx->fd;
+  const int L = f.L;
+  if (!order.waves) return SP_OK;
+  std::vector<int> table;  // lanes, tiles, then the plans of the passes
+  LanePlan plan;
+  const int lps = (int)order.first.size();
+  int ntiles = 0;
+  size_t tiles_at = 0, plan_at = 0;
+  auto align4 = [&] { table.resize((table.size() + 3) & ~size_t(3), 0); };
+  try {
+    auto packed = [](const int *q) { return q[0] | q[1] << 2 | q[2] << 4; };
+    auto perms = [&](int r) { return packed(p->site_perm + 3 * r) | packed(p->inv_perm + 3 * r) << 6; };
+    for (int j = 0; j < lps; ++j) {
+      const int a = order.first[j], b = order.second[j];
+      const int cyc = b >= 0 && p->inv_rid[a] == b;
+      const XyzLane ln{a, b, perms(a), b >= 0 ? perms(b) | cyc << 12 : 0};
+      table.insert(table.end(), {ln.a, ln.b, ln.pa, ln.pb});
+    }
+    // element (a, r1), (b, r2) of the product matrix
+    const int nt = (4 * L + 15) / 16, O = p->ovl_off[L];
+    std::vector<int> tile((size_t)nt * nt, -1);
+    std::vector<int> list;
+    auto rows_cols = [&](int i, int c, int &row, int &col) {
+      row = (c < 3 ? p->ovl_perm1[3 * i + c] : 3) * L + p->ovl_rid1[i];
+      col = (c < 3 ? p->ovl_perm2[3 * i + c] : 3) * L + p->ovl_rid2[i];
+    };
+    for (int i = 0; i < O; ++i)
+      for (int c = 0; c < 4; ++c) {
+        int row, col;
+        rows_cols(i, c, row, col);
+        tile[(row >> 4) * nt + (col >> 4)] = 0;
+      }
+    for (int k = 0; k < nt * nt; ++k)
+      if (tile[k] == 0) {
+        tile[k] = ntiles++;
+        list.push_back((k / nt) * 16 | (k % nt) * 16 << 16);
+      }
+    if (ntiles > kXyzMaxTiles * kRhsWaves) return SP_OK;
+    tiles_at = table.size();
+    table.insert(table.end(), list.begin(), list.end());
+    align4();
+    plan_at = table.size();
+    for (int t0 = 0; t0 < ntiles; t0 += kXyzPassTiles) {
+      plan.begin((size_t)kXyzPassTiles * 256);
+      for (int k = 0; k < 4 * L; ++k) {  // outputs in the order of a device row
+          const int c = 2 * (k / (2 * L)) + (k & 1), r = (k % (2 * L)) / 2;
+          for (int i = p->ovl_off[r]; i < p->ovl_off[r + 1]; ++i) {
+            int row, col;
+            rows_cols(i, c, row, col);
+            const int t = tile[(row >> 4) * nt + (col >> 4)] - t0;
+            if (t >= 0 && t < kXyzPassTiles) plan.add((unsigned)(t * 256 + (row & 15) * 16 + (col & 15)));
+          }
+          plan.end_output();
+        }
+      plan.deal(64 * kRhsWaves);
+      table.push_back(plan.quads());
+      table.insert(table.end(), plan.lane_of.begin(), plan.lane_of.end());
+      table.insert(table.end(), plan.count.begin(), plan.count.end());
+      align4();
+      for (unsigned e : plan.ent) table.push_back((int)e);
+    }
+  } catch (...) { return xfail(ctx, SP_ENOMEM, "host buffer"); }
+  const size_t lds = xyz_t_lds(f.nw, L, lps);
+  if (lds > (size_t)max_lds) return SP_OK;
+  int *d = nullptr;
+  int rc = xalloc(ctx, &d, table.size());
+  if (rc) return rc;
+  SP_XHIP(hipMemcpy(d, table.data(), table.size() * 4, hipMemcpyHostToDevice));
+  f.lps = lps;
+  f.ntiles = ntiles;
+  f.lanes = reinterpret_cast<const XyzLane *>(d);
+  f.tiles = d + tiles_at;
+  f.plan = d + plan_at;
+  SP_XHIP(hipFuncSetAttribute((const void *)k_xyz_t<4>, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
+  SP_XHIP(hipFuncSetAttribute((const void *)k_xyz_t<7>, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
+  SP_XHIP(hipFuncSetAttribute((const void *)k_xyz_t<kXyzMaxTiles>, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
+  ctx->waves = true;
+  return SP_OK;
+}
+
+// A problem's tables in the device numbering.
+struct XyzTables {
+  std::vector<int> site, sitep, inv, invp, off, r1, r2, p1, p2, fwd, rev, corr;
+  sp_xyz_problem q;
+  XyzTables(const sp_xyz_problem *p, const std::vector<int> &order) : q(*p) {
+    const int L = p->L;
+    auto sites = [&](std::vector<int> &to, const int *from, size_t n) {
+      to.resize(n);
+      for (size_t i = 0; i < n; ++i) to[i] = order[from[i]];
+    };
+    std::vector<int> old(L);
+    for (int r = 0; r < L; ++r) old[order[r]] = r;
+    auto moved = [&](std::vector<int> &rid, std::vector<int> &perm, const int *frid, const int *fperm) {
+      for (int s = 0; s < L; ++s) {
+        rid.push_back(order[frid[old[s]]]);
+        perm.insert(perm.end(), fperm + 3 * old[s], fperm + 3 * old[s] + 3);
+      }
+    };
+    moved(site, sitep, p->site_rid, p->site_perm);
+    moved(inv, invp, p->inv_rid, p->inv_perm);
+    off.push_back(0);
+    for (int s = 0; s < L; ++s) {
+      for (int i = p->ovl_off[old[s]]; i < p->ovl_off[old[s] + 1]; ++i) {
+        r1.push_back(order[p->ovl_rid1[i]]);
+        r2.push_back(order[p->ovl_rid2[i]]);
+        p1.insert(p1.end(), p->ovl_perm1 + 3 * i, p->ovl_perm1 + 3 * i + 3);
+        p2.insert(p2.end(), p->ovl_perm2 + 3 * i, p->ovl_perm2 + 3 * i + 3);
+      }
+      off.push_back((int)r1.size());
+    }
+    sites(fwd, p->range_fwd, p->R);
+    sites(rev, p->range_inv, p->R);
+    sites(corr, p->corr_rid, (size_t)p->B * p->Rb);
+    q.site_rid = site.data();
+    q.site_perm = sitep.data();
+    q.inv_rid = inv.data();
+    q.inv_perm = invp.data();
+    q.ovl_off = off.data();
+    q.ovl_rid1 = r1.data();
+    q.ovl_rid2 = r2.data();
+    q.ovl_perm1 = p1.data();
+    q.ovl_perm2 = p2.data();
+    q.range_fwd = fwd.data();
+    q.range_inv = rev.data();
+    q.corr_rid = corr.data();
+  }
+};
+
+// the reference's four planes X, Y, Z, D <-> the device layout (place: position
+// of (rid, component) within a row)
+void planes_to_rows(const double *planes, double *out, size_t np, int L, const int *place) {
+  for (int c = 0; c < 4; ++c)
+    for (size_t row = 0; row * L < np; ++row)
+      for (int r = 0; r < L; ++r) out[row * 4 * L + place[4 * r + c]] = planes[c * np + row * L + r];
+}
+void rows_to_planes(const double *in, double *planes, size_t np, int L, const int *place) {
+  for (int c = 0; c < 4; ++c)
+    for (size_t row = 0; row * L < np; ++row)
+      for (int r = 0; r < L; ++r) planes[c * np + row * L + r] = in[row * 4 * L + place[4 * r + c]];
 }
 
 }  // namespace
@@ -1064,6 +1271,8 @@ int sp_xyz_ctx_footprint(const sp_xyz_problem *p, long long *bytes) {
   return SP_OK;
 }
 
+static int xyz_ctx_init(sp_xyz_ctx *ctx, const sp_xyz_problem *p, const XyzOrder &order);
+
 int sp_xyz_ctx_create(const sp_xyz_problem *p, sp_xyz_ctx **out) {
   if (!out) return SP_EARG;
   *out = nullptr;
@@ -1072,6 +1281,19 @@ int sp_xyz_ctx_create(const sp_xyz_problem *p, sp_xyz_ctx **out) {
   *out = ctx;
   int rc = check_xyz_problem(ctx, p);
   if (rc != SP_OK) return rc;
+  try {
+    const XyzOrder order = xyz_order(p);
+    const XyzTables tables(p, order.order);
+    ctx->place.resize(4 * (size_t)p->L);
+    for (int r = 0; r < p->L; ++r)
+      for (int c = 0; c < 4; ++c) ctx->place[4 * r + c] = xyz_el(p->L, order.order[r], c);
+    return xyz_ctx_init(ctx, &tables.q, order);
+  } catch (...) { return xfail(ctx, SP_ENOMEM, "host buffer"); }
+}
+
+// p: the tables in the device numbering
+static int xyz_ctx_init(sp_xyz_ctx *ctx, const sp_xyz_problem *p, const XyzOrder &order) {
+  int rc = SP_OK;
   SP_XHIP(hipGetDevice(&ctx->device));
   SP_XHIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
   XyzDev &f = ctx->fd;
@@ -1182,6 +1404,7 @@ int sp_xyz_ctx_create(const sp_xyz_problem *p, sp_xyz_ctx **out) {
   SP_XHIP(hipMemcpy(ri, p->range_inv, (size_t)f.R * 4, hipMemcpyHostToDevice));
   SP_XHIP(hipMemcpy(corr, p->corr_rid, nc * 4, hipMemcpyHostToDevice));
   SP_XHIP(hipMemcpy(corrp, p->corr_perm, 3 * nc * 4, hipMemcpyHostToDevice));
+  if (!(force && std::strcmp(force, "direct") == 0) && (rc = xyz_wave_tables(ctx, p, order, max_lds))) return rc;
   SP_XHIP(hipMemset(f.G, 0, nv * 8));
   SP_XHIP(hipMemset(f.dG, 0, nv * 8));
   SP_XHIP(hipMemset(f.v2, 0, f.nw * 8));
@@ -1211,7 +1434,7 @@ int sp_xyz_set_state(sp_xyz_ctx *ctx, double cutoff, const double *v2, const dou
   if (!std::isfinite(cutoff) || !(cutoff > 0.0)) return xfail(ctx, SP_EARG, "cutoff must be finite and positive");
   SP_XHIP(hipStreamSynchronize(ctx->stream));
   SP_XHIP(hipMemcpy(ctx->fd.v2, v2, ctx->fd.nw * 8, hipMemcpyHostToDevice));
-  planes_to_interleaved(v4, ctx->host.data(), (size_t)ctx->fd.np);
+  planes_to_rows(v4, ctx->host.data(), (size_t)ctx->fd.np, ctx->fd.L, ctx->place.data());
   SP_XHIP(hipMemcpy(ctx->fd.G, ctx->host.data(), 4 * (size_t)ctx->fd.np * 8, hipMemcpyHostToDevice));
   SP_XHIP(hipMemset(ctx->fd.flags, 0, 16));
   ctx->cutoff = cutoff;
@@ -1226,7 +1449,7 @@ int sp_xyz_get_state(sp_xyz_ctx *ctx, double *cutoff, double *v2, double *v4) {
   if (v2) SP_XHIP(hipMemcpy(v2, ctx->fd.v2, ctx->fd.nw * 8, hipMemcpyDeviceToHost));
   if (v4) {
     SP_XHIP(hipMemcpy(ctx->host.data(), ctx->fd.G, 4 * (size_t)ctx->fd.np * 8, hipMemcpyDeviceToHost));
-    interleaved_to_planes(ctx->host.data(), v4, (size_t)ctx->fd.np);
+    rows_to_planes(ctx->host.data(), v4, (size_t)ctx->fd.np, ctx->fd.L, ctx->place.data());
   }
   return SP_OK;
 }
@@ -1238,7 +1461,7 @@ int sp_xyz_get_flow(sp_xyz_ctx *ctx, double *dv2, double *dv4) {
   if (dv2) SP_XHIP(hipMemcpy(dv2, ctx->fd.dv2, ctx->fd.nw * 8, hipMemcpyDeviceToHost));
   if (dv4) {
     SP_XHIP(hipMemcpy(ctx->host.data(), ctx->fd.dG, 4 * (size_t)ctx->fd.np * 8, hipMemcpyDeviceToHost));
-    interleaved_to_planes(ctx->host.data(), dv4, (size_t)ctx->fd.np);
+    rows_to_planes(ctx->host.data(), dv4, (size_t)ctx->fd.np, ctx->fd.L, ctx->place.data());
   }
   return SP_OK;
 }
