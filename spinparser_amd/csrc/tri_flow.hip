@@ -12,7 +12,8 @@
 //
 // Device memory (per flow):
 //   Gamma, dGamma  FP64 [N_f][16][L] in the reference order
-//                  ((s(s+1)/2 + u) * N_w + t) * 16 L + (4 s1 + s2) L + rid
+//                  ((s(s+1)/2 + u) * N_w + t) * 16 L + (4 s1 + s2) L + rid,
+//                  or [N_f][L][16] for the wave kernels
 //   Sigma, dSigma  FP64 [N_w]
 //   weight tables  per exact index x: evaluation points and weights at the cutoff
 //
@@ -21,7 +22,11 @@
 // density-spin components carrying a factor i); no coefficient is spelled out
 // by hand.  Each table expands into straight-line FMAs on register arrays.
 //
-// dGamma kernel: one workgroup per frequency triple (s, t, u), 128 threads for
+// dGamma: the wave kernels of tri_rhs.h, or, for lattices outside their reach
+// (more than 32 sites, tables that are no symmetry operations, too many distinct
+// products), the general kernel of this file.
+//
+// General kernel: one workgroup per frequency triple (s, t, u), 128 threads for
 // lattices of at most 32 sites and 256 above, items walked t-major in XCD
 // runs; lattices of 13 to 32 sites run instantiations with the LDS bundle
 // geometry compiled in (every component offset an immediate).  Per channel
@@ -54,6 +59,7 @@
 
 #include "frg_common.h"
 #include "spfrg.h"
+#include "wave_rhs.h"
 
 namespace {
 
@@ -237,6 +243,15 @@ struct TriDev {
   double cut, step;
   int geo;  // geometric mesh: bracket guess from the logarithm (count_le_geo)
   float ga, gb;
+  // strides of a component and a site within a row of G, dG (doubles): the
+  // kernels of tri_rhs.h keep a site's components together
+  int cst, sst;
+  // k_tri_t: waves per item (0: the general kernel), groups per wave, points
+  // described at a time, entries in LDS, groups per pass of the overlap sums,
+  // instructions per wave for edge entries, tables of TriPlan
+  int t_waves, t_ng, t_points, t_entries, t_pass, t_edges;
+  const int *t_dst, *t_plan, *t_edge_ops;
+  const int4 *t_ops;
 };
 
 // lattice bubble: load the next overlap entry's packed sites ahead (1) or
@@ -319,8 +334,10 @@ __global__ __launch_bounds__(64) void k_tri_weights(TriDev F, int corr_only) {
 // getValue(i1, i2, s, t, u, s1, s2, FrequencyChannel::None) for pairs that keep
 // the requested components (density-density, or the pair (0, 0)); rid_fwd /
 // rid_inv = symmetryTransform(i1, i2) / (i2, i1)
-__device__ double tri_value_none(const double *G, const double *m, int nw, int L, int rid_fwd, int rid_inv, double s,
-                                 double t, double u, int s1, int s2) {
+__device__ double tri_value_none(const TriDev &F, int rid_fwd, int rid_inv, double s, double t, double u, int s1,
+                                 int s2) {
+  const double *G = F.G, *m = F.mesh;
+  const int nw = F.nw;
   double sign = 1.0;
   bool swap = false;
   if (s < 0) { s = -s; const int q = s1; s1 = s2; s2 = q; swap = !swap; }
@@ -332,8 +349,8 @@ __device__ double tri_value_none(const double *G, const double *m, int nw, int L
   interp(m, nw, s, lS, uS, bS);
   interp(m, nw, t, lT, uT, bT);
   interp(m, nw, u, lU, uU, bU);
-  const size_t FS = 16 * (size_t)L;
-  const int comp = (4 * s1 + s2) * L + rid;
+  const size_t FS = 16 * (size_t)F.L;
+  const int comp = (4 * s1 + s2) * F.cst + rid * F.sst;
   auto A = [&](int so, int to, int uo) {
     if (so < uo) return -double(zeta(s2)) * G[((size_t)tri(uo, so) * nw + to) * FS + comp];
     return G[((size_t)tri(so, uo) * nw + to) * FS + comp];
@@ -349,21 +366,21 @@ __global__ __launch_bounds__(64) void k_tri_dsigma(TriDev F) {
   const int i = blockIdx.x;
   if (i >= F.nw) return;
   const int lane = threadIdx.x;
-  const int nw = F.nw, L = F.L;
+  const int nw = F.nw;
   const double *m = F.mesh;
   const double cut = F.cut;
   const double w = m[i];
   double sum = 0.0;
   for (int j = lane; j < F.R; j += 64) {
-    sum += tri_value_none(F.G, m, nw, L, F.range_fwd[j], F.range_inv[j], w + cut, 0.0, w - cut, 3, 3) -
-           tri_value_none(F.G, m, nw, L, F.range_fwd[j], F.range_inv[j], w - cut, 0.0, w + cut, 3, 3);
+    sum += tri_value_none(F, F.range_fwd[j], F.range_inv[j], w + cut, 0.0, w - cut, 3, 3) -
+           tri_value_none(F, F.range_fwd[j], F.range_inv[j], w - cut, 0.0, w + cut, 3, 3);
   }
   sum = wave_sum(sum);
   if (lane == 0) {
     double v = -2.0 * sum;
     for (int k = 0; k < 4; ++k)
-      v += tri_value_none(F.G, m, nw, L, 0, 0, w + cut, w - cut, 0.0, k, k) -
-           tri_value_none(F.G, m, nw, L, 0, 0, w - cut, w + cut, 0.0, k, k);
+      v += tri_value_none(F, 0, 0, w + cut, w - cut, 0.0, k, k) -
+           tri_value_none(F, 0, 0, w - cut, w + cut, 0.0, k, k);
     v /= (kTwoPi * (cut + sigma_at(m, nw, F.v2, cut)));
     F.dv2[i] = v;
     if (isnan(v)) atomicOr(&F.flags[0], 1);
@@ -724,6 +741,26 @@ __global__ __launch_bounds__(NT, SPFRG_TRI_MIN_BLOCKS) void k_tri_dgamma(TriDev 
   }
 }
 
+#include "tri_rhs.h"
+
+__global__ void k_tri_clear(double2 *p, long long n) {
+  const long long stride = (long long)gridDim.x * blockDim.x;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = make_double2(0.0, 0.0);
+}
+
+// rows of 16 L values between the reference's order (site fastest) and the
+// component-fastest order of G; to_rows: out in the latter
+__global__ void k_tri_reorder(const double *__restrict__ in, double *__restrict__ out, long long n, int L, int to_rows) {
+  const long long stride = (long long)gridDim.x * blockDim.x;
+  const int row = 16 * L;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const long long r = i / row;
+    const int q = (int)(i - r * row);
+    const int c = to_rows ? q & 15 : q / L, site = to_rows ? q >> 4 : q - (q / L) * L;
+    out[i] = in[r * row + (to_rows ? c * L + site : 16 * site + c)];
+  }
+}
+
 // in-place explicit Euler step (src/TRI/TRIFrgCore.cpp:98-120); skipped when
 // the flow holds a NaN (src/SpinParser.cpp:151-159)
 __global__ void k_tri_euler(TriDev F) {
@@ -821,7 +858,7 @@ __global__ __launch_bounds__(kTriThreads) void k_tri_corr_partial(TriDev F) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const double sg = ((d.fl >> (2 + i)) & 1) ? tsign * fsign : tsign;
-          v = fma(sg * d.w[i], G[(size_t)d.off[i] + (4 * a + b) * L + srid], v);
+          v = fma(sg * d.w[i], G[(size_t)d.off[i] + (4 * a + b) * F.cst + srid * F.sst], v);
         }
         r[g] = (c == 15 ? -4.0 : -1.0) * v;
       }
@@ -840,7 +877,7 @@ __global__ __launch_bounds__(kTriThreads) void k_tri_corr_partial(TriDev F) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
             const double sg = ((q.fl >> (2 + i)) & 1) ? tsign * fsign : tsign;
-            x = fma(sg * q.w[i], G[(size_t)q.off[i] + (4 * s1 + s2) * L], x);
+            x = fma(sg * q.w[i], G[(size_t)q.off[i] + (4 * s1 + s2) * F.cst], x);
           }
           v[cc] = x;
         }
@@ -911,6 +948,7 @@ struct sp_tri_ctx {
   double cutoff = 0.0;
   bool have_flow = false;
   size_t lds = 0;
+  double *stage = nullptr;  // rows in the reference's order on their way to and from the host
   std::vector<void *> allocs;
   bool prof = false;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> pending[4];
@@ -939,6 +977,33 @@ template <class T> int talloc(sp_tri_ctx *ctx, T **p, size_t count) {
   if (e != hipSuccess) return tfail(ctx, SP_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
   ctx->allocs.push_back(q);
   *p = static_cast<T *>(q);
+  return SP_OK;
+}
+
+// rows of the staging buffer: at most 32 MiB
+long long tri_stage_rows(const TriDev &f) {
+  const long long rows = (32ll << 20) / (16 * f.L * 8);
+  return rows < f.nf ? rows : f.nf;
+}
+// a vertex from (to_rows) or to the host in the reference's order
+int tri_copy(sp_tri_ctx *ctx, double *dev, double *host, bool to_rows) {
+  const TriDev &F = ctx->fd;
+  if (!ctx->stage) {
+    SP_THIP(hipMemcpy(to_rows ? dev : host, to_rows ? host : dev, (size_t)F.nv * 8,
+                      to_rows ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost));
+    return SP_OK;
+  }
+  const long long rows = tri_stage_rows(F), row = 16 * F.L;
+  for (long long r0 = 0; r0 < F.nf; r0 += rows) {
+    const long long n = (F.nf - r0 < rows ? F.nf - r0 : rows) * row;
+    const dim3 grid((unsigned)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096));
+    if (to_rows) SP_THIP(hipMemcpy(ctx->stage, host + r0 * row, (size_t)n * 8, hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_tri_reorder, grid, dim3(256), 0, ctx->stream, to_rows ? ctx->stage : dev + r0 * row,
+                       to_rows ? dev + r0 * row : ctx->stage, n, F.L, to_rows ? 1 : 0);
+    SP_THIP(hipGetLastError());
+    SP_THIP(hipStreamSynchronize(ctx->stream));
+    if (!to_rows) SP_THIP(hipMemcpy(host + r0 * row, ctx->stage, (size_t)n * 8, hipMemcpyDeviceToHost));
+  }
   return SP_OK;
 }
 
@@ -1031,6 +1096,27 @@ template <int... SH> hipError_t tri_allow_lds(int bytes, std::integer_sequence<i
   return e;
 }
 
+// groups per wave compiled into k_tri_t
+using TriGroups = std::integer_sequence<int, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10>;
+static_assert(TriGroups::size() == kTriMaxGroups, "instantiations of k_tri_t");
+template <int NG> bool launch_tri_t(const TriDev &F, dim3 grid, size_t lds, hipStream_t st) {
+  if (NG != F.t_ng) return false;
+  hipLaunchKernelGGL((k_tri_t<NG>), grid, dim3(64 * F.t_waves), lds, st, F);
+  return true;
+}
+template <int... NG>
+void launch_tri_t(const TriDev &F, dim3 grid, size_t lds, hipStream_t st, std::integer_sequence<int, NG...>) {
+  (launch_tri_t<NG>(F, grid, lds, st) || ...);
+}
+template <int... NG> hipError_t tri_t_allow_lds(int bytes, std::integer_sequence<int, NG...>) {
+  hipError_t e = hipFuncSetAttribute((const void *)k_tri_su, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  ((e == hipSuccess ? (e = hipFuncSetAttribute((const void *)k_tri_t<NG>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               bytes))
+                    : e),
+   ...);
+  return e;
+}
+
 hipError_t tri_launch_compute(sp_tri_ctx *ctx) {
   TriDev &F = ctx->fd;
   F.cut = ctx->cutoff;
@@ -1045,8 +1131,22 @@ hipError_t tri_launch_compute(sp_tri_ctx *ctx) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   TriProf ps(ctx, 0);
-  const long long rounds = (F.nf + 8 * kTriChunk - 1) / (8 * kTriChunk);
-  const dim3 grid((unsigned)(rounds * 8 * kTriChunk));
+  auto grid_of = [](long long n) {
+    const long long rounds = (n + 8 * kTriChunk - 1) / (8 * kTriChunk);
+    return dim3((unsigned)(rounds * 8 * kTriChunk));
+  };
+  const dim3 grid = grid_of(F.nf);
+  if (F.t_waves) {
+    long long blocks = (F.nv / 2 + 255) / 256;
+    if (blocks > 4096) blocks = 4096;
+    hipLaunchKernelGGL(k_tri_clear, dim3((unsigned)blocks), dim3(256), 0, ctx->stream,
+                       reinterpret_cast<double2 *>(F.dG), F.nv / 2);
+    const long long teams = (su_units(F.nw) + kRhsWaves - 1) / kRhsWaves;
+    hipLaunchKernelGGL(k_tri_su, grid_of(teams), dim3(64 * kRhsWaves),
+                       (size_t)(((F.nw * 8 + 15) & ~15) + kRhsWaves * tri_su_wave_bytes(F.L)), ctx->stream, F, teams);
+    launch_tri_t(F, grid, ctx->lds, ctx->stream, TriGroups{});
+    return hipGetLastError();
+  }
   if (F.nt == kTriSmallThreads)
     launch_tri_small(F, grid, ctx->lds, ctx->stream, TriShapes{});
   else
@@ -1068,6 +1168,9 @@ int sp_tri_ctx_footprint(const sp_tri_problem *p, long long *bytes) {
   b += 2 * (long long)p->nw * emax * 8 + 2 * emax * 8 + (p->nw + 1) * 4;      // weight tables
   b += emax * 10 * p->L * 8 + 10LL * p->B * p->Rb * 8 + 16;                   // correlation scratch, output, flags
   b += 4LL * (10 * p->L + 1 + 5 * O + 2 * p->R + 4 * p->B * p->Rb);           // lattice tables
+  if (p->L <= kMaxTriRhsL)
+    b += std::min<long long>(nf * 16 * p->L * 8, 32ll << 20) + 4LL * 32 * p->L +
+         64LL * 16 * 8 * kTriMaxGroups + 64LL * (32 * p->L + 512 + O);  // staging rows, tables of the T kernel
   *bytes = b;
   return SP_OK;
 }
@@ -1102,8 +1205,25 @@ int sp_tri_ctx_create(const sp_tri_problem *p, sp_tri_ctx **out) {
     if (tri_shape_compiled(cs, f.nb, TriShapes{}) && tri_lds(f.nw, f.L, cs, f.nb).total <= kTriLdsBudget) f.cs = cs;
   }
   ctx->lds = (size_t)tri_lds(f.nw, f.L, f.cs, f.nb).total;
+  f.cst = f.L;
+  f.sst = 1;
   int max_lds = 0;
   SP_THIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device));
+  TriPlan plan;
+  try {
+    plan = build_tri_plan(p);
+  } catch (...) { return tfail(ctx, SP_ENOMEM, "host buffer"); }
+  if (plan.ok && plan.lds <= max_lds && ((f.nw * 8 + 15) & ~15) + kRhsWaves * tri_su_wave_bytes(f.L) <= max_lds) {
+    f.t_waves = plan.waves;
+    f.t_ng = plan.ng;
+    f.t_points = plan.points;
+    f.t_entries = plan.entries;
+    f.t_edges = plan.edges;
+    f.t_pass = plan.pass;
+    f.cst = 1;
+    f.sst = 16;
+    ctx->lds = (size_t)plan.lds;
+  }
   if (ctx->lds > (size_t)max_lds) return tfail(ctx, SP_EARG, "problem too large for the LDS plan of the dGamma kernel");
   if (f.nv * 8 >= (1LL << 31)) return tfail(ctx, SP_EARG, "vertex too large for 32-bit byte offsets");
   f.g_bytes = (unsigned)(f.nv * 8);
@@ -1171,7 +1291,8 @@ int sp_tri_ctx_create(const sp_tri_problem *p, sp_tri_ctx **out) {
   });
   int *site = nullptr, *sitep = nullptr, *inv = nullptr, *invp = nullptr, *goff = nullptr, *bent = nullptr,
       *rf = nullptr, *ri = nullptr, *corr = nullptr, *corrp = nullptr, *sorder = nullptr;
-  int4 *bgrp = nullptr;
+  int4 *bgrp = nullptr, *tops = nullptr;
+  int *tdst = nullptr, *tplan = nullptr, *tedge = nullptr;
   if ((rc = talloc(ctx, &mesh, f.nw)) || (rc = talloc(ctx, &site, f.L)) || (rc = talloc(ctx, &sitep, 3 * f.L)) ||
       (rc = talloc(ctx, &inv, f.L)) || (rc = talloc(ctx, &invp, 3 * f.L)) || (rc = talloc(ctx, &goff, f.L + 1)) ||
       (rc = talloc(ctx, &sorder, f.L)) ||
@@ -1182,8 +1303,15 @@ int sp_tri_ctx_create(const sp_tri_problem *p, sp_tri_ctx **out) {
       (rc = talloc(ctx, &f.Wwp, (size_t)f.nw * emax)) || (rc = talloc(ctx, &f.Wc, (size_t)f.nw * emax)) ||
       (rc = talloc(ctx, &f.Wn, f.nw)) || (rc = talloc(ctx, &f.Cwp, emax)) || (rc = talloc(ctx, &f.Cw, emax)) ||
       (rc = talloc(ctx, &f.Cn, 1)) || (rc = talloc(ctx, &f.corr_partial, (size_t)emax * 10 * f.L)) ||
-      (rc = talloc(ctx, &f.corr_out, 10 * nc)) || (rc = talloc(ctx, &f.flags, 4)))
+      (rc = talloc(ctx, &f.corr_out, 10 * nc)) || (rc = talloc(ctx, &f.flags, 4)) ||
+      (f.t_waves && ((rc = talloc(ctx, &tdst, plan.dst.size())) || (rc = talloc(ctx, &tedge, plan.edge_ops.size())) || (rc = talloc(ctx, &tplan, plan.plan.size())) ||
+                     (rc = talloc(ctx, &tops, plan.ops.size())) ||
+                     (rc = talloc(ctx, &ctx->stage, (size_t)tri_stage_rows(f) * 16 * f.L)))))
     return rc;
+  f.t_dst = tdst;
+  f.t_edge_ops = tedge;
+  f.t_plan = tplan;
+  f.t_ops = tops;
   f.mesh = mesh;
   f.site_rid = site;
   f.site_perm = sitep;
@@ -1211,6 +1339,13 @@ int sp_tri_ctx_create(const sp_tri_problem *p, sp_tri_ctx **out) {
     SP_THIP(hipMemcpy(bent, ent.data(), ent.size() * 4, hipMemcpyHostToDevice));
     SP_THIP(hipMemcpy(bgrp, grp.data(), grp.size() * sizeof(int4), hipMemcpyHostToDevice));
   }
+  if (f.t_waves) {
+    SP_THIP(hipMemcpy(tdst, plan.dst.data(), plan.dst.size() * 4, hipMemcpyHostToDevice));
+    SP_THIP(hipMemcpy(tplan, plan.plan.data(), plan.plan.size() * 4, hipMemcpyHostToDevice));
+    if (!plan.edge_ops.empty())
+      SP_THIP(hipMemcpy(tedge, plan.edge_ops.data(), plan.edge_ops.size() * 4, hipMemcpyHostToDevice));
+    SP_THIP(hipMemcpy(tops, plan.ops.data(), plan.ops.size() * sizeof(int4), hipMemcpyHostToDevice));
+  }
   SP_THIP(hipMemcpy(rf, p->range_fwd, (size_t)f.R * 4, hipMemcpyHostToDevice));
   SP_THIP(hipMemcpy(ri, p->range_inv, (size_t)f.R * 4, hipMemcpyHostToDevice));
   SP_THIP(hipMemcpy(corr, p->corr_rid, nc * 4, hipMemcpyHostToDevice));
@@ -1225,6 +1360,7 @@ int sp_tri_ctx_create(const sp_tri_problem *p, sp_tri_ctx **out) {
   SP_THIP(hipFuncSetAttribute((const void *)k_tri_dgamma<kTriThreads, 0, 0>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
   SP_THIP(tri_allow_lds(max_lds, TriShapes{}));
+  SP_THIP(tri_t_allow_lds(max_lds, TriGroups{}));
   return SP_OK;
 }
 
@@ -1244,7 +1380,7 @@ int sp_tri_set_state(sp_tri_ctx *ctx, double cutoff, const double *v2, const dou
   if (!std::isfinite(cutoff) || !(cutoff > 0.0)) return tfail(ctx, SP_EARG, "cutoff must be finite and positive");
   SP_THIP(hipStreamSynchronize(ctx->stream));
   SP_THIP(hipMemcpy(ctx->fd.v2, v2, ctx->fd.nw * 8, hipMemcpyHostToDevice));
-  SP_THIP(hipMemcpy(ctx->fd.G, v4, (size_t)ctx->fd.nv * 8, hipMemcpyHostToDevice));
+  if (int rc = tri_copy(ctx, ctx->fd.G, const_cast<double *>(v4), true)) return rc;
   SP_THIP(hipMemset(ctx->fd.flags, 0, 16));
   ctx->cutoff = cutoff;
   ctx->have_flow = false;
@@ -1256,7 +1392,8 @@ int sp_tri_get_state(sp_tri_ctx *ctx, double *cutoff, double *v2, double *v4) {
   SP_THIP(hipStreamSynchronize(ctx->stream));
   if (cutoff) *cutoff = ctx->cutoff;
   if (v2) SP_THIP(hipMemcpy(v2, ctx->fd.v2, ctx->fd.nw * 8, hipMemcpyDeviceToHost));
-  if (v4) SP_THIP(hipMemcpy(v4, ctx->fd.G, (size_t)ctx->fd.nv * 8, hipMemcpyDeviceToHost));
+  if (v4)
+    if (int rc = tri_copy(ctx, ctx->fd.G, v4, false)) return rc;
   return SP_OK;
 }
 
@@ -1265,7 +1402,8 @@ int sp_tri_get_flow(sp_tri_ctx *ctx, double *dv2, double *dv4) {
   if (!ctx->have_flow) return tfail(ctx, SP_ESTATE, "no flow computed at the current cutoff");
   SP_THIP(hipStreamSynchronize(ctx->stream));
   if (dv2) SP_THIP(hipMemcpy(dv2, ctx->fd.dv2, ctx->fd.nw * 8, hipMemcpyDeviceToHost));
-  if (dv4) SP_THIP(hipMemcpy(dv4, ctx->fd.dG, (size_t)ctx->fd.nv * 8, hipMemcpyDeviceToHost));
+  if (dv4)
+    if (int rc = tri_copy(ctx, ctx->fd.dG, dv4, false)) return rc;
   return SP_OK;
 }
 
