@@ -311,15 +311,18 @@ __global__ __launch_bounds__(64 * kRhsWaves, 4) void k_su(const FlowDev *__restr
 // T channel and the final sum
 // ---------------------------------------------------------------------------
 // A wave evaluates the T channel of an item, eight points at a time, its lanes
-// in the operand layout of the 16 x 16 x 4 FP64 matrix instruction (lane l =
+// in the operand layout of the FP64 matrix instructions (lane l =
 // row l % 16 of point l / 16): the gathered values are the operands of the
 // lattice-bubble update C[a][b] += sum_e P_e[a] Q_e[b] without a pass through
 // LDS.  Sites come in FT full tiles of 16 and, with HT, a half tile of 8 whose
 // lanes take eight points at once; in the matrix operands its even points sit
-// in rows 0-7 and its odd points in rows 8-15.  The matrix instructions run at
+// in rows 0-7 and its odd points in rows 8-15.  The blocks of 4 x 4 that the
+// overlap lists need are updated and no others: 36 instructions for eight points
+// and both channels at L = 23 (612 cycles of a SIMD; 14 of 16 x 16 x 4 took 1800,
+// cubic r6 at cutoff 60 0.987 -> 0.967 ms).  The matrix instructions run at
 // the vector FP64 rate; what they save is the LDS traffic of a rank update from
-// shared factors.  Two tiles need 64 registers of sums: three waves per SIMD
-// (two: 5 to 8 % slower at L = 23), single tiles four.
+// shared factors.  Two tiles: three waves per SIMD (two: 5 to 8 % slower at
+// L = 23), single tiles four.
 struct TShape {
   int ft, ht, lp;  // full tiles, half tile, row stride of the bubble matrix
 };
@@ -401,9 +404,17 @@ __global__ __launch_bounds__(64 * kRhsWaves, FT + HT == 1 ? 4 : 3) void k_t(cons
   double rs[NT], rd[NT];
 #pragma unroll
   for (int k = 0; k < NT; ++k) rs[k] = rd[k] = 0.0;
-  d4 C[2][NT * NT];
+  // bubble matrix: full tiles, full rows x half columns, half rows x full columns, half tile
+  d4 C[2][FT ? FT * FT : 1];
+  double2 Cr[2][FT ? FT : 1], Cc[2][FT ? FT : 1], Ch[2];
 #pragma unroll
-  for (int k = 0; k < NT * NT; ++k) C[0][k] = C[1][k] = d4{0.0, 0.0, 0.0, 0.0};
+  for (int ch = 0; ch < 2; ++ch) {
+#pragma unroll
+    for (int k = 0; k < FT * FT; ++k) C[ch][k] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < FT; ++k) Cr[ch][k] = Cc[ch][k] = make_double2(0.0, 0.0);
+    Ch[ch] = make_double2(0.0, 0.0);
+  }
 
   // producer role: point pe, pair pp, argument pj: A (pj 0) and B (pj 1) of
   // pair 0: A = w1 - w', B = w1p + w'; pair 1: A = w2p - w', B = w2 + w'
@@ -553,12 +564,12 @@ __global__ __launch_bounds__(64 * kRhsWaves, FT + HT == 1 ? 4 : 3) void k_t(cons
         gather(FT, eb + (lane >> 3), ph, qh);
 #pragma unroll
         for (int ch = 0; ch < 2; ++ch) {
-          d4 &m = C[ch][NT * NT - 1];
-          m = __builtin_amdgcn_mfma_f64_16x16x4f64(ph[ch], qh[ch], m, 0, 0, 0);
+          // even and odd points in blocks of their own
+          Ch[ch].x = mfma_blocks(ph[ch], qh[ch], Ch[ch].x);
+          Ch[ch].y = mfma_blocks(ph[ch], half_mirror(qh[ch]), Ch[ch].y);
         }
       }
-      // the full tiles' even points, then the odd ones (the half tile's rows
-      // exchanged, so that its odd points meet them)
+      // the full tiles' even points, then the odd ones
 #pragma unroll
       for (int par = 0; par < (FT ? 2 : 0); ++par) {
         double P[FT ? FT : 1][2], Q[FT ? FT : 1][2];
@@ -569,21 +580,18 @@ __global__ __launch_bounds__(64 * kRhsWaves, FT + HT == 1 ? 4 : 3) void k_t(cons
 #pragma unroll
           for (int i = 0; i < FT; ++i)
 #pragma unroll
-            for (int j = 0; j < FT; ++j) {
-              d4 &m = C[ch][i * NT + j];
-              m = __builtin_amdgcn_mfma_f64_16x16x4f64(P[i][ch], Q[j][ch], m, 0, 0, 0);
-            }
+            for (int j = 0; j < FT; ++j) outer_update(C[ch][i * FT + j], P[i][ch], Q[j][ch]);
           if (HT) {
-            if (par) {
-              ph[ch] = half_row_swap(ph[ch]);
-              qh[ch] = half_row_swap(qh[ch]);
-            }
+            // the half tile at these points in both halves of the rows
+            const double p = par ? row_move<0x128, 0x3>(ph[ch]) : row_move<0x128, 0xc>(ph[ch]);
+            const double q = par ? row_move<0x128, 0x3>(qh[ch]) : row_move<0x128, 0xc>(qh[ch]);
+            const double pm = half_mirror(p), qm = half_mirror(q);
 #pragma unroll
             for (int i = 0; i < FT; ++i) {
-              d4 &m = C[ch][i * NT + FT];
-              m = __builtin_amdgcn_mfma_f64_16x16x4f64(P[i][ch], qh[ch], m, 0, 0, 0);
-              d4 &mt = C[ch][FT * NT + i];
-              mt = __builtin_amdgcn_mfma_f64_16x16x4f64(ph[ch], Q[i][ch], mt, 0, 0, 0);
+              Cr[ch][i].x = mfma_blocks(P[i][ch], q, Cr[ch][i].x);
+              Cr[ch][i].y = mfma_blocks(P[i][ch], qm, Cr[ch][i].y);
+              Cc[ch][i].x = mfma_blocks(p, Q[i][ch], Cc[ch][i].x);
+              Cc[ch][i].y = mfma_blocks(pm, Q[i][ch], Cc[ch][i].y);
             }
           }
         }
@@ -595,29 +603,36 @@ __global__ __launch_bounds__(64 * kRhsWaves, FT + HT == 1 ? 4 : 3) void k_t(cons
   // RPA(rid) = sum over getOverlap(rid) of C[rid1][rid2] (src/SU2/SU2FrgCore.cpp:250-266)
   double *s_C = reinterpret_cast<double *>(wl);
   double *s_part = s_C + LP * LP;
-  const int cnt = F.plan_count[lane], row0 = lane >> 4, col = lane & 15;
+  const int cnt = F.plan_count[lane];
+  // lane (ri, b, rj) holds elements (4 b + ri, rj of another block of columns)
+  const int ri = lane >> 4, cb = (lane >> 2) & 3, rj = lane & 3;
   double rpa[2] = {0.0, 0.0};
 #pragma unroll
   for (int ch = 0; ch < 2; ++ch) {
     wave_lds_fence();
 #pragma unroll
-    for (int i = 0; i < NT; ++i)
+    for (int i = 0; i < FT; ++i) {
+      const int row = (16 * i + 4 * cb + ri) * LP;
 #pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        const d4 m = C[ch][i * NT + j];
-        if (i == FT && j == FT) {
-          // even points in the first, odd points in the last 8 x 8 block
-          const double v0 = m[0] + half_row_swap(m[2]), v1 = m[1] + half_row_swap(m[3]);
-          if (col < 8) {
-            s_C[(16 * FT + row0) * LP + 16 * FT + col] = v0;
-            s_C[(16 * FT + 4 + row0) * LP + 16 * FT + col] = v1;
-          }
-        } else {
+      for (int j = 0; j < FT; ++j)
 #pragma unroll
-          for (int z = 0; z < 4; ++z)
-            if ((i < FT || z < 2) && (j < FT || col < 8)) s_C[(16 * i + 4 * z + row0) * LP + 16 * j + col] = m[z];
-        }
+        for (int z = 0; z < 4; ++z) s_C[row + 16 * j + 4 * ((cb + z) & 3) + rj] = C[ch][i * FT + j][z];
+      if (HT) {
+        const int h = 16 * FT, lo = 4 * (cb & 1), hi = 4 * (1 - (cb & 1)) + 3;
+        s_C[row + h + lo + rj] = Cr[ch][i].x;
+        s_C[row + h + hi - rj] = Cr[ch][i].y;
+        s_C[(h + lo + ri) * LP + 16 * i + 4 * cb + rj] = Cc[ch][i].x;
+        s_C[(h + hi - ri) * LP + 16 * i + 4 * cb + rj] = Cc[ch][i].y;
       }
+    }
+    if (HT) {
+      const double x = Ch[ch].x + half_row_swap(Ch[ch].x), y = Ch[ch].y + half_row_swap(Ch[ch].y);
+      if (cb < 2) {
+        double *o = s_C + (16 * FT + 4 * cb + ri) * LP + 16 * FT;
+        o[4 * cb + rj] = x;
+        o[4 * (1 - cb) + 3 - rj] = y;
+      }
+    }
     wave_lds_fence();
     s_part[lane] = plan_sum(reinterpret_cast<const uint4 *>(F.plan_ent) + lane, 64, cnt, s_C);
     wave_lds_fence();
