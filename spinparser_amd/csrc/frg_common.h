@@ -19,24 +19,6 @@ constexpr double kTwoPi = 2.0 * kPi;
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double mesh_at(const double *m, int i) { return i >= 0 ? m[i] : -m[-i - 1]; }
 
-__device__ inline int greater_pos(const double *m, int n, double w) {
-  if (w <= m[0]) return 0;
-  for (int i = 1; i < n; ++i)
-    if (m[i] > w) return i;
-  return n - 1;
-}
-
-__device__ inline int lesser_pos(const double *m, int n, double w) {
-  if (w <= m[0]) return 0;
-  for (int i = 1; i < n; ++i)
-    if (m[i] > w) return i - 1;
-  return n - 1;
-}
-
-// FrequencyDiscretization::lesser / greater (src/FrequencyDiscretization.hpp:253-296)
-__device__ inline int mesh_lesser(const double *m, int n, double w) { return w < 0 ? -(greater_pos(m, n, -w) + 1) : lesser_pos(m, n, w); }
-__device__ inline int mesh_greater(const double *m, int n, double w) { return w < 0 ? -(lesser_pos(m, n, -w) + 1) : greater_pos(m, n, w); }
-
 // number of mesh points <= w (branch-free binary lifting)
 __device__ __forceinline__ int count_le(const double *m, int n, double w) {
   int pos = 0;
@@ -46,6 +28,19 @@ __device__ __forceinline__ int count_le(const double *m, int n, double w) {
   }
   return pos;
 }
+
+// first mesh point > w, and the one before it, within [0, n)
+__device__ inline int greater_pos(const double *m, int n, double w) {
+  if (w <= m[0]) return 0;
+  const int c = count_le(m, n, w);
+  return c < n ? c : n - 1;
+}
+
+__device__ inline int lesser_pos(const double *m, int n, double w) { return w <= m[0] ? 0 : count_le(m, n, w) - 1; }
+
+// FrequencyDiscretization::lesser / greater (src/FrequencyDiscretization.hpp:253-296)
+__device__ inline int mesh_lesser(const double *m, int n, double w) { return w < 0 ? -(greater_pos(m, n, -w) + 1) : lesser_pos(m, n, w); }
+__device__ inline int mesh_greater(const double *m, int n, double w) { return w < 0 ? -(lesser_pos(m, n, -w) + 1) : greater_pos(m, n, w); }
 
 // FrequencyDiscretization::interpolateOffset (src/FrequencyDiscretization.hpp:326-356)
 // (written as !(w > m[0]) so that a NaN argument clamps to index 0 instead of
@@ -77,132 +72,138 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 // ---------------------------------------------------------------------------
 // trapezoid windows: evaluation points and weights (0.5 folded in), in the
-// order ImplicitIntegrator visits them (src/lib/Integrator.hpp:137-287)
+// order ImplicitIntegrator visits them (src/lib/Integrator.hpp:137-287).  A
+// window is its two end indices and its number of points; every point follows
+// from its position, so that lanes form them side by side.
 // ---------------------------------------------------------------------------
-struct PointList {
-  double *wp;
-  double *w;
-  int cnt;
-  int cap;
-  __device__ inline void push(double x, double weight) {
-    if (cnt < cap) { wp[cnt] = x; w[cnt] = weight; }
-    ++cnt;
-  }
+struct PointWeight {
+  double x, w;
+};
+struct Window {
+  double min, max;
+  int lo, hi, cnt;
 };
 
-__device__ inline void window_right(const double *m, int n, double max, PointList &o) {
-  int umin = -n;
-  const int umax = mesh_lesser(m, n, max);
-  if (umin != umax) {
-    o.push(mesh_at(m, umin), 0.5 * (mesh_at(m, umin + 1) - mesh_at(m, umin)));
-    while (++umin != umax) o.push(mesh_at(m, umin), 0.5 * (mesh_at(m, umin + 1) - mesh_at(m, umin - 1)));
-    o.push(mesh_at(m, umin), 0.5 * (max - mesh_at(m, umin - 1)));
-    o.push(max, 0.5 * (max - mesh_at(m, umin)));
-  } else {
-    const double h = 0.5 * (max - mesh_at(m, umin));
-    o.push(max, h);
-    o.push(mesh_at(m, umin), h);
-  }
+// (-inf, max]
+__device__ inline Window window_right(const double *m, int n, double max) {
+  const int hi = mesh_lesser(m, n, max);
+  return Window{0.0, max, -n, hi, hi != -n ? hi + n + 2 : 2};
 }
-
-__device__ inline void window_both(const double *m, int n, double min, double max, PointList &o) {
-  int umin = mesh_greater(m, n, min);
-  const int umax = mesh_lesser(m, n, max);
-  if (umax >= umin) {
-    o.push(min, 0.5 * (mesh_at(m, umin) - min));
-    if (umax != umin) {
-      o.push(mesh_at(m, umin), 0.5 * (mesh_at(m, umin + 1) - min));
-      while (++umin != umax) o.push(mesh_at(m, umin), 0.5 * (mesh_at(m, umin + 1) - mesh_at(m, umin - 1)));
-      o.push(mesh_at(m, umin), 0.5 * (max - mesh_at(m, umin - 1)));
-    } else {
-      o.push(mesh_at(m, umin), 0.5 * (max - min));
-    }
-    o.push(max, 0.5 * (max - mesh_at(m, umin)));
-  } else {
-    const double h = 0.5 * (max - min);
-    o.push(max, h);
-    o.push(min, h);
-  }
+__device__ inline PointWeight right_point(const double *m, const Window &w, int k) {
+  const double first = mesh_at(m, w.lo);
+  if (w.hi == w.lo) return PointWeight{k == 0 ? w.max : first, 0.5 * (w.max - first)};
+  const int i = w.lo + k;
+  if (i > w.hi) return PointWeight{w.max, 0.5 * (w.max - mesh_at(m, w.hi))};
+  const double up = i == w.hi ? w.max : mesh_at(m, i + 1), down = mesh_at(m, i == w.lo ? i : i - 1);
+  return PointWeight{mesh_at(m, i), 0.5 * (up - down)};
 }
-
-__device__ inline void window_left(const double *m, int n, double min, PointList &o) {
-  int umin = mesh_greater(m, n, min);
-  const int max = n - 1;
-  if (umin != max) {
-    o.push(min, 0.5 * (mesh_at(m, umin) - min));
-    o.push(mesh_at(m, umin), 0.5 * (mesh_at(m, umin + 1) - min));
-    while (++umin != max) o.push(mesh_at(m, umin), 0.5 * (mesh_at(m, umin + 1) - mesh_at(m, umin - 1)));
-    o.push(mesh_at(m, umin), 0.5 * (mesh_at(m, umin) - mesh_at(m, umin - 1)));
-  } else {
-    const double h = 0.5 * (mesh_at(m, umin) - min);
-    o.push(min, h);
-    o.push(mesh_at(m, umin), h);
-  }
+// [min, max]
+__device__ inline Window window_both(const double *m, int n, double min, double max) {
+  const int lo = mesh_greater(m, n, min), hi = mesh_lesser(m, n, max);
+  return Window{min, max, lo, hi, hi >= lo ? hi - lo + 3 : 2};
 }
-
-// the three Katanin windows of a channel with transfer frequency X
-// (src/SU2/SU2FrgCore.cpp:378-392; with X = nu = 0 the correlation windows,
-// src/SU2/SU2MeasurementCorrelation.cpp:145-159)
-__device__ inline void katanin_windows(const double *m, int n, double X, double cut, PointList &o) {
-  if (-(X + cut) > mesh_at(m, -n)) window_right(m, n, -(X + cut), o);
-  if (X - cut > cut) window_both(m, n, cut - X, -cut, o);
-  if (cut < mesh_at(m, n - 1)) window_left(m, n, cut, o);
+__device__ inline PointWeight both_point(const double *m, const Window &w, int k) {
+  if (w.hi < w.lo) return PointWeight{k == 0 ? w.max : w.min, 0.5 * (w.max - w.min)};
+  if (k == 0) return PointWeight{w.min, 0.5 * (mesh_at(m, w.lo) - w.min)};
+  const int i = w.lo + k - 1;
+  if (i > w.hi) return PointWeight{w.max, 0.5 * (w.max - mesh_at(m, w.hi))};
+  const double up = i == w.hi ? w.max : mesh_at(m, i + 1), down = i == w.lo ? w.min : mesh_at(m, i - 1);
+  return PointWeight{mesh_at(m, i), 0.5 * (up - down)};
+}
+// [min, inf)
+__device__ inline Window window_left(const double *m, int n, double min) {
+  const int lo = mesh_greater(m, n, min);
+  return Window{min, 0.0, lo, n - 1, lo != n - 1 ? n - lo + 1 : 2};
+}
+__device__ inline PointWeight left_point(const double *m, const Window &w, int k) {
+  if (k == 0) return PointWeight{w.min, 0.5 * (mesh_at(m, w.lo) - w.min)};
+  const int i = w.lo + k - 1;
+  if (w.lo == w.hi) return PointWeight{mesh_at(m, i), 0.5 * (mesh_at(m, i) - w.min)};
+  const double up = mesh_at(m, i == w.hi ? i : i + 1), down = i == w.lo ? w.min : mesh_at(m, i - 1);
+  return PointWeight{mesh_at(m, i), 0.5 * (up - down)};
 }
 
 // Evaluation points and weights of one channel with exact transfer frequency
 // m[x] at cutoff cut: the conventional points +-cut with p(cut, cut +- X)
 // (src/SU2/SU2FrgCore.cpp:349-371, src/TRI/TRIFrgCore.cpp:2917-2940), then the
-// Katanin windows with dSigma(w') G(w')^2 G(X + w') folded into the trapezoid
-// weight (src/SU2/SU2FrgCore.cpp:343-347,373-424).  Depends on (x, cut) only,
-// so every item of a flow shares the table.
+// three Katanin windows (src/SU2/SU2FrgCore.cpp:378-392) with
+// dSigma(w') G(w')^2 G(X + w') folded into the trapezoid weight
+// (src/SU2/SU2FrgCore.cpp:343-347,373-424).  Depends on (x, cut) only, so every
+// item of a flow shares the table.
 //
 // weight_tables_wave: one 64-lane workgroup per table, x < nw a channel list,
-// x == nw the plain trapezoid list of the correlation integrals at nu = 0
-// (src/SU2/SU2MeasurementCorrelation.cpp:145-159,
+// x == nw the plain trapezoid list of the correlation integrals at nu = 0 (the
+// windows with X = 0; src/SU2/SU2MeasurementCorrelation.cpp:145-159,
 // src/TRI/TRIMeasurementCorrelation.cpp:270-284).  s_m is LDS space for the
-// nw mesh values; lane 0 builds the point list (the window walks are
-// sequential), then the lanes fold the Katanin weights of its points in
-// parallel.  *overflow is raised if a list exceeds emax entries.
+// nw mesh values.  *overflow is raised if a list exceeds emax entries.  What
+// bounds it is latency: one lane that walked the windows in turn took 18 us
+// (32 frequencies).
 __device__ inline void weight_tables_wave(int x, const double *mesh, int nw, double cut, const double *v2,
                                           const double *dv2, double *Wwp, double *Wc, int *Wn, double *Cwp,
                                           double *Cw, int *Cn, int emax, int *overflow, double *s_m) {
-  __shared__ int s_k[2];
   const int lane = threadIdx.x;
   for (int i = lane; i < nw; i += 64) s_m[i] = mesh[i];
   __syncthreads();
   const double *m = s_m;
-  if (x == nw) {
-    if (lane == 0) {
-      PointList o{Cwp, Cw, 0, emax};
-      katanin_windows(m, nw, 0.0, cut, o);
-      *Cn = o.cnt < emax ? o.cnt : emax;
-      if (o.cnt > emax) atomicOr(overflow, 1);
-    }
-    return;
-  }
-  const double X = m[x];
-  double *wp = Wwp + (size_t)x * emax, *w = Wc + (size_t)x * emax;
-  if (lane == 0) {
-    PointList o{wp, w, 0, emax};
-    auto p = [&](double a, double b) { return 1.0 / ((a + sigma_at(m, nw, v2, a)) * (b + sigma_at(m, nw, v2, b))); };
-    o.push(cut, p(cut, cut + X));
-    if (X > 2.0 * cut) o.push(-cut, p(cut, cut - X));
-    s_k[0] = o.cnt;
-    katanin_windows(m, nw, X, cut, o);
-    s_k[1] = o.cnt;
-  }
-  __syncthreads();  // the list in global memory is visible to the workgroup
-  const int k0 = s_k[0], cnt = s_k[1];
+  const bool plain = x == nw;
+  const double X = plain ? 0.0 : m[x];
+  double *wp = plain ? Cwp : Wwp + (size_t)x * emax, *w = plain ? Cw : Wc + (size_t)x * emax;
+  const int k0 = plain ? 0 : (X > 2.0 * cut ? 2 : 1);
+  const bool right = -(X + cut) > mesh_at(m, -nw), both = X - cut > cut, left = cut < mesh_at(m, nw - 1);
+  Window R{}, B{}, Lw{};
+  if (right) R = window_right(m, nw, -(X + cut));
+  if (both) B = window_both(m, nw, cut - X, -cut);
+  if (left) Lw = window_left(m, nw, cut);
+  const int k1 = k0 + R.cnt, k2 = k1 + B.cnt, cnt = k2 + Lw.cnt;
   const int kend = cnt < emax ? cnt : emax;
-  for (int k = k0 + lane; k < kend; k += 64) {
-    const double e = wp[k];
-    const double d1 = e + sigma_at(m, nw, v2, e);
-    w[k] *= sigma_at(m, nw, dv2, e) / (d1 * d1 * (X + e + sigma_at(m, nw, v2, X + e)));
+  for (int k = lane; k < kend; k += 64) {
+    if (k < k0) {
+      const double b = k ? cut - X : cut + X;
+      wp[k] = k ? -cut : cut;
+      w[k] = 1.0 / ((cut + sigma_at(m, nw, v2, cut)) * (b + sigma_at(m, nw, v2, b)));
+      continue;
+    }
+    const PointWeight q = k < k1 ? right_point(m, R, k - k0) : (k < k2 ? both_point(m, B, k - k1) : left_point(m, Lw, k - k2));
+    wp[k] = q.x;
+    if (plain) {
+      w[k] = q.w;
+    } else {
+      const double d1 = q.x + sigma_at(m, nw, v2, q.x);
+      w[k] = q.w * (sigma_at(m, nw, dv2, q.x) / (d1 * d1 * (X + q.x + sigma_at(m, nw, v2, X + q.x))));
+    }
   }
   if (lane == 0) {
-    Wn[x] = kend;
+    (plain ? *Cn : Wn[x]) = kend;
     if (cnt > emax) atomicOr(overflow, 1);
   }
+}
+
+constexpr int kSigmaThreads = 320;  // workgroup of the dSigma kernels: four waves of the range sum and one
+
+// correlation kernels: workgroup, of which the first threads evaluate the
+// site-local vertices and the rest (point, site) pairs
+constexpr int kCorrThreads = 1024, kCorrEggs = 128, kCorrPoints = kCorrThreads - kCorrEggs;
+
+// out[q] = sum over o < n of partial[o * nq + q] by a workgroup (nq <= 1024):
+// the points dealt to the threads of an output, so that one waits for n / 8
+// loads or fewer where there are threads for it
+__device__ inline void sum_partials(const double *partial, int n, int nq, double *out) {
+  __shared__ double part[1024];
+  const int nt = blockDim.x, tid = threadIdx.x;
+  const int parts = nq < nt ? (nt / nq < 1024 / nq ? nt / nq : 1024 / nq) : 1;
+  for (int k = tid; k < parts * nq; k += nt) {
+    const int q = k % nq;
+    double v = 0.0;
+    for (int o = k / nq; o < n; o += parts) v += partial[(size_t)o * nq + q];
+    part[k] = v;
+  }
+  __syncthreads();
+  for (int q = tid; q < nq; q += nt) {
+    double v = part[q];
+    for (int p = 1; p < parts; ++p) v += part[p * nq + q];
+    out[q] = v;
+  }
+  __syncthreads();
 }
 
 // ---------------------------------------------------------------------------

@@ -195,7 +195,8 @@ struct FlowDev {
   double *Cwp, *Cw;
   int *Cn;
   double *corr_partial, *corr_out;
-  int *flags;  // [0] NaN in the flow, [1] evaluation-list overflow, [2] stopped flow,
+  int *flags;  // [0] NaN in the flow, [1] evaluation-list overflow, [2] stopped flow, [3] [0] of
+               // the step whose update is queued (sp_run_flow),
                // [4] scale exponent S of the FP32 shadow (G32 = G * 2^-S), [5] largest
                // binary exponent of G written since the last plan, [6] planned S
   int nw, L, R, B, Rb, emax, nb, slots, precision, euler;
@@ -240,41 +241,46 @@ __global__ __launch_bounds__(64) void k_weights(const FlowDev *__restrict__ fl, 
 }
 
 // ---------------------------------------------------------------------------
-// dSigma/dLambda (src/SU2/SU2FrgCore.cpp:139-169): one 256-thread workgroup
-// per mesh point, the range sum spread over its four waves; the mesh in LDS
-// (dynamic, nw doubles)
+// dSigma/dLambda (src/SU2/SU2FrgCore.cpp:139-169): one workgroup per mesh
+// point, the range sum spread over its first four waves, the two site-local
+// values on lanes of the fifth beside them; the mesh in LDS (dynamic, nw doubles)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_dsigma(const FlowDev *__restrict__ fl) {
+__global__ __launch_bounds__(kSigmaThreads) void k_dsigma(const FlowDev *__restrict__ fl) {
   extern __shared__ double s_dmesh[];
-  __shared__ double part[4];
+  __shared__ double part[8];
   const FlowDev &F = fl[blockIdx.y];
   const int i = blockIdx.x;
   if (i >= F.nw) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int nw = F.nw, L = F.L;
-  for (int k = tid; k < nw; k += 256) s_dmesh[k] = F.mesh[k];
+  for (int k = tid; k < nw; k += kSigmaThreads) s_dmesh[k] = F.mesh[k];
   __syncthreads();
   const double *m = s_dmesh;
   const double2 *G = F.G;
   const double cut = F.cut;
   const double w = m[i];
-  double sum = 0.0;
-  for (int j = tid; j < F.R; j += 256) {
-    const double2 a = value_none(G, m, nw, L, F.range_fwd[j], F.range_inv[j], w + cut, 0.0, w - cut, F.geo, F.ga, F.gb);
-    const double2 b = value_none(G, m, nw, L, F.range_fwd[j], F.range_inv[j], w - cut, 0.0, w + cut, F.geo, F.ga, F.gb);
-    sum += a.y - b.y;
+  if (tid < 256) {
+    double sum = 0.0;
+    for (int j = tid; j < F.R; j += 256) {
+      const double2 a = value_none(G, m, nw, L, F.range_fwd[j], F.range_inv[j], w + cut, 0.0, w - cut, F.geo, F.ga, F.gb);
+      const double2 b = value_none(G, m, nw, L, F.range_fwd[j], F.range_inv[j], w - cut, 0.0, w + cut, F.geo, F.ga, F.gb);
+      sum += a.y - b.y;
+    }
+    sum = wave_sum(sum);
+    if (lane == 0) part[tid >> 6] = sum;
+  } else if (lane < 2) {
+    const double c = lane ? -cut : cut;
+    const double2 p = value_none(G, m, nw, L, 0, 0, w + c, w - c, 0.0, F.geo, F.ga, F.gb);
+    part[4 + 2 * lane] = p.x;
+    part[5 + 2 * lane] = p.y;
   }
-  sum = wave_sum(sum);
-  if (lane == 0) part[tid >> 6] = sum;
   __syncthreads();
   if (tid == 0) {
-    sum = (part[0] + part[1]) + (part[2] + part[3]);
+    const double sum = (part[0] + part[1]) + (part[2] + part[3]);
     double v = 0.0;
     v -= 4.0 * F.spin * sum;
-    const double2 p = value_none(G, m, nw, L, 0, 0, w + cut, w - cut, 0.0, F.geo, F.ga, F.gb);
-    const double2 q = value_none(G, m, nw, L, 0, 0, w - cut, w + cut, 0.0, F.geo, F.ga, F.gb);
-    v += 0.75 * (p.x - q.x);
-    v += (p.y - q.y);
+    v += 0.75 * (part[4] - part[6]);
+    v += (part[5] - part[7]);
     v /= (kTwoPi * (cut + sigma_at(m, nw, F.v2, cut)));
     F.dv2[i] = v;
     if (isnan(v)) atomicOr(&F.flags[0], 1);
@@ -874,11 +880,15 @@ __device__ __forceinline__ void atomic_max_wave(int *dst, int v) {
 // stopped: later steps enqueued behind it (sp_run_flow) leave it untouched
 // too.  A flow in the mixed form also rewrites the FP32 shadow with the
 // planned scale and records the largest exponent of the new G.
+// FlowDev::euler: none, the update unless the derivative holds a NaN, the same as
+// part of a queued run, the update in any case
+enum { kEulerNone = 0, kEulerChecked = 1, kEulerQueued = 2, kEulerForced = 3 };
 __global__ void k_euler(const FlowDev *__restrict__ fl) {
   const FlowDev &F = fl[blockIdx.y];
   if (!F.euler) return;
-  if (F.flags[0] != 0 || F.flags[2] != 0) {
-    if (F.flags[0] != 0 && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&F.flags[2], 1);
+  const bool nan = F.euler == kEulerQueued ? F.flags[3] != 0 : F.flags[0] != 0 && F.euler != kEulerForced;
+  if (nan || F.flags[2] != 0) {
+    if (nan && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&F.flags[2], 1);
     return;
   }
   const double step = F.step;
@@ -947,28 +957,49 @@ __global__ void k_shadow(const FlowDev *__restrict__ fl) {
 // ---------------------------------------------------------------------------
 // static susceptibility (src/SU2/SU2MeasurementCorrelation.cpp:77-177), nu = 0
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void k_corr_partial(const FlowDev *__restrict__ fl) {
-  __shared__ double red[kThreads * 2];
-  extern __shared__ double s_cmesh[];  // the mesh (dynamic, nw doubles)
+__global__ __launch_bounds__(kCorrThreads) void k_corr_partial(const FlowDev *__restrict__ fl) {
+  __shared__ double red[kCorrPoints * 2], sums[2 * 256], eggs[2 * kCorrEggs / 64];
+  extern __shared__ double s_cmesh[];  // the mesh and Sigma (dynamic, 2 nw doubles)
   const FlowDev &F = fl[blockIdx.y];
   const int o = blockIdx.x;
   const int n = *F.Cn;
   if (o >= n) return;
   const int nw = F.nw, L = F.L;
-  for (int k = threadIdx.x; k < nw; k += kThreads) s_cmesh[k] = F.mesh[k];
+  for (int k = threadIdx.x; k < nw; k += kCorrThreads) {
+    s_cmesh[k] = F.mesh[k];
+    s_cmesh[nw + k] = F.v2[k];
+  }
   __syncthreads();
-  const double *m = s_cmesh, *v2 = F.v2;
+  const double *m = s_cmesh, *v2 = s_cmesh + nw;
   const double2 *G = F.G;
   const double spin = F.spin;
-  const int slots = kThreads / L;
-  const int tid = threadIdx.x;
+  const int slots = kCorrPoints / L;
+  const int tid = (int)threadIdx.x - kCorrEggs;  // negative: site-local part
   const int slot = tid / L, rid = tid - (tid / L) * L;
-  const bool active = slot < slots;
+  const bool active = tid >= 0 && slot < slots;
   const double nu = 0.0;
   const double w = F.Cwp[o];
   const double gw = (w + sigma_at(m, nw, v2, w)) * (w + nu + sigma_at(m, nw, v2, w + nu));
+  auto weight = [&](int e, double wp) {
+    return F.Cw[e] / (gw * (wp + sigma_at(m, nw, v2, wp)) * (wp + nu + sigma_at(m, nw, v2, wp + nu)) * (4.0 * kPi * kPi));
+  };
   double acc_s = 0.0, acc_d = 0.0;
-  if (active) {
+  if (tid < 0) {
+    // site-local vertices (they enter site 0), beside the sites' bundles
+    for (int e = threadIdx.x; e < n; e += kCorrEggs) {
+      const double wp = F.Cwp[e];
+      const double2 vv = value_none(G, m, nw, L, 0, 0, w + wp + nu, w - wp, nu, F.geo, F.ga, F.gb);
+      const double cf = weight(e, wp);
+      acc_s = fma(cf, spin * (-vv.x / 4.0 + vv.y), acc_s);
+      acc_d = fma(cf, spin * (3.0 * vv.x + 4.0 * vv.y), acc_d);
+    }
+    acc_s = wave_sum(acc_s);
+    acc_d = wave_sum(acc_d);
+    if ((threadIdx.x & 63) == 0) {
+      eggs[threadIdx.x >> 5] = acc_s;
+      eggs[(threadIdx.x >> 5) + 1] = acc_d;
+    }
+  } else if (active) {
     for (int e = slot; e < n; e += slots) {
       const double wp = F.Cwp[e];
       // generateAccessBuffer(w + wp + nu, nu, w - wp): trilinear, 8 supports (:500-557)
@@ -1003,49 +1034,33 @@ __global__ __launch_bounds__(kThreads) void k_corr_partial(const FlowDev *__rest
       }
       double rs = -(spin * spin) * sbs;
       double rd = -(16.0 * spin * spin) * sbd;
-      if (rid == 0) {
-        const double2 vv = value_none(G, m, nw, L, 0, 0, w + wp + nu, w - wp, nu, F.geo, F.ga, F.gb);
-        rs += spin * (-vv.x / 4.0 + vv.y);
-        rd += spin * (3.0 * vv.x + 4.0 * vv.y);
-      }
-      const double norm = 1.0 / (gw * (wp + sigma_at(m, nw, v2, wp)) * (wp + nu + sigma_at(m, nw, v2, wp + nu)) *
-                                 (4.0 * kPi * kPi));
-      const double cf = F.Cw[e] * norm;
+      const double cf = weight(e, wp);
       acc_s = fma(cf, rs, acc_s);
       acc_d = fma(cf, rd, acc_d);
     }
   }
-  red[2 * tid] = active ? acc_s : 0.0;
-  red[2 * tid + 1] = active ? acc_d : 0.0;
+  if (active) {
+    red[2 * tid] = acc_s;
+    red[2 * tid + 1] = acc_d;
+  }
   __syncthreads();
-  if (tid < L) {
-    double ts = 0.0, td = 0.0;
-    for (int k = 0; k < slots; ++k) { ts += red[2 * (k * L + tid)]; td += red[2 * (k * L + tid) + 1]; }
-    if (tid == 0) {
+  sum_partials(red, slots, 2 * L, sums);
+  for (int q = threadIdx.x; q < 2 * L; q += kCorrThreads) {
+    double v = sums[q];
+    if (q < 2) {
       const double term1 = 1.0 / gw;
-      ts += spin * term1 / kTwoPi;
-      td += 2.0 * spin * term1 / kPi;
+      for (int k = 0; k < kCorrEggs / 64; ++k) v += eggs[2 * k + q];
+      v += q ? 2.0 * spin * term1 / kPi : spin * term1 / kTwoPi;
     }
-    F.corr_partial[((size_t)o * L + tid) * 2] = F.Cw[o] * ts;
-    F.corr_partial[((size_t)o * L + tid) * 2 + 1] = F.Cw[o] * td;
+    F.corr_partial[(size_t)o * 2 * L + q] = F.Cw[o] * v;
   }
 }
 
-__global__ void k_corr_final(const FlowDev *__restrict__ fl) {
+__global__ __launch_bounds__(1024) void k_corr_final(const FlowDev *__restrict__ fl) {
   __shared__ double susc[2 * 256];
   const FlowDev &F = fl[blockIdx.y];
   const int n = *F.Cn;
-  const int L = F.L;
-  for (int r = threadIdx.x; r < L; r += blockDim.x) {
-    double s = 0.0, d = 0.0;
-    for (int o = 0; o < n; ++o) {
-      s += F.corr_partial[((size_t)o * L + r) * 2];
-      d += F.corr_partial[((size_t)o * L + r) * 2 + 1];
-    }
-    susc[2 * r] = s;
-    susc[2 * r + 1] = d;
-  }
-  __syncthreads();
+  sum_partials(F.corr_partial, n, 2 * F.L, susc);
   const int nout = F.B * F.Rb;
   for (int k = threadIdx.x; k < nout; k += blockDim.x) {
     F.corr_out[k] = susc[2 * F.corr_rid[k]];
@@ -1057,6 +1072,11 @@ __global__ void k_corr_final(const FlowDev *__restrict__ fl) {
     double packed;
     __builtin_memcpy(&packed, &fl, 8);
     F.corr_out[2 * nout] = packed;
+    if (F.euler == kEulerQueued) {
+      // the update reads the step's flag here, the next step starts without it
+      F.flags[3] = fl.x;
+      F.flags[0] = F.flags[1] = 0;
+    }
   }
 }
 
@@ -1073,6 +1093,8 @@ struct sp_ctx {
   hipStream_t stream = nullptr;
   FlowDev fd{};             // host copy of the flow descriptor
   FlowDev *d_fd = nullptr;  // device copy used by single-flow launches
+  FlowDev fd_sent{};        // what it holds
+  bool fd_valid = false;
   // descriptor uploads go through pinned slots, so that they are truly
   // asynchronous; a slot is refilled only after the copy that read it ran
   FlowDev *h_ring = nullptr;
@@ -1343,7 +1365,7 @@ hipError_t launch_compute(hipStream_t st, const FlowDev *d, const FlowDev *h, in
   const Geometry geo = geometry(h, n);
   {
     ProfScope ps(prof, 1);
-    hipLaunchKernelGGL(k_dsigma, dim3(geo.maxnw, n), dim3(256), geo.maxnw * sizeof(double), st, d);
+    hipLaunchKernelGGL(k_dsigma, dim3(geo.maxnw, n), dim3(kSigmaThreads), geo.maxnw * sizeof(double), st, d);
   }
   {
     ProfScope ps(prof, 2);
@@ -1409,8 +1431,8 @@ hipError_t launch_compute(hipStream_t st, const FlowDev *d, const FlowDev *h, in
 hipError_t launch_measure(hipStream_t st, const FlowDev *d, const FlowDev *h, int n, bool build_list) {
   const Geometry geo = geometry(h, n);
   if (build_list) hipLaunchKernelGGL(k_weights, dim3(1, n), dim3(64), geo.maxnw * sizeof(double), st, d, 1);
-  hipLaunchKernelGGL(k_corr_partial, dim3(geo.maxemax, n), dim3(kThreads), geo.maxnw * sizeof(double), st, d);
-  hipLaunchKernelGGL(k_corr_final, dim3(1, n), dim3(256), 0, st, d);
+  hipLaunchKernelGGL(k_corr_partial, dim3(geo.maxemax, n), dim3(kCorrThreads), 2 * geo.maxnw * sizeof(double), st, d);
+  hipLaunchKernelGGL(k_corr_final, dim3(1, n), dim3(1024), 0, st, d);
   return hipGetLastError();
 }
 
@@ -1421,17 +1443,23 @@ hipError_t launch_euler(hipStream_t st, const FlowDev *d, const FlowDev *h, int 
   if (blocks < 1) blocks = 1;
   ProfScope ps(prof, 3);
   hipLaunchKernelGGL(k_euler, dim3((unsigned)blocks, n), dim3(256), 0, st, d);
-  hipLaunchKernelGGL(k_plan, dim3(1, n), dim3(64), 0, st, d);
+  bool plan = false;
+  for (int i = 0; i < n; ++i) plan = plan || h[i].G32;
+  if (plan) hipLaunchKernelGGL(k_plan, dim3(1, n), dim3(64), 0, st, d);
   return hipGetLastError();
 }
 
+// the descriptor on the device, if it differs from what is there
 int upload_fd(sp_ctx *ctx) {
+  if (ctx->fd_valid && std::memcmp(&ctx->fd_sent, &ctx->fd, sizeof(FlowDev)) == 0) return SP_OK;
   const int s = ctx->ring_pos;
   ctx->ring_pos = (s + 1) % kRing;
   SP_HIP(hipEventSynchronize(ctx->ring_ev[s]));
   ctx->h_ring[s] = ctx->fd;
   SP_HIP(hipMemcpyAsync(ctx->d_fd, ctx->h_ring + s, sizeof(FlowDev), hipMemcpyHostToDevice, ctx->stream));
   SP_HIP(hipEventRecord(ctx->ring_ev[s], ctx->stream));
+  std::memcpy(&ctx->fd_sent, &ctx->fd, sizeof(FlowDev));
+  ctx->fd_valid = true;
   return SP_OK;
 }
 
@@ -1702,6 +1730,7 @@ int sp_compute_step(sp_ctx *ctx) {
   if (!ctx) return SP_EARG;
   FlowDev &f = ctx->fd;
   f.cut = ctx->cutoff;
+  f.corr_out = ctx->h_meas;
   int rc = upload_fd(ctx);
   if (rc) return rc;
   SP_HIP(hipMemsetAsync(f.flags, 0, 16, ctx->stream));
@@ -1718,15 +1747,17 @@ int sp_finalize_step(sp_ctx *ctx, double new_cutoff) {
   if (!std::isfinite(new_cutoff) || new_cutoff <= 0.0) return fail(ctx, SP_EARG, "cutoff must be finite and positive");
   FlowDev &f = ctx->fd;
   f.step = new_cutoff - ctx->cutoff;
-  f.euler = 1;
+  // the reference updates even a flow the caller did not check for NaN
+  f.euler = kEulerForced;
   f.cut = new_cutoff;
   int rc = upload_fd(ctx);
-  if (rc) return rc;
-  // the reference updates even a flow the caller did not check for NaN; the
-  // kernel only skips on the flag, so clear it for this explicit call
-  SP_HIP(hipMemsetAsync(f.flags, 0, 4, ctx->stream));
-  SP_HIP(launch_euler(ctx->stream, ctx->d_fd, &f, 1, ctx));
-  f.euler = 0;
+  if (rc) {
+    f.euler = kEulerNone;
+    return rc;
+  }
+  const hipError_t e = launch_euler(ctx->stream, ctx->d_fd, &f, 1, ctx);
+  f.euler = kEulerNone;
+  SP_HIP(e);
   ctx->cutoff = new_cutoff;
   ctx->have_flow = false;
   ctx->flags_cached = false;
@@ -1750,12 +1781,12 @@ int sp_measure_correlation(sp_ctx *ctx, double *zz, double *dd) {
   if (!ctx || !zz || !dd) return SP_EARG;
   FlowDev &f = ctx->fd;
   f.cut = ctx->cutoff;
+  f.corr_out = ctx->h_meas;  // (pinned: the record needs no copy of its own)
   int rc = upload_fd(ctx);
   if (rc) return rc;
   SP_HIP(launch_measure(ctx->stream, ctx->d_fd, &f, 1, !(ctx->list_cut == f.cut)));
   ctx->list_cut = f.cut;
   const int nout = f.B * f.Rb;
-  SP_HIP(hipMemcpyAsync(ctx->h_meas, f.corr_out, (2 * (size_t)nout + 1) * 8, hipMemcpyDeviceToHost, ctx->stream));
   SP_HIP(hipStreamSynchronize(ctx->stream));
   // the flags that k_corr_final stored after the record
   std::memcpy(ctx->h_flags, ctx->h_meas + 2 * nout, 8);
@@ -1782,22 +1813,20 @@ int sp_run_flow(sp_ctx *ctx, const double *cutoffs, int ncut, double *zz, double
     for (int j = kb; j < ke; ++j) {
       // computeStep and takeMeasurements at cutoffs[j]
       f.cut = cutoffs[j];
-      f.euler = 0;
-      int rc = upload_fd(ctx);
-      if (rc) return rc;
-      SP_HIP(hipMemsetAsync(f.flags, 0, 8, ctx->stream));
-      SP_HIP(launch_compute(ctx->stream, ctx->d_fd, &f, 1, ctx));
-      SP_HIP(launch_measure(ctx->stream, ctx->d_fd, &f, 1, false));
-      double *rec = ctx->h_run + (size_t)(j - kb) * slot;  // record, then the step's flags
-      SP_HIP(hipMemcpyAsync(rec, f.corr_out, (2 * nout + 1) * 8, hipMemcpyDeviceToHost, ctx->stream));
+      f.corr_out = ctx->h_run + (size_t)(j - kb) * slot;  // record, then the step's flags
       // finalizeStep(cutoffs[j + 1]): skipped, and the flow stopped, on a NaN
       f.step = cutoffs[j + 1] - cutoffs[j];
-      f.euler = 1;
-      f.cut = cutoffs[j + 1];
-      rc = upload_fd(ctx);
+      f.euler = kEulerQueued;
+      const int rc = upload_fd(ctx);
+      hipError_t e = hipSuccess;
+      if (rc == SP_OK) {
+        e = launch_compute(ctx->stream, ctx->d_fd, &f, 1, ctx);
+        if (e == hipSuccess) e = launch_measure(ctx->stream, ctx->d_fd, &f, 1, false);
+        if (e == hipSuccess) e = launch_euler(ctx->stream, ctx->d_fd, &f, 1, ctx);
+      }
+      f.euler = kEulerNone;
       if (rc) return rc;
-      SP_HIP(launch_euler(ctx->stream, ctx->d_fd, &f, 1, ctx));
-      f.euler = 0;
+      SP_HIP(e);
     }
     SP_HIP(hipStreamSynchronize(ctx->stream));
     for (int j = kb; j < ke; ++j) {
@@ -1964,7 +1993,7 @@ int sp_group_step(sp_group *grp, sp_ctx *const *ctxs, int n, const double *new_c
       const double nc = new_cutoffs[i];
       FlowDev &f = grp->h_fd[j];
       if (std::isfinite(nc) && nc > 0.0) {
-        f.euler = 1;
+        f.euler = kEulerChecked;
         f.step = nc - ctxs[i]->cutoff;
       }
     }

@@ -334,9 +334,9 @@ __global__ __launch_bounds__(64) void k_tri_weights(TriDev F, int corr_only) {
 // getValue(i1, i2, s, t, u, s1, s2, FrequencyChannel::None) for pairs that keep
 // the requested components (density-density, or the pair (0, 0)); rid_fwd /
 // rid_inv = symmetryTransform(i1, i2) / (i2, i1)
-__device__ double tri_value_none(const TriDev &F, int rid_fwd, int rid_inv, double s, double t, double u, int s1,
+__device__ double tri_value_none(const TriDev &F, const double *m, int rid_fwd, int rid_inv, double s, double t, double u, int s1,
                                  int s2) {
-  const double *G = F.G, *m = F.mesh;
+  const double *G = F.G;
   const int nw = F.nw;
   double sign = 1.0;
   bool swap = false;
@@ -361,26 +361,37 @@ __device__ double tri_value_none(const TriDev &F, int rid_fwd, int rid_inv, doub
                        bT * ((1 - bS) * A(lS, uT, uU) + bS * A(uS, uT, uU))));
 }
 
-// dSigma/dLambda (src/TRI/TRIFrgCore.cpp:122-151): one wavefront per mesh point
-__global__ __launch_bounds__(64) void k_tri_dsigma(TriDev F) {
+// dSigma/dLambda (src/TRI/TRIFrgCore.cpp:122-151): one workgroup per mesh point,
+// the site-local values beside the range sum
+__global__ __launch_bounds__(kSigmaThreads) void k_tri_dsigma(TriDev F) {
+  extern __shared__ double s_dmesh[];  // the mesh (dynamic, nw doubles)
+  __shared__ double part[12];
   const int i = blockIdx.x;
   if (i >= F.nw) return;
-  const int lane = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
   const int nw = F.nw;
-  const double *m = F.mesh;
+  for (int k = tid; k < nw; k += kSigmaThreads) s_dmesh[k] = F.mesh[k];
+  __syncthreads();
+  const double *m = s_dmesh;
   const double cut = F.cut;
   const double w = m[i];
-  double sum = 0.0;
-  for (int j = lane; j < F.R; j += 64) {
-    sum += tri_value_none(F, F.range_fwd[j], F.range_inv[j], w + cut, 0.0, w - cut, 3, 3) -
-           tri_value_none(F, F.range_fwd[j], F.range_inv[j], w - cut, 0.0, w + cut, 3, 3);
+  if (tid < 256) {
+    double sum = 0.0;
+    for (int j = tid; j < F.R; j += 256)
+      sum += tri_value_none(F, m, F.range_fwd[j], F.range_inv[j], w + cut, 0.0, w - cut, 3, 3) -
+             tri_value_none(F, m, F.range_fwd[j], F.range_inv[j], w - cut, 0.0, w + cut, 3, 3);
+    sum = wave_sum(sum);
+    if (lane == 0) part[tid >> 6] = sum;
+  } else if (lane < 8) {
+    // site-local values, component k at w + cut and w - cut
+    const int k = lane >> 1;
+    const double c = (lane & 1) ? -cut : cut;
+    part[4 + lane] = tri_value_none(F, m, 0, 0, w + c, w - c, 0.0, k, k);
   }
-  sum = wave_sum(sum);
-  if (lane == 0) {
-    double v = -2.0 * sum;
-    for (int k = 0; k < 4; ++k)
-      v += tri_value_none(F, 0, 0, w + cut, w - cut, 0.0, k, k) -
-           tri_value_none(F, 0, 0, w - cut, w + cut, 0.0, k, k);
+  __syncthreads();
+  if (tid == 0) {
+    double v = -2.0 * ((part[0] + part[1]) + (part[2] + part[3]));
+    for (int k = 0; k < 4; ++k) v += part[4 + 2 * k] - part[5 + 2 * k];
     v /= (kTwoPi * (cut + sigma_at(m, nw, F.v2, cut)));
     F.dv2[i] = v;
     if (isnan(v)) atomicOr(&F.flags[0], 1);
@@ -819,25 +830,69 @@ __device__ __forceinline__ Ab8 ab8(const double *m, int nw, int FS, double a, do
   return r;
 }
 
-__global__ __launch_bounds__(kTriThreads) void k_tri_corr_partial(TriDev F) {
-  __shared__ double red[kTriThreads * 10];
+// (fewer threads than the other cores: ten outputs each)
+constexpr int kTriCorrThreads = 512, kTriCorrEggs = 64;
+__global__ __launch_bounds__(kTriCorrThreads) void k_tri_corr_partial(TriDev F) {
+  __shared__ double red[(kTriCorrThreads - kTriCorrEggs) * 10], sums[10 * 64], eggs[10 * kTriCorrEggs / 64];
   const int o = blockIdx.x;
   const int n = *F.Cn;
   if (o >= n) return;
   const int nw = F.nw, L = F.L, FS = 16 * L;
-  const double *m = F.mesh, *v2 = F.v2;
+  extern __shared__ double s_cmesh[];  // the mesh and Sigma (dynamic, 2 nw doubles)
+  for (int k = threadIdx.x; k < nw; k += kTriCorrThreads) {
+    s_cmesh[k] = F.mesh[k];
+    s_cmesh[nw + k] = F.v2[k];
+  }
+  __syncthreads();
+  const double *m = s_cmesh, *v2 = s_cmesh + nw;
   const double *G = F.G;
-  const int slots = kTriThreads / L;
-  const int tid = threadIdx.x;
+  const int slots = (kTriCorrThreads - kTriCorrEggs) / L;
+  const int tid = (int)threadIdx.x - kTriCorrEggs;  // negative: site-local part
   const int slot = tid / L, rid = tid - (tid / L) * L;
-  const bool active = slot < slots;
+  const bool active = tid >= 0 && slot < slots;
   const double nu = 0.0;
   const double w = F.Cwp[o];
   const double gw = (w + sigma_at(m, nw, v2, w)) * (w + nu + sigma_at(m, nw, v2, w + nu));
   double acc[10];
 #pragma unroll
   for (int g = 0; g < 10; ++g) acc[g] = 0.0;
-  if (active) {
+  auto weight = [&](int e, double wp) {
+    return F.Cw[e] / (gw * (wp + sigma_at(m, nw, v2, wp)) * (wp + nu + sigma_at(m, nw, v2, wp + nu)) * (4.0 * kPi * kPi));
+  };
+  if (tid < 0) {
+    // site-local vertices (they enter site 0), beside the sites' bundles
+    for (int e = threadIdx.x; e < n; e += kTriCorrEggs) {
+      const double wp = F.Cwp[e];
+      double r[10] = {};
+      // egg: site-local vertex of generateAccessBuffer(w + wp + nu, w - wp, nu)
+      const Ab8 q = ab8(m, nw, FS, w + wp + nu, w - wp, nu);
+      const bool qx = q.fl & 1, qt = (q.fl >> 1) & 1;
+      double v[16];
+#pragma unroll
+      for (int cc = 0; cc < 16; ++cc) {
+        int s1 = cc / 4, s2 = cc % 4;
+        if (qx) { const int z = s1; s1 = s2; s2 = z; }
+        const double tsign = qt ? double(zeta(s1) * zeta(s2)) : 1.0;
+        const double fsign = -double(zeta(qx ? s1 : s2));
+        double x = 0.0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const double sg = ((q.fl >> (2 + i)) & 1) ? tsign * fsign : tsign;
+          x = fma(sg * q.w[i], G[(size_t)q.off[i] + (4 * s1 + s2) * F.cst], x);
+        }
+        v[cc] = x;
+      }
+      egg_rows(r, v, std::make_integer_sequence<int, 10>{});
+      const double cf = weight(e, wp);
+#pragma unroll
+      for (int g = 0; g < 10; ++g) acc[g] = fma(cf, r[g], acc[g]);
+    }
+#pragma unroll
+    for (int g = 0; g < 10; ++g) {
+      acc[g] = wave_sum(acc[g]);
+      if ((threadIdx.x & 63) == 0) eggs[(threadIdx.x >> 6) * 10 + g] = acc[g];
+    }
+  } else if (active) {
     for (int e = slot; e < n; e += slots) {
       const double wp = F.Cwp[e];
       double r[10];
@@ -862,63 +917,35 @@ __global__ __launch_bounds__(kTriThreads) void k_tri_corr_partial(TriDev F) {
         }
         r[g] = (c == 15 ? -4.0 : -1.0) * v;
       }
-      if (rid == 0) {
-        // egg: site-local vertex of generateAccessBuffer(w + wp + nu, w - wp, nu)
-        const Ab8 q = ab8(m, nw, FS, w + wp + nu, w - wp, nu);
-        const bool qx = q.fl & 1, qt = (q.fl >> 1) & 1;
-        double v[16];
-#pragma unroll
-        for (int cc = 0; cc < 16; ++cc) {
-          int s1 = cc / 4, s2 = cc % 4;
-          if (qx) { const int z = s1; s1 = s2; s2 = z; }
-          const double tsign = qt ? double(zeta(s1) * zeta(s2)) : 1.0;
-          const double fsign = -double(zeta(qx ? s1 : s2));
-          double x = 0.0;
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const double sg = ((q.fl >> (2 + i)) & 1) ? tsign * fsign : tsign;
-            x = fma(sg * q.w[i], G[(size_t)q.off[i] + (4 * s1 + s2) * F.cst], x);
-          }
-          v[cc] = x;
-        }
-        egg_rows(r, v, std::make_integer_sequence<int, 10>{});
-      }
-      const double norm = 1.0 / (gw * (wp + sigma_at(m, nw, v2, wp)) * (wp + nu + sigma_at(m, nw, v2, wp + nu)) *
-                                 (4.0 * kPi * kPi));
-      const double cf = F.Cw[e] * norm;
+      const double cf = weight(e, wp);
 #pragma unroll
       for (int g = 0; g < 10; ++g) acc[g] = fma(cf, r[g], acc[g]);
     }
   }
+  if (active)
 #pragma unroll
-  for (int g = 0; g < 10; ++g) red[g * kTriThreads + tid] = active ? acc[g] : 0.0;
+    for (int g = 0; g < 10; ++g) red[10 * tid + g] = acc[g];
   __syncthreads();
-  for (int q = tid; q < 10 * L; q += kTriThreads) {
-    const int g = q / L, r = q - (q / L) * L;
-    double tsum = 0.0;
-    for (int k = 0; k < slots; ++k) tsum += red[g * kTriThreads + k * L + r];
+  sum_partials(red, slots, 10 * L, sums);
+  for (int q = threadIdx.x; q < 10 * L; q += kTriCorrThreads) {
+    const int r = q / 10, g = q - (q / 10) * 10;
+    double v = sums[q];
     if (r == 0) {
+      for (int k = 0; k < kTriCorrEggs / 64; ++k) v += eggs[k * 10 + g];
       // bubble term (site 0): density 2, spin diagonal 1/2
       const double term1 = 1.0 / gw;
-      if (g == 0) tsum += 2.0 * term1 / kTwoPi;
-      else if (g == 1 || g == 5 || g == 9) tsum += 0.5 * term1 / kTwoPi;
+      if (g == 0) v += 2.0 * term1 / kTwoPi;
+      else if (g == 1 || g == 5 || g == 9) v += 0.5 * term1 / kTwoPi;
     }
-    F.corr_partial[((size_t)o * 10 + g) * L + r] = F.Cw[o] * tsum;
+    F.corr_partial[((size_t)o * 10 + g) * L + r] = F.Cw[o] * v;
   }
 }
 
-// sum over outer points; output groups DD, XX, XY, XZ, YX, YY, YZ, ZX, ZY, ZZ
-// with the components of each (basis, site) pair through its spin permutation
-__global__ void k_tri_corr_final(TriDev F) {
+__global__ __launch_bounds__(1024) void k_tri_corr_final(TriDev F) {
   __shared__ double susc[10 * 64];
   const int n = *F.Cn;
   const int L = F.L;
-  for (int q = threadIdx.x; q < 10 * L; q += blockDim.x) {
-    double v = 0.0;
-    for (int o = 0; o < n; ++o) v += F.corr_partial[(size_t)o * 10 * L + q];
-    susc[q] = v;
-  }
-  __syncthreads();
+  sum_partials(F.corr_partial, n, 10 * L, susc);
   // position of component c among the 10 stored outputs
   auto slot_of = [](int c) {
     for (int g = 0; g < 10; ++g)
@@ -934,6 +961,13 @@ __global__ void k_tri_corr_final(TriDev F) {
 #pragma unroll
     for (int g = 0; g < 10; ++g) F.corr_out[(size_t)g * nout + k] = susc[slot_of(comp[g]) * L + rid];
   }
+  if (threadIdx.x == 0) {
+    // the flags of the step before the record, so that a run reads both at once
+    const int2 fl = make_int2(F.flags[0], F.flags[1]);
+    double packed;
+    __builtin_memcpy(&packed, &fl, 8);
+    F.corr_out[(size_t)10 * nout] = packed;
+  }
 }
 
 }  // namespace
@@ -947,6 +981,10 @@ struct sp_tri_ctx {
   TriDev fd{};
   double cutoff = 0.0;
   bool have_flow = false;
+  bool flags_known = false;  // step_flags: flags of the step computed last
+  int step_flags[2] = {0, 0};
+  double list_cut = 0.0;     // cutoff of the correlation point list (0: none)
+  double *h_meas = nullptr;  // pinned: the record of a measurement
   size_t lds = 0;
   double *stage = nullptr;  // rows in the reference's order on their way to and from the host
   std::vector<void *> allocs;
@@ -1122,7 +1160,7 @@ hipError_t tri_launch_compute(sp_tri_ctx *ctx) {
   F.cut = ctx->cutoff;
   {
     TriProf ps(ctx, 1);
-    hipLaunchKernelGGL(k_tri_dsigma, dim3(F.nw), dim3(64), 0, ctx->stream, F);
+    hipLaunchKernelGGL(k_tri_dsigma, dim3(F.nw), dim3(kSigmaThreads), F.nw * sizeof(double), ctx->stream, F);
   }
   {
     TriProf ps(ctx, 2);
@@ -1303,7 +1341,7 @@ int sp_tri_ctx_create(const sp_tri_problem *p, sp_tri_ctx **out) {
       (rc = talloc(ctx, &f.Wwp, (size_t)f.nw * emax)) || (rc = talloc(ctx, &f.Wc, (size_t)f.nw * emax)) ||
       (rc = talloc(ctx, &f.Wn, f.nw)) || (rc = talloc(ctx, &f.Cwp, emax)) || (rc = talloc(ctx, &f.Cw, emax)) ||
       (rc = talloc(ctx, &f.Cn, 1)) || (rc = talloc(ctx, &f.corr_partial, (size_t)emax * 10 * f.L)) ||
-      (rc = talloc(ctx, &f.corr_out, 10 * nc)) || (rc = talloc(ctx, &f.flags, 4)) ||
+      (rc = talloc(ctx, &f.corr_out, 10 * nc + 1)) || (rc = talloc(ctx, &f.flags, 4)) ||
       (f.t_waves && ((rc = talloc(ctx, &tdst, plan.dst.size())) || (rc = talloc(ctx, &tedge, plan.edge_ops.size())) || (rc = talloc(ctx, &tplan, plan.plan.size())) ||
                      (rc = talloc(ctx, &tops, plan.ops.size())) ||
                      (rc = talloc(ctx, &ctx->stage, (size_t)tri_stage_rows(f) * 16 * f.L)))))
@@ -1312,6 +1350,11 @@ int sp_tri_ctx_create(const sp_tri_problem *p, sp_tri_ctx **out) {
   f.t_edge_ops = tedge;
   f.t_plan = tplan;
   f.t_ops = tops;
+  {
+    void *q = nullptr;
+    SP_THIP(hipHostMalloc(&q, (10 * nc + 1) * 8, 0));
+    ctx->h_meas = static_cast<double *>(q);
+  }
   f.mesh = mesh;
   f.site_rid = site;
   f.site_perm = sitep;
@@ -1370,6 +1413,7 @@ int sp_tri_ctx_destroy(sp_tri_ctx *ctx) {
   for (int k = 0; k < 4; ++k)
     for (auto &pr : ctx->pending[k]) { (void)hipEventDestroy(pr.first); (void)hipEventDestroy(pr.second); }
   for (void *q : ctx->allocs) (void)hipFree(q);
+  if (ctx->h_meas) (void)hipHostFree(ctx->h_meas);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return SP_OK;
@@ -1412,6 +1456,8 @@ int sp_tri_compute_step(sp_tri_ctx *ctx) {
   SP_THIP(hipMemsetAsync(ctx->fd.flags, 0, 16, ctx->stream));
   SP_THIP(tri_launch_compute(ctx));
   ctx->have_flow = true;
+  ctx->flags_known = false;
+  ctx->list_cut = ctx->cutoff;
   return SP_OK;
 }
 
@@ -1437,9 +1483,12 @@ int sp_tri_finalize_step(sp_tri_ctx *ctx, double new_cutoff) {
 int sp_tri_is_diverged(sp_tri_ctx *ctx, int *diverged) {
   if (!ctx || !diverged) return SP_EARG;
   if (!ctx->have_flow) return tfail(ctx, SP_ESTATE, "no flow computed at the current cutoff");
-  int fl[2] = {0, 0};
-  SP_THIP(hipMemcpyAsync(fl, ctx->fd.flags, 8, hipMemcpyDeviceToHost, ctx->stream));
-  SP_THIP(hipStreamSynchronize(ctx->stream));
+  int *fl = ctx->step_flags;
+  if (!ctx->flags_known) {
+    SP_THIP(hipMemcpyAsync(fl, ctx->fd.flags, 8, hipMemcpyDeviceToHost, ctx->stream));
+    SP_THIP(hipStreamSynchronize(ctx->stream));
+    ctx->flags_known = true;
+  }
   if (fl[1]) return tfail(ctx, SP_EARG, "evaluation list overflow");
   *diverged = fl[0] ? 1 : 0;
   return SP_OK;
@@ -1449,13 +1498,18 @@ int sp_tri_measure_correlation(sp_tri_ctx *ctx, double *out) {
   if (!ctx || !out) return SP_EARG;
   TriDev F = ctx->fd;
   F.cut = ctx->cutoff;
-  hipLaunchKernelGGL(k_tri_weights, dim3(1), dim3(64), F.nw * sizeof(double), ctx->stream, F, 1);
-  hipLaunchKernelGGL(k_tri_corr_partial, dim3(F.emax), dim3(kTriThreads), 0, ctx->stream, F);
-  hipLaunchKernelGGL(k_tri_corr_final, dim3(1), dim3(256), 0, ctx->stream, F);
+  F.corr_out = ctx->h_meas;  // (pinned: the record needs no copy of its own)
+  // the point list is there already where a derivative was computed at this cutoff
+  if (!(ctx->list_cut == F.cut)) hipLaunchKernelGGL(k_tri_weights, dim3(1), dim3(64), F.nw * sizeof(double), ctx->stream, F, 1);
+  hipLaunchKernelGGL(k_tri_corr_partial, dim3(F.emax), dim3(kTriCorrThreads), 2 * F.nw * sizeof(double), ctx->stream, F);
+  hipLaunchKernelGGL(k_tri_corr_final, dim3(1), dim3(1024), 0, ctx->stream, F);
   SP_THIP(hipGetLastError());
   const size_t n = 10 * (size_t)F.B * F.Rb;
-  SP_THIP(hipMemcpyAsync(out, F.corr_out, n * 8, hipMemcpyDeviceToHost, ctx->stream));
   SP_THIP(hipStreamSynchronize(ctx->stream));
+  ctx->list_cut = F.cut;
+  std::memcpy(out, ctx->h_meas, n * 8);
+  std::memcpy(ctx->step_flags, ctx->h_meas + n, 8);
+  ctx->flags_known = ctx->have_flow;
   return SP_OK;
 }
 

@@ -169,26 +169,37 @@ __device__ double xyz_value_none(const double *G, const double *m, int nw, int L
                bT * ((1 - bS) * A(lS, uT, uU) + bS * A(uS, uT, uU)));
 }
 
-// dSigma/dLambda (src/XYZ/XYZFrgCore.cpp:164-193): one wavefront per mesh point
-__global__ __launch_bounds__(64) void k_xyz_dsigma(XyzDev F) {
+// dSigma/dLambda (src/XYZ/XYZFrgCore.cpp:164-193): one workgroup per mesh point,
+// the site-local values beside the range sum
+__global__ __launch_bounds__(kSigmaThreads) void k_xyz_dsigma(XyzDev F) {
+  extern __shared__ double s_dmesh[];  // the mesh (dynamic, nw doubles)
+  __shared__ double part[12];
   const int i = blockIdx.x;
   if (i >= F.nw) return;
-  const int lane = threadIdx.x;
-  const int nw = F.nw, L = F.L;
-  const double *m = F.mesh;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int nw = F.nw;
+  for (int k = tid; k < nw; k += kSigmaThreads) s_dmesh[k] = F.mesh[k];
+  __syncthreads();
+  const double *m = s_dmesh;
   const double cut = F.cut;
   const double w = m[i];
-  double sum = 0.0;
-  for (int j = lane; j < F.R; j += 64) {
-    sum += xyz_value_none(F.G, m, nw, L, F.range_fwd[j], F.range_inv[j], w + cut, 0.0, w - cut, kD) -
-           xyz_value_none(F.G, m, nw, L, F.range_fwd[j], F.range_inv[j], w - cut, 0.0, w + cut, kD);
+  if (tid < 256) {
+    double sum = 0.0;
+    for (int j = tid; j < F.R; j += 256)
+      sum += xyz_value_none(F.G, m, nw, F.L, F.range_fwd[j], F.range_inv[j], w + cut, 0.0, w - cut, kD) -
+             xyz_value_none(F.G, m, nw, F.L, F.range_fwd[j], F.range_inv[j], w - cut, 0.0, w + cut, kD);
+    sum = wave_sum(sum);
+    if (lane == 0) part[tid >> 6] = sum;
+  } else if (lane < 8) {
+    // site-local values, component k at w + cut and w - cut
+    const int k = lane >> 1;
+    const double c = (lane & 1) ? -cut : cut;
+    part[4 + lane] = xyz_value_none(F.G, m, nw, F.L, 0, 0, w + c, w - c, 0.0, k);
   }
-  sum = wave_sum(sum);
-  if (lane == 0) {
-    double v = -2.0 * sum;
-    for (int k = 0; k < 4; ++k)
-      v += xyz_value_none(F.G, m, nw, L, 0, 0, w + cut, w - cut, 0.0, k) -
-           xyz_value_none(F.G, m, nw, L, 0, 0, w - cut, w + cut, 0.0, k);
+  __syncthreads();
+  if (tid == 0) {
+    double v = -2.0 * ((part[0] + part[1]) + (part[2] + part[3]));
+    for (int k = 0; k < 4; ++k) v += part[4 + 2 * k] - part[5 + 2 * k];
     v /= (kTwoPi * (cut + sigma_at(m, nw, F.v2, cut)));
     F.dv2[i] = v;
     if (isnan(v)) atomicOr(&F.flags[0], 1);
@@ -836,23 +847,54 @@ __global__ void k_xyz_euler(XyzDev F) {
 // ---------------------------------------------------------------------------
 // static susceptibility (src/XYZ/XYZMeasurementCorrelation.cpp:98-212), nu = 0
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kXyzThreads) void k_xyz_corr_partial(XyzDev F) {
-  __shared__ double red[kXyzThreads * 4];
+__global__ __launch_bounds__(kCorrThreads) void k_xyz_corr_partial(XyzDev F) {
+  __shared__ double red[(kCorrThreads - kCorrEggs) * 4], sums[4 * 64], eggs[4 * kCorrEggs / 64];
   const int o = blockIdx.x;
   const int n = *F.Cn;
   if (o >= n) return;
   const int nw = F.nw, L = F.L;
-  const double *m = F.mesh, *v2 = F.v2;
+  extern __shared__ double s_cmesh[];  // the mesh and Sigma (dynamic, 2 nw doubles)
+  for (int k = threadIdx.x; k < nw; k += kCorrThreads) {
+    s_cmesh[k] = F.mesh[k];
+    s_cmesh[nw + k] = F.v2[k];
+  }
+  __syncthreads();
+  const double *m = s_cmesh, *v2 = s_cmesh + nw;
   const double *G = F.G;
-  const int slots = kXyzThreads / L;
-  const int tid = threadIdx.x;
+  const int slots = (kCorrThreads - kCorrEggs) / L;
+  const int tid = (int)threadIdx.x - kCorrEggs;  // negative: site-local part
   const int slot = tid / L, rid = tid - (tid / L) * L;
-  const bool active = slot < slots;
+  const bool active = tid >= 0 && slot < slots;
   const double nu = 0.0;
   const double w = F.Cwp[o];
   const double gw = (w + sigma_at(m, nw, v2, w)) * (w + nu + sigma_at(m, nw, v2, w + nu));
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  if (active) {
+  auto weight = [&](int e, double wp) {
+    return F.Cw[e] / (gw * (wp + sigma_at(m, nw, v2, wp)) * (wp + nu + sigma_at(m, nw, v2, wp + nu)) * (4.0 * kPi * kPi));
+  };
+  if (tid < 0) {
+    // site-local vertices (they enter site 0), beside the sites' bundles
+    for (int e = threadIdx.x; e < n; e += kCorrEggs) {
+      const double wp = F.Cwp[e];
+      double r[4];
+      // egg: getValue(0, 0, w + wp + nu, w - wp, nu, c, None)
+      double vv[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) vv[k] = xyz_value_none(G, m, nw, L, 0, 0, w + wp + nu, w - wp, nu, k);
+      r[kX] = 0.5 * (vv[kX] - vv[kY] - vv[kZ] + vv[kD]);
+      r[kY] = 0.5 * (-vv[kX] + vv[kY] - vv[kZ] + vv[kD]);
+      r[kZ] = 0.5 * (-vv[kX] - vv[kY] + vv[kZ] + vv[kD]);
+      r[kD] = 2.0 * (vv[kX] + vv[kY] + vv[kZ] + vv[kD]);
+      const double cf = weight(e, wp);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) acc[g] = fma(cf, r[g], acc[g]);
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      acc[g] = wave_sum(acc[g]);
+      if ((threadIdx.x & 63) == 0) eggs[(threadIdx.x >> 6) * 4 + g] = acc[g];
+    }
+  } else if (active) {
     for (int e = slot; e < n; e += slots) {
       const double wp = F.Cwp[e];
       double r[4];
@@ -888,57 +930,47 @@ __global__ __launch_bounds__(kXyzThreads) void k_xyz_corr_partial(XyzDev F) {
         r[kZ] = -v[kZ];
         r[kD] = -4.0 * v[kD];
       }
-      if (rid == 0) {
-        // egg: getValue(0, 0, w + wp + nu, w - wp, nu, c, None)
-        double vv[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) vv[k] = xyz_value_none(G, m, nw, L, 0, 0, w + wp + nu, w - wp, nu, k);
-        r[kX] += 0.5 * (vv[kX] - vv[kY] - vv[kZ] + vv[kD]);
-        r[kY] += 0.5 * (-vv[kX] + vv[kY] - vv[kZ] + vv[kD]);
-        r[kZ] += 0.5 * (-vv[kX] - vv[kY] + vv[kZ] + vv[kD]);
-        r[kD] += 2.0 * (vv[kX] + vv[kY] + vv[kZ] + vv[kD]);
-      }
-      const double norm = 1.0 / (gw * (wp + sigma_at(m, nw, v2, wp)) * (wp + nu + sigma_at(m, nw, v2, wp + nu)) *
-                                 (4.0 * kPi * kPi));
-      const double cf = F.Cw[e] * norm;
+      const double cf = weight(e, wp);
 #pragma unroll
       for (int g = 0; g < 4; ++g) acc[g] = fma(cf, r[g], acc[g]);
     }
   }
+  if (active)
 #pragma unroll
-  for (int g = 0; g < 4; ++g) red[g * kXyzThreads + tid] = active ? acc[g] : 0.0;
+    for (int g = 0; g < 4; ++g) red[4 * tid + g] = acc[g];
   __syncthreads();
-  for (int q = tid; q < 4 * L; q += kXyzThreads) {
-    const int g = q / L, r = q - (q / L) * L;
-    double tsum = 0.0;
-    for (int k = 0; k < slots; ++k) tsum += red[g * kXyzThreads + k * L + r];
+  sum_partials(red, slots, 4 * L, sums);
+  for (int q = threadIdx.x; q < 4 * L; q += kCorrThreads) {
+    const int r = q / 4, g = q - (q / 4) * 4;
+    double v = sums[q];
     if (r == 0) {
+      for (int k = 0; k < kCorrEggs / 64; ++k) v += eggs[k * 4 + g];
       // bubble term (site 0): spin components 1/(4 pi), density 1/pi
       const double term1 = 1.0 / gw;
-      tsum += g == kD ? term1 / kPi : term1 / (4.0 * kPi);
+      v += g == kD ? term1 / kPi : term1 / (4.0 * kPi);
     }
-    F.corr_partial[((size_t)o * 4 + g) * L + r] = F.Cw[o] * tsum;
+    F.corr_partial[((size_t)o * 4 + g) * L + r] = F.Cw[o] * v;
   }
 }
 
-// sum over outer points; output groups XX, YY, ZZ, DD, each spin component of
-// a (basis, site) pair through its spin permutation (XYZMeasurementCorrelation.cpp:186-211)
-__global__ void k_xyz_corr_final(XyzDev F) {
+__global__ __launch_bounds__(1024) void k_xyz_corr_final(XyzDev F) {
   __shared__ double susc[4 * 64];
   const int n = *F.Cn;
   const int L = F.L;
-  for (int q = threadIdx.x; q < 4 * L; q += blockDim.x) {
-    double v = 0.0;
-    for (int o = 0; o < n; ++o) v += F.corr_partial[(size_t)o * 4 * L + q];
-    susc[q] = v;
-  }
-  __syncthreads();
+  sum_partials(F.corr_partial, n, 4 * L, susc);
   const int nout = F.B * F.Rb;
   for (int k = threadIdx.x; k < nout; k += blockDim.x) {
     const int rid = F.corr_rid[k];
 #pragma unroll
     for (int g = 0; g < 3; ++g) F.corr_out[(size_t)g * nout + k] = susc[F.corr_perm[3 * k + g] * L + rid];
     F.corr_out[(size_t)3 * nout + k] = susc[kD * L + rid];
+  }
+  if (threadIdx.x == 0) {
+    // the flags of the step before the record, so that a run reads both at once
+    const int2 fl = make_int2(F.flags[0], F.flags[1]);
+    double packed;
+    __builtin_memcpy(&packed, &fl, 8);
+    F.corr_out[(size_t)4 * nout] = packed;
   }
 }
 
@@ -953,6 +985,10 @@ struct sp_xyz_ctx {
   XyzDev fd{};
   double cutoff = 0.0;
   bool have_flow = false;
+  bool flags_known = false;  // step_flags: flags of the step computed last
+  int step_flags[2] = {0, 0};
+  double list_cut = 0.0;     // cutoff of the correlation point list (0: none)
+  double *h_meas = nullptr;  // pinned: the record of a measurement
   bool waves = false;   // dGamma by the wave kernels (xyz_rhs.h)
   bool direct = false;  // bubble summed per point (k_xyz_dgamma_direct)
   size_t lds = 0;
@@ -1042,7 +1078,7 @@ hipError_t xyz_launch_compute(sp_xyz_ctx *ctx) {
   F.cut = ctx->cutoff;
   {
     XyzProf ps(ctx, 1);
-    hipLaunchKernelGGL(k_xyz_dsigma, dim3(F.nw), dim3(64), 0, ctx->stream, F);
+    hipLaunchKernelGGL(k_xyz_dsigma, dim3(F.nw), dim3(kSigmaThreads), F.nw * sizeof(double), ctx->stream, F);
   }
   {
     XyzProf ps(ctx, 2);
@@ -1365,12 +1401,17 @@ static int xyz_ctx_init(sp_xyz_ctx *ctx, const sp_xyz_problem *p, const XyzOrder
       (rc = xalloc(ctx, &f.Wwp, (size_t)f.nw * emax)) || (rc = xalloc(ctx, &f.Wc, (size_t)f.nw * emax)) ||
       (rc = xalloc(ctx, &f.Wn, f.nw)) || (rc = xalloc(ctx, &f.Cwp, emax)) || (rc = xalloc(ctx, &f.Cw, emax)) ||
       (rc = xalloc(ctx, &f.Cn, 1)) || (rc = xalloc(ctx, &f.corr_partial, (size_t)emax * 4 * f.L)) ||
-      (rc = xalloc(ctx, &f.corr_out, 4 * nc)) || (rc = xalloc(ctx, &f.flags, 4)))
+      (rc = xalloc(ctx, &f.corr_out, 4 * nc + 1)) || (rc = xalloc(ctx, &f.flags, 4)))
     return rc;
   int4 *midx_d = nullptr;
   if ((rc = xalloc(ctx, &midx_d, midx.size()))) return rc;
   SP_XHIP(hipMemcpy(midx_d, midx.data(), midx.size() * sizeof(int4), hipMemcpyHostToDevice));
   f.ovl_midx = midx_d;
+  {
+    void *q = nullptr;
+    SP_XHIP(hipHostMalloc(&q, (4 * nc + 1) * 8, 0));
+    ctx->h_meas = static_cast<double *>(q);
+  }
   f.mesh = mesh;
   f.site_rid = site;
   f.site_perm = sitep;
@@ -1424,6 +1465,7 @@ int sp_xyz_ctx_destroy(sp_xyz_ctx *ctx) {
   for (int k = 0; k < 4; ++k)
     for (auto &pr : ctx->pending[k]) { (void)hipEventDestroy(pr.first); (void)hipEventDestroy(pr.second); }
   for (void *q : ctx->allocs) (void)hipFree(q);
+  if (ctx->h_meas) (void)hipHostFree(ctx->h_meas);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return SP_OK;
@@ -1471,6 +1513,8 @@ int sp_xyz_compute_step(sp_xyz_ctx *ctx) {
   SP_XHIP(hipMemsetAsync(ctx->fd.flags, 0, 16, ctx->stream));
   SP_XHIP(xyz_launch_compute(ctx));
   ctx->have_flow = true;
+  ctx->flags_known = false;
+  ctx->list_cut = ctx->cutoff;
   return SP_OK;
 }
 
@@ -1496,9 +1540,12 @@ int sp_xyz_finalize_step(sp_xyz_ctx *ctx, double new_cutoff) {
 int sp_xyz_is_diverged(sp_xyz_ctx *ctx, int *diverged) {
   if (!ctx || !diverged) return SP_EARG;
   if (!ctx->have_flow) return xfail(ctx, SP_ESTATE, "no flow computed at the current cutoff");
-  int fl[2] = {0, 0};
-  SP_XHIP(hipMemcpyAsync(fl, ctx->fd.flags, 8, hipMemcpyDeviceToHost, ctx->stream));
-  SP_XHIP(hipStreamSynchronize(ctx->stream));
+  int *fl = ctx->step_flags;
+  if (!ctx->flags_known) {
+    SP_XHIP(hipMemcpyAsync(fl, ctx->fd.flags, 8, hipMemcpyDeviceToHost, ctx->stream));
+    SP_XHIP(hipStreamSynchronize(ctx->stream));
+    ctx->flags_known = true;
+  }
   if (fl[1]) return xfail(ctx, SP_EARG, "evaluation list overflow");
   *diverged = fl[0] ? 1 : 0;
   return SP_OK;
@@ -1508,13 +1555,18 @@ int sp_xyz_measure_correlation(sp_xyz_ctx *ctx, double *out) {
   if (!ctx || !out) return SP_EARG;
   XyzDev F = ctx->fd;
   F.cut = ctx->cutoff;
-  hipLaunchKernelGGL(k_xyz_weights, dim3(1), dim3(64), F.nw * sizeof(double), ctx->stream, F, 1);
-  hipLaunchKernelGGL(k_xyz_corr_partial, dim3(F.emax), dim3(kXyzThreads), 0, ctx->stream, F);
-  hipLaunchKernelGGL(k_xyz_corr_final, dim3(1), dim3(256), 0, ctx->stream, F);
+  F.corr_out = ctx->h_meas;  // (pinned: the record needs no copy of its own)
+  // the point list is there already where a derivative was computed at this cutoff
+  if (!(ctx->list_cut == F.cut)) hipLaunchKernelGGL(k_xyz_weights, dim3(1), dim3(64), F.nw * sizeof(double), ctx->stream, F, 1);
+  hipLaunchKernelGGL(k_xyz_corr_partial, dim3(F.emax), dim3(kCorrThreads), 2 * F.nw * sizeof(double), ctx->stream, F);
+  hipLaunchKernelGGL(k_xyz_corr_final, dim3(1), dim3(1024), 0, ctx->stream, F);
   SP_XHIP(hipGetLastError());
   const size_t n = 4 * (size_t)F.B * F.Rb;
-  SP_XHIP(hipMemcpyAsync(out, F.corr_out, n * 8, hipMemcpyDeviceToHost, ctx->stream));
   SP_XHIP(hipStreamSynchronize(ctx->stream));
+  ctx->list_cut = F.cut;
+  std::memcpy(out, ctx->h_meas, n * 8);
+  std::memcpy(ctx->step_flags, ctx->h_meas + n, 8);
+  ctx->flags_known = ctx->have_flow;
   return SP_OK;
 }
 
