@@ -91,14 +91,6 @@ namespace {
 #define SPFRG_MIN_BLOCKS_MIXED 5
 #endif
 constexpr int kThreads = SPFRG_THREADS;
-// small lattices: the producer's work per evaluation point does not shrink
-// with L while the workers' does, so flows with L <= kSmallL run the dGamma
-// kernel in workgroups of kSmallThreads (one worker wave per producer wave,
-// twice the workgroups per CU); measured 17-43 % faster for L = 7, 9, 11 and
-// 16, slower for L = 23 and 31
-constexpr int kSmallThreads = 128;
-constexpr int kSmallL = 16;
-inline int dgamma_threads(int L) { return L <= kSmallL ? kSmallThreads : kThreads; }
 constexpr int kMaxBatch = SPFRG_MAX_BATCH;
 constexpr int kMaxBatchMixed = SPFRG_MAX_BATCH_MIXED;
 #ifndef SPFRG_UNROLL_FP64
@@ -231,7 +223,7 @@ __global__ __launch_bounds__(64) void k_weights(const FlowDev *__restrict__ fl, 
   const FlowDev &F = fl[blockIdx.y];
   const int x = corr_only ? F.nw : (int)blockIdx.x;
   if (x > F.nw) {
-    if (!F.plan_ent || F.precision != SP_PRECISION_FP64) return;
+    if (!F.plan_ent) return;
     const size_t n = (size_t)F.nv, stride = (size_t)(gridDim.x - F.nw - 1) * 64;
     for (size_t i = (size_t)(x - F.nw - 1) * 64 + threadIdx.x; i < n; i += stride) F.dG[i] = make_double2(0.0, 0.0);
     return;
@@ -288,6 +280,7 @@ __global__ __launch_bounds__(kSigmaThreads) void k_dsigma(const FlowDev *__restr
 }
 
 #include "su2_rhs.h"
+#include "su2_mixed.h"
 
 // ---------------------------------------------------------------------------
 // dGamma/dLambda, general kernel: the mixed form, and lattices of more than
@@ -1228,19 +1221,14 @@ int check_problem(sp_ctx *ctx, const sp_su2_problem *p) {
 // SIMD each for the 256-thread shape, so SPFRG_MIN_BLOCKS (FP64, 4) or
 // SPFRG_MIN_BLOCKS_MIXED (mixed form, 5: it needs fewer registers; the mixed
 // 256-thread kernel is also compiled for 4, which flows whose LDS plan needs
-// more than 160 KB / 5 run, since its code is 1-3 % faster at L = 31).  The
-// 128-thread shape of small lattices is compiled for 4 in both forms.
-constexpr int resident_blocks(int vs, int nt) {
-  return (vs == 4 && nt != kSmallThreads) ? SPFRG_MIN_BLOCKS_MIXED : SPFRG_MIN_BLOCKS;
+// more than 160 KB / 5 run).
+constexpr int resident_blocks(int vs) {
+  return vs == 4 ? SPFRG_MIN_BLOCKS_MIXED : SPFRG_MIN_BLOCKS;
 }
 // LDS budget of one dGamma workgroup: a quarter of the CU's 160 KB keeps four
-// workgroups resident.  The 128-thread workgroups of small lattices keep it
-// too: more points per chunk at six or seven workgroups per CU measured 2-6 %
-// faster than the eighth of the LDS that eight resident workgroups would allow
-// (L = 9, 11, 16).  Where the registers allow more workgroups per CU, the
+// workgroups resident.  Where the registers allow more workgroups per CU, the
 // plan takes the smaller share 160 KB / resident_blocks if its chunks still
-// hold at least three points per worker slot (mixed form, L = 23: 24 instead
-// of 32 points, 3-14 % faster); with fewer (L = 31: 12 instead of 24) the
+// hold at least three points per worker slot; with fewer, the
 // larger chunks at four workgroups per CU were faster at small cutoffs.  A
 // flow whose plan ends up within the smaller share runs the kernel compiled
 // for more workgroups, any other the one compiled for four.
@@ -1258,7 +1246,7 @@ void launch_shape(int nw, int L, int vs, int nt, int &slots, int &nb, size_t &ld
   slots = (nt - 64) / L;
   const int maxb = vs == 4 ? kMaxBatchMixed : kMaxBatch;
   const int per0 = maxb / slots > 1 ? maxb / slots : 1;
-  const int rb = resident_blocks(vs, nt);
+  const int rb = resident_blocks(vs);
   if (rb > 4) {
     for (int per = per0; per >= kMinPerSlotHigh; --per) {
       nb = slots * per < 32 ? slots * per : 32;
@@ -1279,26 +1267,27 @@ size_t lds_of(const FlowDev &f) {
 
 // Flows of one dGamma launch share its workgroup size and its dynamic LDS
 // size, the largest of them; a flow whose plan fits a budget must not run at
-// the occupancy of a larger one.  Launch class = precision x workgroup size x
+// the occupancy of a larger one.  Launch class = precision x
 // LDS level (within 160 KB / resident_blocks, within kLdsBudget, above); a
 // batch issues one launch per class.
-// FP64 flows of up to kMaxRhsL sites run the wave kernels of su2_rhs.h, whose
-// class is the compiled lane shapes of k_su and k_t.
-constexpr int kLdsClasses = 12;
-constexpr int kLaunchClasses = kLdsClasses + 3 * 4 * 2;
+// Flows of up to kMaxRhsL sites run the wave kernels of su2_rhs.h and
+// su2_mixed.h, whose class is the compiled lane shapes and the precision.
+constexpr int kLdsClasses = 6;
+constexpr int kLaunchClasses = kLdsClasses + 3 * 4 * 2 * 2;
 int t_index(const TShape &t) { return t.ft == 2 ? 3 : (t.ft == 0 ? 0 : 1 + t.ht); }
-bool wave_form(const FlowDev &f) { return f.precision == SP_PRECISION_FP64 && f.plan_ent; }
+bool wave_form(const FlowDev &f) { return f.plan_ent != nullptr; }
 int lds_level(const FlowDev &f) {
   const int vs = f.precision == SP_PRECISION_MIXED ? 4 : 8;
   const size_t lds = lds_of(f);
-  return lds <= (size_t)160 * 1024 / resident_blocks(vs, f.nt) ? 0 : (lds <= kLdsBudget ? 1 : 2);
+  return lds <= (size_t)160 * 1024 / resident_blocks(vs) ? 0 : (lds <= kLdsBudget ? 1 : 2);
 }
 int launch_class(const FlowDev &f) {
   if (wave_form(f)) {
     const TShape t = t_shape(f.L);
-    return kLdsClasses + ((su_shape(f.L).rho - 1) * 4 + t_index(t)) * 2 + f.asym;
+    return kLdsClasses + (((su_shape(f.L).rho - 1) * 4 + t_index(t)) * 2 + f.asym) * 2 +
+           (f.precision == SP_PRECISION_MIXED ? 1 : 0);
   }
-  return ((f.precision == SP_PRECISION_MIXED ? 2 : 0) + (f.nt == kSmallThreads ? 1 : 0)) * 3 + lds_level(f);
+  return (f.precision == SP_PRECISION_MIXED ? 1 : 0) * 3 + lds_level(f);
 }
 
 // Launch geometry of a set of flows held in a host array (h) whose device copy is d.
@@ -1322,14 +1311,20 @@ long long su_flow_blocks(const FlowDev &f) { return (su_units(f.nw) + kRhsWaves 
 long long t_flow_blocks(const FlowDev &f) { return (f.nf + kRhsWaves - 1) / kRhsWaves; }
 
 template <int RHO>
-void launch_su(bool asym, dim3 grid, size_t lds, hipStream_t st, const FlowDev *d, int n, long long blocks) {
-  if (asym) hipLaunchKernelGGL((k_su<RHO, true>), grid, dim3(64 * kRhsWaves), lds, st, d, n, blocks);
-  else hipLaunchKernelGGL((k_su<RHO, false>), grid, dim3(64 * kRhsWaves), lds, st, d, n, blocks);
+void launch_su(bool mixed, bool asym, dim3 grid, size_t lds, hipStream_t st, const FlowDev *d, int n, long long blocks) {
+  const dim3 nt(64 * kRhsWaves);
+  if (mixed && asym) hipLaunchKernelGGL((k_su32<RHO, true>), grid, nt, lds, st, d, n, blocks);
+  else if (mixed) hipLaunchKernelGGL((k_su32<RHO, false>), grid, nt, lds, st, d, n, blocks);
+  else if (asym) hipLaunchKernelGGL((k_su<RHO, true>), grid, nt, lds, st, d, n, blocks);
+  else hipLaunchKernelGGL((k_su<RHO, false>), grid, nt, lds, st, d, n, blocks);
 }
 template <int FT, int HT>
-void launch_t(bool asym, dim3 grid, size_t lds, hipStream_t st, const FlowDev *d, int n, long long blocks) {
-  if (asym) hipLaunchKernelGGL((k_t<FT, HT, true>), grid, dim3(64 * kRhsWaves), lds, st, d, n, blocks);
-  else hipLaunchKernelGGL((k_t<FT, HT, false>), grid, dim3(64 * kRhsWaves), lds, st, d, n, blocks);
+void launch_t(bool mixed, bool asym, dim3 grid, size_t lds, hipStream_t st, const FlowDev *d, int n, long long blocks) {
+  const dim3 nt(64 * kRhsWaves);
+  if (mixed && asym) hipLaunchKernelGGL((k_t32<FT, HT, true>), grid, nt, lds, st, d, n, blocks);
+  else if (mixed) hipLaunchKernelGGL((k_t32<FT, HT, false>), grid, nt, lds, st, d, n, blocks);
+  else if (asym) hipLaunchKernelGGL((k_t<FT, HT, true>), grid, nt, lds, st, d, n, blocks);
+  else hipLaunchKernelGGL((k_t<FT, HT, false>), grid, nt, lds, st, d, n, blocks);
 }
 
 // dGamma of n flows of one wave class
@@ -1338,23 +1333,23 @@ hipError_t launch_wave_form(hipStream_t st, const FlowDev *d, const FlowDev *h, 
   size_t su_lds = 0, t_lds = 0;
   for (int i = 0; i < n; ++i) {
     const size_t mesh = (size_t)(h[i].nw * 8 + 15) & ~size_t(15);
-    su_lds = std::max(su_lds, mesh + (size_t)kRhsWaves * kSuWaveBytes);
+    su_lds = std::max(su_lds, mesh + (size_t)kRhsWaves * (h[i].precision == SP_PRECISION_MIXED ? su32_wave_bytes(h[i].L, su_shape(h[i].L).rho) : kSuWaveBytes));
     t_lds = std::max(t_lds, mesh + (size_t)kRhsWaves * t_wave_bytes(h[i].L));
   }
   auto grid = [](long long blocks) {
     return dim3((unsigned)((blocks + 8 * kChunk - 1) / (8 * kChunk) * 8 * kChunk));
   };
-  const bool asym = h[0].asym != 0;
+  const bool asym = h[0].asym != 0, mixed = h[0].precision == SP_PRECISION_MIXED;
   switch (su_shape(h[0].L).rho) {
-    case 1: launch_su<1>(asym, grid(su_blocks), su_lds, st, d, n, su_blocks); break;
-    case 2: launch_su<2>(asym, grid(su_blocks), su_lds, st, d, n, su_blocks); break;
-    default: launch_su<3>(asym, grid(su_blocks), su_lds, st, d, n, su_blocks); break;
+    case 1: launch_su<1>(mixed, asym, grid(su_blocks), su_lds, st, d, n, su_blocks); break;
+    case 2: launch_su<2>(mixed, asym, grid(su_blocks), su_lds, st, d, n, su_blocks); break;
+    default: launch_su<3>(mixed, asym, grid(su_blocks), su_lds, st, d, n, su_blocks); break;
   }
   switch (t_index(t_shape(h[0].L))) {
-    case 0: launch_t<0, 1>(asym, grid(t_blocks), t_lds, st, d, n, t_blocks); break;
-    case 1: launch_t<1, 0>(asym, grid(t_blocks), t_lds, st, d, n, t_blocks); break;
-    case 2: launch_t<1, 1>(asym, grid(t_blocks), t_lds, st, d, n, t_blocks); break;
-    default: launch_t<2, 0>(asym, grid(t_blocks), t_lds, st, d, n, t_blocks); break;
+    case 0: launch_t<0, 1>(mixed, asym, grid(t_blocks), t_lds, st, d, n, t_blocks); break;
+    case 1: launch_t<1, 0>(mixed, asym, grid(t_blocks), t_lds, st, d, n, t_blocks); break;
+    case 2: launch_t<1, 1>(mixed, asym, grid(t_blocks), t_lds, st, d, n, t_blocks); break;
+    default: launch_t<2, 0>(mixed, asym, grid(t_blocks), t_lds, st, d, n, t_blocks); break;
   }
   return hipGetLastError();
 }
@@ -1405,11 +1400,8 @@ hipError_t launch_compute(hipStream_t st, const FlowDev *d, const FlowDev *h, in
       const int nt = h[i0].nt;
       // plans within 160 KB / resident_blocks run the kernel compiled for
       // that many resident workgroups
-      const bool high = lds_level(h[i0]) == 0 && resident_blocks(mixed ? 4 : 8, nt) > SPFRG_MIN_BLOCKS;
-      if (mixed && nt == kSmallThreads)
-        hipLaunchKernelGGL((k_dgamma<true, kSmallThreads, SPFRG_MIN_BLOCKS>), dim3(grid), dim3(nt), lds, st, d + i0,
-                           i1 - i0, total, per_xcd);
-      else if (mixed && high)
+      const bool high = lds_level(h[i0]) == 0 && resident_blocks(mixed ? 4 : 8) > SPFRG_MIN_BLOCKS;
+      if (mixed && high)
         hipLaunchKernelGGL((k_dgamma<true, kThreads, SPFRG_MIN_BLOCKS_MIXED>), dim3(grid), dim3(nt), lds, st, d + i0,
                            i1 - i0, total, per_xcd);
       else if (mixed)
@@ -1521,7 +1513,7 @@ int sp_ctx_create(const sp_su2_problem *p, sp_ctx **out) {
   f.spin = p->spin;
   f.precision = p->precision;
   f.item_base = 0;
-  f.nt = dgamma_threads(f.L);
+  f.nt = kThreads;
   launch_shape(f.nw, f.L, f.precision == SP_PRECISION_MIXED ? 4 : 8, f.nt, f.slots, f.nb, ctx->lds);
   int max_lds = 0;
   SP_HIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device));
@@ -1630,8 +1622,6 @@ int sp_ctx_create(const sp_su2_problem *p, sp_ctx **out) {
   SP_HIP(hipFuncSetAttribute((const void *)k_dgamma<true, kThreads, SPFRG_MIN_BLOCKS>,
                              hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
   SP_HIP(hipFuncSetAttribute((const void *)k_dgamma<true, kThreads, SPFRG_MIN_BLOCKS_MIXED>,
-                             hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
-  SP_HIP(hipFuncSetAttribute((const void *)k_dgamma<true, kSmallThreads, SPFRG_MIN_BLOCKS>,
                              hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
   SP_HIP(hipMemcpy(ctx->d_fd, &f, sizeof(FlowDev), hipMemcpyHostToDevice));
   return SP_OK;

@@ -352,10 +352,155 @@ inline void build_overlap_plan(LanePlan &plan, int L, const int *off, const int 
   plan.deal(64);
 }
 
+// the bubble matrix of both channels in a wave's registers: full tiles, full
+// rows x half columns, half rows x full columns, half tile
+template <int FT, int HT> struct BubbleTiles {
+  d4 c[2][FT ? FT * FT : 1];
+  double2 r[2][FT ? FT : 1], l[2][FT ? FT : 1], h[2];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int ch = 0; ch < 2; ++ch) {
+#pragma unroll
+      for (int k = 0; k < FT * FT; ++k) c[ch][k] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < FT; ++k) r[ch][k] = l[ch][k] = make_double2(0.0, 0.0);
+      h[ch] = make_double2(0.0, 0.0);
+    }
+  }
+  // half tile: even and odd points in blocks of their own
+  __device__ __forceinline__ void half(const double (&ph)[2], const double (&qh)[2]) {
+#pragma unroll
+    for (int ch = 0; ch < 2; ++ch) {
+      h[ch].x = mfma_blocks(ph[ch], qh[ch], h[ch].x);
+      h[ch].y = mfma_blocks(ph[ch], half_mirror(qh[ch]), h[ch].y);
+    }
+  }
+  // the even (par 0) or odd points of the full tiles, and of the half tile with them
+  __device__ __forceinline__ void full(int par, const double (&P)[FT ? FT : 1][2], const double (&Q)[FT ? FT : 1][2],
+                                       const double (&ph)[2], const double (&qh)[2]) {
+#pragma unroll
+    for (int ch = 0; ch < 2; ++ch) {
+#pragma unroll
+      for (int i = 0; i < FT; ++i)
+#pragma unroll
+        for (int j = 0; j < FT; ++j) outer_update(c[ch][i * FT + j], P[i][ch], Q[j][ch]);
+      if (HT) {
+        // the half tile at these points in both halves of the rows
+        const double p = par ? row_move<0x128, 0x3>(ph[ch]) : row_move<0x128, 0xc>(ph[ch]);
+        const double q = par ? row_move<0x128, 0x3>(qh[ch]) : row_move<0x128, 0xc>(qh[ch]);
+        const double pm = half_mirror(p), qm = half_mirror(q);
+#pragma unroll
+        for (int i = 0; i < FT; ++i) {
+          r[ch][i].x = mfma_blocks(P[i][ch], q, r[ch][i].x);
+          r[ch][i].y = mfma_blocks(P[i][ch], qm, r[ch][i].y);
+          l[ch][i].x = mfma_blocks(p, Q[i][ch], l[ch][i].x);
+          l[ch][i].y = mfma_blocks(pm, Q[i][ch], l[ch][i].y);
+        }
+      }
+    }
+  }
+  // channel ch into LDS, rows of 16 FT + 8 HT
+  __device__ __forceinline__ void store(int ch, double *s_C, int lane) const {
+    constexpr int LP = 16 * FT + 8 * HT;
+    // lane (ri, b, rj) holds elements (4 b + ri, rj of another block of columns)
+    const int ri = lane >> 4, cb = (lane >> 2) & 3, rj = lane & 3;
+#pragma unroll
+    for (int i = 0; i < FT; ++i) {
+      const int row = (16 * i + 4 * cb + ri) * LP;
+#pragma unroll
+      for (int j = 0; j < FT; ++j)
+#pragma unroll
+        for (int z = 0; z < 4; ++z) s_C[row + 16 * j + 4 * ((cb + z) & 3) + rj] = c[ch][i * FT + j][z];
+      if (HT) {
+        const int h0 = 16 * FT, lo = 4 * (cb & 1), hi = 4 * (1 - (cb & 1)) + 3;
+        s_C[row + h0 + lo + rj] = r[ch][i].x;
+        s_C[row + h0 + hi - rj] = r[ch][i].y;
+        s_C[(h0 + lo + ri) * LP + 16 * i + 4 * cb + rj] = l[ch][i].x;
+        s_C[(h0 + hi - ri) * LP + 16 * i + 4 * cb + rj] = l[ch][i].y;
+      }
+    }
+    if (HT) {
+      const double x = h[ch].x + half_row_swap(h[ch].x), y = h[ch].y + half_row_swap(h[ch].y);
+      if (cb < 2) {
+        double *o = s_C + (16 * FT + 4 * cb + ri) * LP + 16 * FT;
+        o[4 * cb + rj] = x;
+        o[4 * (1 - cb) + 3 - rj] = y;
+      }
+    }
+  }
+};
+
+// the end of an item: the overlap sums of the bubble matrix, the sums over the
+// points (rs, rd: per tile of sites), S and U values, prefactor and 2^scale.
+// wl: the wave's LDS.  MIXED: an FP32 term that overflowed makes the value NaN,
+// as it does a compensated FP32 sum, so that the flow counts as diverged.
+template <bool MIXED, int FT, int HT>
+__device__ __forceinline__ void t_finish(const FlowDev &F, const BubbleTiles<FT, HT> &C, const double (&rs)[FT + HT],
+                                         const double (&rd)[FT + HT], unsigned char *wl, int item, int scale) {
+  // RPA(rid) = sum over getOverlap(rid) of C[rid1][rid2] (src/SU2/SU2FrgCore.cpp:250-266)
+  constexpr int LP = 16 * FT + 8 * HT, NT = FT + HT;
+  const int L = F.L, lane = threadIdx.x & 63;
+  double *s_C = reinterpret_cast<double *>(wl);
+  double *s_part = s_C + LP * LP;
+  const int cnt = F.plan_count[lane];
+  double rpa[2] = {0.0, 0.0};
+#pragma unroll
+  for (int ch = 0; ch < 2; ++ch) {
+    wave_lds_fence();
+    C.store(ch, s_C, lane);
+    wave_lds_fence();
+    s_part[lane] = plan_sum(reinterpret_cast<const uint4 *>(F.plan_ent) + lane, 64, cnt, s_C);
+    wave_lds_fence();
+    if (lane < L) {
+      const int l1 = F.plan_lane[lane + 1];
+      for (int l = F.plan_lane[lane]; l < l1; ++l) rpa[ch] += s_part[l];
+    }
+  }
+  // sum over the points, S and U values, prefactor 1/(2 pi) (src/SU2/SU2FrgCore.cpp:426-430)
+  double ts = 0.0, td = 0.0;
+#pragma unroll
+  for (int k = 0; k < NT; ++k) {
+    double x = rs[k], y = rd[k];
+    if (k >= FT) {
+      x += __shfl_xor(x, 8, 64);
+      y += __shfl_xor(y, 8, 64);
+    }
+    x += __shfl_xor(x, 16, 64);
+    y += __shfl_xor(y, 16, 64);
+    x += __shfl_xor(x, 32, 64);
+    y += __shfl_xor(y, 32, 64);
+    if (lane >= 16 * k) {
+      ts = x;
+      td = y;
+    }
+  }
+  if (lane < L) {
+    double2 *out = F.dG + (size_t)item * L + lane;
+    const double2 su_sum = *out;
+    if (MIXED) {
+      const double nan = __builtin_nan("");
+      ts += su_sum.x;
+      td += su_sum.y;
+      if (isinf(ts)) ts = nan;
+      if (isinf(td)) td = nan;
+      ts = fma(2.0 * F.spin, rpa[0], ts) * (1.0 / kTwoPi);
+      td = fma(8.0 * F.spin, rpa[1], td) * (1.0 / kTwoPi);
+    } else {
+      ts = (fma(2.0 * F.spin, rpa[0], ts) + su_sum.x) * (1.0 / kTwoPi);
+      td = (fma(8.0 * F.spin, rpa[1], td) + su_sum.y) * (1.0 / kTwoPi);
+    }
+    if (scale != 0) {
+      ts = ldexp(ts, scale);
+      td = ldexp(td, scale);
+    }
+    *out = make_double2(ts, td);
+    if (isnan(ts) || isnan(td)) atomicOr(&F.flags[0], 1);
+  }
+}
+
 template <int FT, int HT, bool ASYM>
 __global__ __launch_bounds__(64 * kRhsWaves, FT + HT == 1 ? 4 : 3) void k_t(const FlowDev *__restrict__ fl, int nflows, long long total) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  constexpr int LP = 16 * FT + 8 * HT;
   constexpr int NT = FT + HT;
   const long long blk = xcd_position(blockIdx.x, kChunk);
   if (blk >= total) return;
@@ -404,17 +549,8 @@ __global__ __launch_bounds__(64 * kRhsWaves, FT + HT == 1 ? 4 : 3) void k_t(cons
   double rs[NT], rd[NT];
 #pragma unroll
   for (int k = 0; k < NT; ++k) rs[k] = rd[k] = 0.0;
-  // bubble matrix: full tiles, full rows x half columns, half rows x full columns, half tile
-  d4 C[2][FT ? FT * FT : 1];
-  double2 Cr[2][FT ? FT : 1], Cc[2][FT ? FT : 1], Ch[2];
-#pragma unroll
-  for (int ch = 0; ch < 2; ++ch) {
-#pragma unroll
-    for (int k = 0; k < FT * FT; ++k) C[ch][k] = d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int k = 0; k < FT; ++k) Cr[ch][k] = Cc[ch][k] = make_double2(0.0, 0.0);
-    Ch[ch] = make_double2(0.0, 0.0);
-  }
+  BubbleTiles<FT, HT> C;
+  C.clear();
 
   // producer role: point pe, pair pp, argument pj: A (pj 0) and B (pj 1) of
   // pair 0: A = w1 - w', B = w1p + w'; pair 1: A = w2p - w', B = w2 + w'
@@ -562,12 +698,7 @@ __global__ __launch_bounds__(64 * kRhsWaves, FT + HT == 1 ? 4 : 3) void k_t(cons
       double ph[2], qh[2];
       if (HT) {
         gather(FT, eb + (lane >> 3), ph, qh);
-#pragma unroll
-        for (int ch = 0; ch < 2; ++ch) {
-          // even and odd points in blocks of their own
-          Ch[ch].x = mfma_blocks(ph[ch], qh[ch], Ch[ch].x);
-          Ch[ch].y = mfma_blocks(ph[ch], half_mirror(qh[ch]), Ch[ch].y);
-        }
+        C.half(ph, qh);
       }
       // the full tiles' even points, then the odd ones
 #pragma unroll
@@ -575,96 +706,10 @@ __global__ __launch_bounds__(64 * kRhsWaves, FT + HT == 1 ? 4 : 3) void k_t(cons
         double P[FT ? FT : 1][2], Q[FT ? FT : 1][2];
 #pragma unroll
         for (int i = 0; i < FT; ++i) gather(i, eb + 2 * (lane >> 4) + par, P[i], Q[i]);
-#pragma unroll
-        for (int ch = 0; ch < 2; ++ch) {
-#pragma unroll
-          for (int i = 0; i < FT; ++i)
-#pragma unroll
-            for (int j = 0; j < FT; ++j) outer_update(C[ch][i * FT + j], P[i][ch], Q[j][ch]);
-          if (HT) {
-            // the half tile at these points in both halves of the rows
-            const double p = par ? row_move<0x128, 0x3>(ph[ch]) : row_move<0x128, 0xc>(ph[ch]);
-            const double q = par ? row_move<0x128, 0x3>(qh[ch]) : row_move<0x128, 0xc>(qh[ch]);
-            const double pm = half_mirror(p), qm = half_mirror(q);
-#pragma unroll
-            for (int i = 0; i < FT; ++i) {
-              Cr[ch][i].x = mfma_blocks(P[i][ch], q, Cr[ch][i].x);
-              Cr[ch][i].y = mfma_blocks(P[i][ch], qm, Cr[ch][i].y);
-              Cc[ch][i].x = mfma_blocks(p, Q[i][ch], Cc[ch][i].x);
-              Cc[ch][i].y = mfma_blocks(pm, Q[i][ch], Cc[ch][i].y);
-            }
-          }
-        }
+        C.full(par, P, Q, ph, qh);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
-
-  // RPA(rid) = sum over getOverlap(rid) of C[rid1][rid2] (src/SU2/SU2FrgCore.cpp:250-266)
-  double *s_C = reinterpret_cast<double *>(wl);
-  double *s_part = s_C + LP * LP;
-  const int cnt = F.plan_count[lane];
-  // lane (ri, b, rj) holds elements (4 b + ri, rj of another block of columns)
-  const int ri = lane >> 4, cb = (lane >> 2) & 3, rj = lane & 3;
-  double rpa[2] = {0.0, 0.0};
-#pragma unroll
-  for (int ch = 0; ch < 2; ++ch) {
-    wave_lds_fence();
-#pragma unroll
-    for (int i = 0; i < FT; ++i) {
-      const int row = (16 * i + 4 * cb + ri) * LP;
-#pragma unroll
-      for (int j = 0; j < FT; ++j)
-#pragma unroll
-        for (int z = 0; z < 4; ++z) s_C[row + 16 * j + 4 * ((cb + z) & 3) + rj] = C[ch][i * FT + j][z];
-      if (HT) {
-        const int h = 16 * FT, lo = 4 * (cb & 1), hi = 4 * (1 - (cb & 1)) + 3;
-        s_C[row + h + lo + rj] = Cr[ch][i].x;
-        s_C[row + h + hi - rj] = Cr[ch][i].y;
-        s_C[(h + lo + ri) * LP + 16 * i + 4 * cb + rj] = Cc[ch][i].x;
-        s_C[(h + hi - ri) * LP + 16 * i + 4 * cb + rj] = Cc[ch][i].y;
-      }
-    }
-    if (HT) {
-      const double x = Ch[ch].x + half_row_swap(Ch[ch].x), y = Ch[ch].y + half_row_swap(Ch[ch].y);
-      if (cb < 2) {
-        double *o = s_C + (16 * FT + 4 * cb + ri) * LP + 16 * FT;
-        o[4 * cb + rj] = x;
-        o[4 * (1 - cb) + 3 - rj] = y;
-      }
-    }
-    wave_lds_fence();
-    s_part[lane] = plan_sum(reinterpret_cast<const uint4 *>(F.plan_ent) + lane, 64, cnt, s_C);
-    wave_lds_fence();
-    if (lane < L) {
-      const int l1 = F.plan_lane[lane + 1];
-      for (int l = F.plan_lane[lane]; l < l1; ++l) rpa[ch] += s_part[l];
-    }
-  }
-  // sum over the points, S and U values, prefactor 1/(2 pi) (src/SU2/SU2FrgCore.cpp:426-430)
-  double ts = 0.0, td = 0.0;
-#pragma unroll
-  for (int k = 0; k < NT; ++k) {
-    double x = rs[k], y = rd[k];
-    if (k >= FT) {
-      x += __shfl_xor(x, 8, 64);
-      y += __shfl_xor(y, 8, 64);
-    }
-    x += __shfl_xor(x, 16, 64);
-    y += __shfl_xor(y, 16, 64);
-    x += __shfl_xor(x, 32, 64);
-    y += __shfl_xor(y, 32, 64);
-    if (lane >= 16 * k) {
-      ts = x;
-      td = y;
-    }
-  }
-  if (lane < L) {
-    double2 *out = F.dG + (size_t)item * L + lane;
-    const double2 su_sum = *out;
-    ts = (fma(2.0 * F.spin, rpa[0], ts) + su_sum.x) * (1.0 / kTwoPi);
-    td = (fma(8.0 * F.spin, rpa[1], td) + su_sum.y) * (1.0 / kTwoPi);
-    *out = make_double2(ts, td);
-    if (isnan(ts) || isnan(td)) atomicOr(&F.flags[0], 1);
-  }
+  t_finish<false, FT, HT>(F, C, rs, rd, wl, item, 0);
 }
