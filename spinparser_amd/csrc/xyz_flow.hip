@@ -832,6 +832,18 @@ __global__ __launch_bounds__(kXyzThreads) void k_xyz_dgamma_direct(XyzDev F) {
   }
 }
 
+// rows between the reference's planes (n values each in `in` or `out`) and the
+// device layout; place: position of (rid, component) within a row
+__global__ void k_xyz_reorder(const double *__restrict__ in, double *__restrict__ out, long long n, int L,
+                              const int *__restrict__ place, int to_rows) {
+  const long long stride = (long long)gridDim.x * blockDim.x;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < 4 * n; i += stride) {
+    const long long c = i / n, q = i - c * n, row = q / L, at = row * 4 * L + place[4 * (int)(q - row * L) + (int)c];
+    if (to_rows) out[at] = in[i];
+    else out[i] = in[at];
+  }
+}
+
 // in-place explicit Euler step (src/XYZ/XYZFrgCore.cpp:128-162); skipped when
 // the flow holds a NaN (src/SpinParser.cpp:151-159)
 __global__ void k_xyz_euler(XyzDev F) {
@@ -993,8 +1005,9 @@ struct sp_xyz_ctx {
   bool direct = false;  // bubble summed per point (k_xyz_dgamma_direct)
   size_t lds = 0;
   std::vector<void *> allocs;
-  std::vector<double> host;  // staging of the state between the planes and the device layout
-  std::vector<int> place;    // position of (rid, component) within a device row
+  double *stage = nullptr;  // rows as planes on their way to and from the host
+  std::vector<int> place;   // position of (rid, component) within a device row
+  int *d_place = nullptr;
   bool prof = false;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> pending[4];
   double prof_ms[4] = {0, 0, 0, 0};
@@ -1275,17 +1288,31 @@ struct XyzTables {
   }
 };
 
-// the reference's four planes X, Y, Z, D <-> the device layout (place: position
-// of (rid, component) within a row)
-void planes_to_rows(const double *planes, double *out, size_t np, int L, const int *place) {
-  for (int c = 0; c < 4; ++c)
-    for (size_t row = 0; row * L < np; ++row)
-      for (int r = 0; r < L; ++r) out[row * 4 * L + place[4 * r + c]] = planes[c * np + row * L + r];
+// rows in the staging buffer: at most 32 MiB
+long long xyz_stage_rows(long long np, int L) {
+  const long long rows = (32ll << 20) / (4 * L * 8), all = np / L;
+  return rows < all ? rows : all;
 }
-void rows_to_planes(const double *in, double *planes, size_t np, int L, const int *place) {
-  for (int c = 0; c < 4; ++c)
-    for (size_t row = 0; row * L < np; ++row)
-      for (int r = 0; r < L; ++r) planes[c * np + row * L + r] = in[row * 4 * L + place[4 * r + c]];
+// a vertex from (to_rows) or to the reference's four planes X, Y, Z, D on the host
+int xyz_copy(sp_xyz_ctx *ctx, double *dev, double *planes, bool to_rows) {
+  const XyzDev &F = ctx->fd;
+  const long long total = F.np / F.L, rows = xyz_stage_rows(F.np, F.L);
+  for (long long r0 = 0; r0 < total; r0 += rows) {
+    const long long n = (total - r0 < rows ? total - r0 : rows) * F.L;  // values per plane
+    const unsigned blocks = (unsigned)((4 * n + 255) / 256 < 4096 ? (4 * n + 255) / 256 : 4096);
+    double *at = dev + r0 * 4 * F.L;
+    if (to_rows)
+      for (int c = 0; c < 4; ++c)
+        SP_XHIP(hipMemcpy(ctx->stage + c * n, planes + c * (long long)F.np + r0 * F.L, (size_t)n * 8, hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_xyz_reorder, dim3(blocks), dim3(256), 0, ctx->stream, to_rows ? ctx->stage : at,
+                       to_rows ? at : ctx->stage, n, F.L, ctx->d_place, to_rows ? 1 : 0);
+    SP_XHIP(hipGetLastError());
+    SP_XHIP(hipStreamSynchronize(ctx->stream));
+    if (!to_rows)
+      for (int c = 0; c < 4; ++c)
+        SP_XHIP(hipMemcpy(planes + c * (long long)F.np + r0 * F.L, ctx->stage + c * n, (size_t)n * 8, hipMemcpyDeviceToHost));
+  }
+  return SP_OK;
 }
 
 }  // namespace
@@ -1303,6 +1330,7 @@ int sp_xyz_ctx_footprint(const sp_xyz_problem *p, long long *bytes) {
   b += emax * 4 * p->L * 8 + 4LL * p->B * p->Rb * 8 + 16;                     // correlation scratch, output, flags
   b += 4LL * (8 * p->L + 1 + 8 * O + 2 * p->R + 4 * p->B * p->Rb);            // lattice tables
   b += 16LL * O;                                                              // bubble-matrix indices
+  b += std::min<long long>(nf * 4 * p->L * 8, 32ll << 20) + 16LL * p->L;      // staging rows, their order
   *bytes = b;
   return SP_OK;
 }
@@ -1455,7 +1483,10 @@ static int xyz_ctx_init(sp_xyz_ctx *ctx, const sp_xyz_problem *p, const XyzOrder
   SP_XHIP(hipMemset(f.Cn, 0, 4));
   SP_XHIP(hipFuncSetAttribute((const void *)k_xyz_dgamma, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
   SP_XHIP(hipFuncSetAttribute((const void *)k_xyz_dgamma_direct, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
-  ctx->host.resize(nv);
+  if ((rc = xalloc(ctx, &ctx->stage, (size_t)xyz_stage_rows(f.np, f.L) * 4 * f.L)) ||
+      (rc = xalloc(ctx, &ctx->d_place, ctx->place.size())))
+    return rc;
+  SP_XHIP(hipMemcpy(ctx->d_place, ctx->place.data(), ctx->place.size() * 4, hipMemcpyHostToDevice));
   return SP_OK;
 }
 
@@ -1476,8 +1507,7 @@ int sp_xyz_set_state(sp_xyz_ctx *ctx, double cutoff, const double *v2, const dou
   if (!std::isfinite(cutoff) || !(cutoff > 0.0)) return xfail(ctx, SP_EARG, "cutoff must be finite and positive");
   SP_XHIP(hipStreamSynchronize(ctx->stream));
   SP_XHIP(hipMemcpy(ctx->fd.v2, v2, ctx->fd.nw * 8, hipMemcpyHostToDevice));
-  planes_to_rows(v4, ctx->host.data(), (size_t)ctx->fd.np, ctx->fd.L, ctx->place.data());
-  SP_XHIP(hipMemcpy(ctx->fd.G, ctx->host.data(), 4 * (size_t)ctx->fd.np * 8, hipMemcpyHostToDevice));
+  if (int rc = xyz_copy(ctx, ctx->fd.G, const_cast<double *>(v4), true)) return rc;
   SP_XHIP(hipMemset(ctx->fd.flags, 0, 16));
   ctx->cutoff = cutoff;
   ctx->have_flow = false;
@@ -1489,10 +1519,8 @@ int sp_xyz_get_state(sp_xyz_ctx *ctx, double *cutoff, double *v2, double *v4) {
   SP_XHIP(hipStreamSynchronize(ctx->stream));
   if (cutoff) *cutoff = ctx->cutoff;
   if (v2) SP_XHIP(hipMemcpy(v2, ctx->fd.v2, ctx->fd.nw * 8, hipMemcpyDeviceToHost));
-  if (v4) {
-    SP_XHIP(hipMemcpy(ctx->host.data(), ctx->fd.G, 4 * (size_t)ctx->fd.np * 8, hipMemcpyDeviceToHost));
-    rows_to_planes(ctx->host.data(), v4, (size_t)ctx->fd.np, ctx->fd.L, ctx->place.data());
-  }
+  if (v4)
+    if (int rc = xyz_copy(ctx, ctx->fd.G, v4, false)) return rc;
   return SP_OK;
 }
 
@@ -1501,10 +1529,8 @@ int sp_xyz_get_flow(sp_xyz_ctx *ctx, double *dv2, double *dv4) {
   if (!ctx->have_flow) return xfail(ctx, SP_ESTATE, "no flow computed at the current cutoff");
   SP_XHIP(hipStreamSynchronize(ctx->stream));
   if (dv2) SP_XHIP(hipMemcpy(dv2, ctx->fd.dv2, ctx->fd.nw * 8, hipMemcpyDeviceToHost));
-  if (dv4) {
-    SP_XHIP(hipMemcpy(ctx->host.data(), ctx->fd.dG, 4 * (size_t)ctx->fd.np * 8, hipMemcpyDeviceToHost));
-    rows_to_planes(ctx->host.data(), dv4, (size_t)ctx->fd.np, ctx->fd.L, ctx->place.data());
-  }
+  if (dv4)
+    if (int rc = xyz_copy(ctx, ctx->fd.dG, dv4, false)) return rc;
   return SP_OK;
 }
 
