@@ -1146,11 +1146,11 @@ template <int... NG>
 void launch_tri_t(const TriDev &F, dim3 grid, size_t lds, hipStream_t st, std::integer_sequence<int, NG...>) {
   (launch_tri_t<NG>(F, grid, lds, st) || ...);
 }
-template <int... NG> hipError_t tri_t_allow_lds(int bytes, std::integer_sequence<int, NG...>) {
+template <int... NG> hipError_t tri_t_allow_lds(int ng, int bytes, std::integer_sequence<int, NG...>) {
   hipError_t e = hipFuncSetAttribute((const void *)k_tri_su, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  ((e == hipSuccess ? (e = hipFuncSetAttribute((const void *)k_tri_t<NG>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               bytes))
-                    : e),
+  ((e == hipSuccess && NG == ng
+        ? (e = hipFuncSetAttribute((const void *)k_tri_t<NG>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes))
+        : e),
    ...);
   return e;
 }
@@ -1400,10 +1400,13 @@ int sp_tri_ctx_create(const sp_tri_problem *p, sp_tri_ctx **out) {
   SP_THIP(hipMemset(f.flags, 0, 16));
   SP_THIP(hipMemset(f.Wn, 0, f.nw * 4));
   SP_THIP(hipMemset(f.Cn, 0, 4));
-  SP_THIP(hipFuncSetAttribute((const void *)k_tri_dgamma<kTriThreads, 0, 0>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
-  SP_THIP(tri_allow_lds(max_lds, TriShapes{}));
-  SP_THIP(tri_t_allow_lds(max_lds, TriGroups{}));
+  if (f.t_waves) {
+    SP_THIP(tri_t_allow_lds(f.t_ng, max_lds, TriGroups{}));
+  } else {
+    SP_THIP(hipFuncSetAttribute((const void *)k_tri_dgamma<kTriThreads, 0, 0>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
+    SP_THIP(tri_allow_lds(max_lds, TriShapes{}));
+  }
   return SP_OK;
 }
 

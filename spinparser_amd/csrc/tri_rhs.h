@@ -26,8 +26,11 @@
 //    over the points before the overlap lists are applied (k_tri_t).
 //
 // Kagome with DM exchange, 19 sites, 48 frequencies, against one workgroup per
-// item that forms all terms point by point: 12.9 -> 5.6 ms at cutoff 20, 46.3 ->
-// 15.7 ms at 0.7, 81.9 -> 27.2 ms at 0.02 (k_tri_su 8.2 ms, k_tri_t 19.0 ms).
+// item that forms all terms point by point: 12.9 -> 5.2 ms at cutoff 20, 46.3 ->
+// 14.1 ms at 0.7, 81.9 -> 24.1 ms at 0.02 (k_tri_su 8.2 ms, its gathers 70 % of
+// the cache's rate and its vector instructions 64 %; k_tri_t 15.8 ms, which
+// alternates between gathers, 11 ms by themselves, and matrix products, 13 ms by
+// themselves: the descriptors of the next points are formed beside the products).
 #pragma once
 
 constexpr int kMaxTriRhsL = 32;
@@ -406,14 +409,19 @@ constexpr int kTriTPoints = 8;  // points described at a time, at most
 constexpr int kTriEdges = 4;    // matrix instructions per wave for the kModeEdge entries, at most
 
 // Entries lie in pairs, {entry 2 p, entry 2 p + 1} of an element side by side:
-// one 16-byte read serves two.  Position of element (row, column) of a site's
-// matrix, bytes, less the entry's: rows rotated by the site, so that operands
-// of four sites with different residues come from different banks.
-__host__ __device__ inline int tri_el(int site, int row, int col) { return (site * 16 + ((row + site) & 3) * 4 + col) * 16; }
-__host__ __device__ inline int tri_mat(int L) { return (L + 1) * 256; }  // bytes of the X (or Y) of a pair of entries
+// one 16-byte read serves two.  Byte position of element (row, column) of a
+// site's matrix: equal rows of all sites together, 64 bytes each, so that four
+// sites with different residues (mod 4) lie in different banks (4.4 cycles per
+// wave read, 8 to 10 otherwise).  Rows are a multiple of four sites where the
+// padding is small, which makes this hold whatever the rows.
+__host__ __device__ inline int tri_sites(int L) { return L >= 12 ? (L + 4) & ~3 : L + 1; }
+__host__ __device__ inline int tri_el(int L, int site, int row, int col) {
+  return ((row * tri_sites(L) + site) * 4 + col) * 16;
+}
+__host__ __device__ inline int tri_mat(int L) { return tri_sites(L) * 256; }  // bytes of the X (or Y) of a pair of entries
 
 struct TriTLds {
-  int dst, off, w, fl, c, loff, lw, lfl, ent, loc, area, total;
+  int dst, off, w, pos, c, loff, lw, lfl, head, loc, area, total;
 };
 __host__ __device__ inline int tri_t_lanes(int L, int threads) { return (16 * L + threads - 1) / threads * threads; }
 __host__ __device__ inline TriTLds tri_t_lds(int nw, int L, int points, int entries, int threads) {
@@ -424,12 +432,12 @@ __host__ __device__ inline TriTLds tri_t_lds(int nw, int L, int points, int entr
   l.dst = take(4 * 8 * L * 4);
   l.off = take(2 * points * 16);
   l.w = take(2 * points * 32);
-  l.fl = take(2 * points * 4);
-  l.c = take(points * 8);
+  l.pos = take(2 * points * 16);
+  l.c = take(2 * points * 8);
   l.loff = take(4 * points * 16);
   l.lw = take(4 * points * 32);
   l.lfl = take(4 * points * 4);
-  l.ent = take((points + 1) * 4);
+  l.head = take(16);
   l.loc = take(points * 64 * 8);
   const int bun = entries * tri_mat(L);
   const int sums = 4 * threads * 8 + tri_t_lanes(L, threads) * 8;  // a group's products and the sums of the lanes
@@ -463,12 +471,12 @@ __global__ __launch_bounds__(512, NG <= 5 ? 4 : 2) void k_tri_t(TriDev F) {
   int *s_dst = reinterpret_cast<int *>(lds_raw + lay.dst);
   int4 *s_off = reinterpret_cast<int4 *>(lds_raw + lay.off);         // [(point, pair)]
   double2 *s_w = reinterpret_cast<double2 *>(lds_raw + lay.w);       // [(point, pair)][2], negative: exchanged storage
-  int *s_fl = reinterpret_cast<int *>(lds_raw + lay.fl);             // [(point, pair)]
-  double *s_c = reinterpret_cast<double *>(lds_raw + lay.c);
+  int4 *s_pos = reinterpret_cast<int4 *>(lds_raw + lay.pos);         // [(point, pair)] flags, byte positions of the two entries, mode
+  double *s_c = reinterpret_cast<double *>(lds_raw + lay.c);         // [(point, pair)] factor
   int4 *s_loff = reinterpret_cast<int4 *>(lds_raw + lay.loff);       // [(point, local)]
   double2 *s_lw = reinterpret_cast<double2 *>(lds_raw + lay.lw);
   int *s_lfl = reinterpret_cast<int *>(lds_raw + lay.lfl);
-  int *s_ent = reinterpret_cast<int *>(lds_raw + lay.ent);           // full entries before | edge entries before << 8 | mode << 16
+  int4 *s_head = reinterpret_cast<int4 *>(lds_raw + lay.head);       // points, full entries, edge entries
   double *s_loc = reinterpret_cast<double *>(lds_raw + lay.loc);     // [(point, local)][16]
   unsigned char *area = lds_raw + lay.area;
 
@@ -485,7 +493,7 @@ __global__ __launch_bounds__(512, NG <= 5 ? 4 : 2) void k_tri_t(TriDev F) {
   // (the second of a pair may be multiplied by zero before its first use)
   for (int i = tid; i < nent * mat / 16; i += nt) reinterpret_cast<double2 *>(area)[i] = make_double2(0.0, 0.0);
   // operand positions of the lane: left factor | first right factor << 16, second | third << 16, fourth
-  int pk[NG][3], pe_[kTriEdges];
+  int pk[NG][3];
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
     const int4 q = F.t_ops[(wave * NG + g) * 64 + lane];
@@ -494,8 +502,6 @@ __global__ __launch_bounds__(512, NG <= 5 ? 4 : 2) void k_tri_t(TriDev F) {
     pk[g][2] = q.z;
   }
   const int nedge = F.t_edges;
-#pragma unroll
-  for (int i = 0; i < kTriEdges; ++i) pe_[i] = i < nedge ? F.t_edge_ops[(wave * nedge + i) * 64 + lane] : 0;
   double C[NG][4], CE[kTriEdges];
 #pragma unroll
   for (int g = 0; g < NG; ++g)
@@ -515,174 +521,115 @@ __global__ __launch_bounds__(512, NG <= 5 ? 4 : 2) void k_tri_t(TriDev F) {
   const int pe = lane >> 2, pp = (lane >> 1) & 1, pj = lane & 1;
   const int n = F.Wn[X];
   const double *Wwp = F.Wwp + (size_t)X * F.emax, *Wc = F.Wc + (size_t)X * F.emax;
-  double half;
-  {
-    const double s = s_mesh[so], t = s_mesh[X], u = s_mesh[uo];
-    half = 0.5 * (s + (pj ? t : -t) + (pp ? -u : u));
-  }
-
-  for (int e0 = 0; e0 < n; e0 += npt) {
-    const int nvalid = n - e0 < npt ? n - e0 : npt;
-    if (wave == 0 && lane < 4 * npt) {
-      const bool ok = pe < nvalid;
-      const double wp = ok ? Wwp[e0 + pe] : 0.0, c = ok ? Wc[e0 + pe] : 0.0;
-      const double v = pj ? half + wp : half - wp;
-      const Bracket me = bracket_of(s_mesh, nw, fabs(v), F.geo, F.ga, F.gb);
-      Bracket ot;
-      ot.lo = pair_swap(me.lo);
-      ot.step = pair_swap(me.step);
-      ot.b = pair_swap(me.b);
-      const double vo = pair_swap(v);
-      const Bracket A = pj ? ot : me, B = pj ? me : ot;
-      const double av = pj ? vo : v, bv = pj ? v : vo;
-      // first buffer of the pair: s slot |A|, u slot |B|; lane pj describes the
-      // supports of A's index pj
-      const int ia = A.lo + (pj ? A.step : 0), b0 = B.lo, b1 = B.lo + B.step;
-      const int2 off = make_int2(((b0 > ia ? tri(b0, ia) : tri(ia, b0)) * nw + X) * rowbytes,
-                                 ((b1 > ia ? tri(b1, ia) : tri(ia, b1)) * nw + X) * rowbytes);
-      const double wa = pj ? A.b : 1.0 - A.b;
-      const double w0 = wa * (1.0 - B.b), w1 = wa * B.b;
-      const int mydiag = (b0 == ia ? 1 << (2 * pj) : 0) | (b1 == ia ? 2 << (2 * pj) : 0);
-      const int diag = mydiag | pair_swap(mydiag);
-      // site exchange and t / u sign of the pair's first buffer and of its image
-      const bool ex = (av < 0) != (pp ? bv > 0 : bv < 0), exi = (bv < 0) != (pp ? av > 0 : av < 0);
-      const bool tu = pp ? bv > 0 : bv < 0, tui = pp ? av > 0 : av < 0;
-      // of the point: bit 0 diagonal supports, bit 1 pairs apart, bit 2 not an edge entry
-      int any = (diag ? 1 : 0) | (pp && (av == 0.0 || bv == 0.0) ? 2 : 0) | ((diag && ex == (pp != 0)) || !nedge ? 4 : 0);
-      any |= __shfl_xor(any, 2, 64);
-      any |= __shfl_xor(any, 1, 64);
-      if (ok) {
-        reinterpret_cast<int2 *>(s_off)[lane] = off;
-        s_w[lane] = make_double2(ia < b0 ? -w0 : w0, ia < b1 ? -w1 : w1);
-        if (pj == 0)
-          s_fl[2 * pe + pp] = (ex ? 1 : 0) | (tu ? 2 : 0) | (exi ? 4 : 0) | (tui ? 8 : 0) | diag << 4;
-        if (pp == 0 && pj == 0) s_c[pe] = c;
-        // site-local vertex (u slot exact) with the same brackets: s slot this
-        // lane's argument, t slot the other's; pair 1 with (v, -vo, t): l4 (pj
-        // 0), l5; pair 0 with (v, -vo, -t): l6, l7
-        int lo[4];
-        double lw[4];
-        int fx = 0;
+  // describes the points from e0 on, as many as the entries allow
+  auto describe = [&](int e0) {
+    const double sm = s_mesh[so], tm = s_mesh[X], um = s_mesh[uo];
+    const double half = 0.5 * (sm + (pj ? tm : -tm) + (pp ? -um : um));
+    const bool ok = e0 + pe < n;
+    const double wp = ok ? Wwp[e0 + pe] : 0.0, c = ok ? Wc[e0 + pe] : 0.0;
+    const double v = pj ? half + wp : half - wp;
+    const Bracket me = bracket_of(s_mesh, nw, fabs(v), F.geo, F.ga, F.gb);
+    Bracket ot;
+    ot.lo = pair_swap(me.lo);
+    ot.step = pair_swap(me.step);
+    ot.b = pair_swap(me.b);
+    const double vo = pair_swap(v);
+    const Bracket A = pj ? ot : me, B = pj ? me : ot;
+    const double av = pj ? vo : v, bv = pj ? v : vo;
+    // first buffer of the pair: s slot |A|, u slot |B|; lane pj describes the
+    // supports of A's index pj
+    const int ia = A.lo + (pj ? A.step : 0), b0 = B.lo, b1 = B.lo + B.step;
+    const int2 off = make_int2(((b0 > ia ? tri(b0, ia) : tri(ia, b0)) * nw + X) * rowbytes,
+                               ((b1 > ia ? tri(b1, ia) : tri(ia, b1)) * nw + X) * rowbytes);
+    const double wa = pj ? A.b : 1.0 - A.b;
+    const double w0 = wa * (1.0 - B.b), w1 = wa * B.b;
+    const int mydiag = (b0 == ia ? 1 << (2 * pj) : 0) | (b1 == ia ? 2 << (2 * pj) : 0);
+    const int diag = mydiag | pair_swap(mydiag);
+    // site exchange and t / u sign of the pair's first buffer and of its image
+    const bool ex = (av < 0) != (pp ? bv > 0 : bv < 0), exi = (bv < 0) != (pp ? av > 0 : av < 0);
+    const bool tu = pp ? bv > 0 : bv < 0, tui = pp ? av > 0 : av < 0;
+    // of the point: bit 0 diagonal supports, bit 1 pairs apart, bit 2 not an edge entry
+    int any = (diag ? 1 : 0) | (pp && (av == 0.0 || bv == 0.0) ? 2 : 0) | ((diag && ex == (pp != 0)) || !nedge ? 4 : 0);
+    any |= __shfl_xor(any, 2, 64);
+    any |= __shfl_xor(any, 1, 64);
+    const int mode = any & 2 ? kModeApart : (!(any & 1) ? kModeMain : (any & 4 ? kModeImage : kModeEdge));
+    // entries before the point's among the batch's, and whether they fit
+    const bool twice = mode == kModeImage || mode == kModeApart, mine = pp == 0 && pj == 0 && ok;
+    const unsigned long long two = __ballot(mine && twice), edge = __ballot(mine && mode == kModeEdge);
+    const unsigned long long before = (1ull << (lane & ~3)) - 1;
+    const int f = pe + __popcll(two & before), d = __popcll(edge & before);
+    const int f1 = f + (twice ? 2 : 1), d1 = d + (mode == kModeEdge ? 1 : 0);
+    const bool fits = ok && pe < npt && ((f1 + 1) & ~1) + d1 <= nent;
+    const unsigned long long taken = __ballot(mine && fits);
+    if (!fits) return;
+    if (lane == 63 - __builtin_clzll(taken)) s_head[0] = make_int4(__popcll(taken), f1, d1, 0);
+    reinterpret_cast<int2 *>(s_off)[lane] = off;
+    s_w[lane] = make_double2(ia < b0 ? -w0 : w0, ia < b1 ? -w1 : w1);
+    if (pj == 0) {
+      s_pos[2 * pe + pp] = make_int4((ex ? 1 : 0) | (tu ? 2 : 0) | (exi ? 4 : 0) | (tui ? 8 : 0) | diag << 4,
+                                     full_at(f) + pp * mat, full_at(twice ? f + 1 : nent - 1 - d) + pp * mat, mode);
+      s_c[2 * pe + pp] = pp ? 1.0 : (mode == kModeApart ? 0.5 * c : c);
+    }
+    // site-local vertex (u slot exact) with the same brackets: s slot this
+    // lane's argument, t slot the other's; pair 1 with (v, -vo, t): l4 (pj
+    // 0), l5; pair 0 with (v, -vo, -t): l6, l7
+    int lo[4];
+    double lw[4];
+    int fx = 0;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int is = me.lo + ((q & 1) ? me.step : 0), it = ot.lo + ((q & 2) ? ot.step : 0);
-          lo[q] = ((is > X ? tri(is, X) : tri(X, is)) * nw + it) * rowbytes;
-          lw[q] = ((q & 1) ? me.b : 1.0 - me.b) * ((q & 2) ? ot.b : 1.0 - ot.b);
-          if (is < X) fx |= 4 << q;
-        }
-        const int l = 4 * pe + (pp ? pj : 2 + pj);
-        s_loff[l] = make_int4(lo[0], lo[1], lo[2], lo[3]);
-        s_lw[2 * l] = make_double2(lw[0], lw[1]);
-        s_lw[2 * l + 1] = make_double2(lw[2], lw[3]);
-        const bool lex = pp ? v < 0 : !(v < 0), ltu = pp ? vo > 0 : !(vo > 0);
-        s_lfl[l] = fx | (lex ? 1 : 0) | (ltu ? 2 : 0);
-      }
-      // entries of the points: their positions among the batch's
-      const int mode = any & 2 ? kModeApart : (!(any & 1) ? kModeMain : (any & 4 ? kModeImage : kModeEdge));
-      const bool first = pp == 0 && pj == 0 && ok;
-      const unsigned long long two = __ballot(first && (mode == kModeImage || mode == kModeApart));
-      const unsigned long long edge = __ballot(first && mode == kModeEdge);
-      if (first) {
-        const unsigned long long before = (1ull << lane) - 1;
-        const int f = pe + __popcll(two & before), d = __popcll(edge & before);
-        s_ent[pe] = f | d << 8 | mode << 16;
-        if (pe == nvalid - 1) s_ent[nvalid] = (f + (mode == kModeImage || mode == kModeApart ? 2 : 1)) | (d + (mode == kModeEdge ? 1 : 0)) << 8;
-      }
+    for (int q = 0; q < 4; ++q) {
+      const int is = me.lo + ((q & 1) ? me.step : 0), it = ot.lo + ((q & 2) ? ot.step : 0);
+      lo[q] = ((is > X ? tri(is, X) : tri(X, is)) * nw + it) * rowbytes;
+      lw[q] = ((q & 1) ? me.b : 1.0 - me.b) * ((q & 2) ? ot.b : 1.0 - ot.b);
+      if (is < X) fx |= 4 << q;
     }
-    __syncthreads();
-    // site-local vertices: 8 lanes each, two components per lane
-    for (int q = tid; q < nvalid * 32; q += nt) {
-      const int l = q >> 3, fl = s_lfl[l];
-      const int4 o = s_loff[l];
-      const double2 v0 = buf_load<double2>(rG, o.x + pc * 16), v1 = buf_load<double2>(rG, o.y + pc * 16);
-      const double2 v2 = buf_load<double2>(rG, o.z + pc * 16), v3 = buf_load<double2>(rG, o.w + pc * 16);
-      const double2 wa = s_lw[2 * l], wb = s_lw[2 * l + 1];
-      // getValueLocal (src/TRI/TRIVertexTwoParticle.hpp:300-309): site 0; the
-      // sign of exchanged storage goes by the exchanged components
-      const bool ex = fl & 1;
-      const int nx = ex && kd ? -1 : 0, ny = (ex ? kd : dens) ? -1 : 0;
-      double x = flip_by(wa.x, (fl << 29) & nx) * v0.x, y = flip_by(wa.x, (fl << 29) & ny) * v0.y;
-      x = fma(flip_by(wa.y, (fl << 28) & nx), v1.x, x);
-      y = fma(flip_by(wa.y, (fl << 28) & ny), v1.y, y);
-      x = fma(flip_by(wb.x, (fl << 27) & nx), v2.x, x);
-      y = fma(flip_by(wb.x, (fl << 27) & ny), v2.y, y);
-      x = fma(flip_by(wb.y, (fl << 26) & nx), v3.x, x);
-      y = fma(flip_by(wb.y, (fl << 26) & ny), v3.y, y);
-      const int k = pc >> 1, m = 2 * (pc & 1);
-      s_loc[l * 16 + (ex ? 4 * m + k : 4 * k + m)] = flip_by(x, (fl << 30) & xt);
-      s_loc[l * 16 + (ex ? 4 * (m + 1) + k : 4 * k + m + 1)] = flip_by(y, (fl << 30) & yt);
-    }
-    __syncthreads();
-    for (int pa = 0; pa < nvalid;) {
-      // points pa .. pb whose entries fit the area
-      const int ea = __builtin_amdgcn_readfirstlane(s_ent[pa]);
-      const int fa = ea & 0xff, da = (ea >> 8) & 0xff;
-      int pb = pa + 1, eb = __builtin_amdgcn_readfirstlane(s_ent[pb]);
-      while (pb < nvalid) {
-        const int en = __builtin_amdgcn_readfirstlane(s_ent[pb + 1]);
-        if ((((en & 0xff) - fa + 1) & ~1) + ((en >> 8) & 0xff) - da > nent) break;
-        eb = en;
-        ++pb;
+    const int l = 4 * pe + (pp ? pj : 2 + pj);
+    s_loff[l] = make_int4(lo[0], lo[1], lo[2], lo[3]);
+    s_lw[2 * l] = make_double2(lw[0], lw[1]);
+    s_lw[2 * l + 1] = make_double2(lw[2], lw[3]);
+    const bool lex = pp ? v < 0 : !(v < 0), ltu = pp ? vo > 0 : !(vo > 0);
+    s_lfl[l] = fx | (lex ? 1 : 0) | (ltu ? 2 : 0);
+  };
+  if (wave == 0) describe(0);
+  __syncthreads();
+
+  for (int e0 = 0; e0 < n;) {
+    const int4 head = s_head[0];
+    const int np = __builtin_amdgcn_readfirstlane(head.x);
+    const int nfull = __builtin_amdgcn_readfirstlane(head.y), nedges = __builtin_amdgcn_readfirstlane(head.z);
+    // site-local vertices and their matrices, two points per wave: 8 lanes to
+    // a vertex, two components each; then 16 lanes to a matrix
+    for (int p2 = 2 * wave; p2 < np; p2 += nt / 32) {
+      const int pt = p2 + (lane >> 5);
+      const bool ok = pt < np;
+      if (ok) {
+        const int l = 4 * pt + ((lane >> 3) & 3), fl = s_lfl[l];
+        const int4 o = s_loff[l];
+        const double2 v0 = buf_load<double2>(rG, o.x + pc * 16), v1 = buf_load<double2>(rG, o.y + pc * 16);
+        const double2 v2 = buf_load<double2>(rG, o.z + pc * 16), v3 = buf_load<double2>(rG, o.w + pc * 16);
+        const double2 wa = s_lw[2 * l], wb = s_lw[2 * l + 1];
+        // getValueLocal (src/TRI/TRIVertexTwoParticle.hpp:300-309): site 0; the
+        // sign of exchanged storage goes by the exchanged components
+        const bool ex = fl & 1;
+        const int nx = ex && kd ? -1 : 0, ny = (ex ? kd : dens) ? -1 : 0;
+        double x = flip_by(wa.x, (fl << 29) & nx) * v0.x, y = flip_by(wa.x, (fl << 29) & ny) * v0.y;
+        x = fma(flip_by(wa.y, (fl << 28) & nx), v1.x, x);
+        y = fma(flip_by(wa.y, (fl << 28) & ny), v1.y, y);
+        x = fma(flip_by(wb.x, (fl << 27) & nx), v2.x, x);
+        y = fma(flip_by(wb.x, (fl << 27) & ny), v2.y, y);
+        x = fma(flip_by(wb.y, (fl << 26) & nx), v3.x, x);
+        y = fma(flip_by(wb.y, (fl << 26) & ny), v3.y, y);
+        const int k = pc >> 1, m = 2 * (pc & 1);
+        s_loc[l * 16 + (ex ? 4 * m + k : 4 * k + m)] = flip_by(x, (fl << 30) & xt);
+        s_loc[l * 16 + (ex ? 4 * (m + 1) + k : 4 * k + m + 1)] = flip_by(y, (fl << 30) & yt);
       }
-      const int nfull = (eb & 0xff) - fa, nedges = ((eb >> 8) & 0xff) - da;
-      // bundles into the entries
-      for (int q = tid; q < (pb - pa) * 2 * nch; q += nt) {
-        const int bd = fast_div(q, inv), ch = q - bd * nch;
-        const int pt = pa + (bd >> 1), side = bd & 1, id = 2 * pa + bd;
-        const int4 o = s_off[id];
-        const double2 v0 = buf_load<double2>(rG, o.x + ch * 16), v1 = buf_load<double2>(rG, o.y + ch * 16);
-        const double2 v2 = buf_load<double2>(rG, o.z + ch * 16), v3 = buf_load<double2>(rG, o.w + ch * 16);
-        const int fl = s_fl[id], en = s_ent[pt], mode = en >> 16;
-        const double2 wa = s_w[2 * id], wb = s_w[2 * id + 1];
-        double c = s_c[pt];
-        if (mode == kModeApart) c *= 0.5;
-        if (side) c = 1.0;
-        double x = fabs(wa.x) * v0.x;
-        x = fma(fabs(wa.y), v1.x, x);
-        x = fma(fabs(wb.x), v2.x, x);
-        x = fma(fabs(wb.y), v3.x, x);
-        double y = and_sign(wa.x, mask) * v0.y;
-        y = fma(and_sign(wa.y, mask), v1.y, y);
-        y = fma(and_sign(wb.x, mask), v2.y, y);
-        y = fma(and_sign(wb.y, mask), v3.y, y);
-        x *= c;
-        y *= c;
-        double dg = 0.0;  // l = d component of the diagonal supports
-        if (mode != kModeMain && dens && (fl & 0xf0)) {
-          dg = fl & 16 ? wa.x * v0.y : 0.0;
-          dg = fma(fl & 32 ? wa.y : 0.0, v1.y, dg);
-          dg = fma(fl & 64 ? wb.x : 0.0, v2.y, dg);
-          dg = fma(fl & 128 ? wb.y : 0.0, v3.y, dg);
-          dg *= c;
-          if (mode != kModeApart) y -= dg;
-        }
-        unsigned char *M = area + side * mat;
-        const int *dst = s_dst + 2 * side * nch + ch;
-        auto put = [&](int e, double vx, double vy, bool ex, int tu) {
-          const int d = dst[ex ? nch : 0];
-          unsigned char *E = M + full_at(e);
-          *reinterpret_cast<double *>(E + (d & 0x7fff)) = flip_by(vx, (tu & xt) ^ (d << 16));
-          *reinterpret_cast<double *>(E + ((d >> 16) & 0x7fff)) = flip_by(vy, (tu & yt) ^ d);
-        };
-        const int e = (en & 0xff) - fa;
-        put(e, x, y, fl & 1, fl << 30);
-        if (mode == kModeImage) put(e + 1, 0.0, -dg, fl & 1, fl << 30);
-        if (mode == kModeApart) put(e + 1, x, dens ? fma(2.0, dg, -y) : y, fl & 4, fl << 28);
-        if (mode == kModeEdge && dens) {
-          // row d of X', in the exchanged places, and column d of Y', in the plain ones
-          const int d = dst[side ? 0 : nch];
-          *reinterpret_cast<double *>(M + full_at(nent - 1 - (((en >> 8) & 0xff) - da)) + ((d >> 16) & 0x7fff)) =
-              flip_by(-dg, ((fl << 30) & yt) ^ d);
-        }
-      }
-      // matrices of the site-local vertices: chalice in Y, inverse chalice in X
-      for (int q = tid; q < (pb - pa) * 32; q += nt) {
-        const int pt = pa + (q >> 5), side = (q >> 4) & 1, ij = q & 15;
-        const int en = s_ent[pt], mode = en >> 16;
-        // sides: 1 the chalice of l4, l5 (row i = nu, column j = t), 0 the
-        // inverse chalice of l6, l7 (row r, column ka)
+      wave_lds_fence();
+      if (ok) {
+        // sides: 1 the chalice of l4, l5 (row i = nu, column j = t) in Y, 0 the
+        // inverse chalice of l6, l7 (row r, column ka) in X
+        const int side = (lane >> 4) & 1, ij = lane & 15, i = ij >> 2, j = ij & 3;
+        const int4 ps = s_pos[2 * pt + side];
         const double *la = s_loc + (4 * pt + (side ? 0 : 2)) * 16, *lb = la + 16;
-        const int i = ij >> 2, j = ij & 3;
         const int lab = pauli_label(i) ^ pauli_label(j);
         const int neg = (int)((side ? kChaliceMask : kInverseMask) >> (4 * ij));
         double ka = 0.0, kb = 0.0;
@@ -692,57 +639,105 @@ __global__ __launch_bounds__(512, NG <= 5 ? 4 : 2) void k_tri_t(TriDev F) {
           ka += flip_by(la[o], neg << (31 - k));
           kb += flip_by(lb[o], neg << (31 - k));
         }
-        const double c = side ? 1.0 : s_c[pt];
-        unsigned char *M = area + side * mat + (side ? tri_el(L, i, j) : tri_el(L, j, i));
-        const int e = (en & 0xff) - fa;
-        auto put = [&](int at, double v) { *reinterpret_cast<double *>(M + at) = c * v; };
-        if (mode == kModeApart) {
-          // X carries half the weight here
-          put(full_at(e), side ? 2.0 * ka : ka);
-          put(full_at(e + 1), side ? 2.0 * kb : kb);
-        } else {
-          const double kbd = flip(kb, (side ? i : j) == 3);
-          put(full_at(e), ka + kbd);
-          if (mode == kModeImage) put(full_at(e + 1), kbd - ka);
-          if (mode == kModeEdge) put(full_at(nent - 1 - (((en >> 8) & 0xff) - da)), kbd - ka);
-        }
+        const double c = s_c[2 * pt + side];
+        const double kbd = flip(kb, (side ? i : j) == 3);
+        const bool apart = ps.w == kModeApart;  // X carries half the weight there
+        unsigned char *M = area + (side ? tri_el(L, L, i, j) : tri_el(L, L, j, i));
+        *reinterpret_cast<double *>(M + ps.y) = c * (apart ? 2.0 * ka : ka + kbd);
+        if (ps.w != kModeMain) *reinterpret_cast<double *>(M + ps.z) = c * (apart ? 2.0 * kb : kbd - ka);
       }
-      // an odd number of entries: nothing from the other half of the last pair
-      if (nfull & 1)
-        for (int q = tid; q < 16 * (L + 1); q += nt)
-          *reinterpret_cast<double *>(area + full_at(nfull) + q * 16) = 0.0;
-      __syncthreads();
-      for (int p = 0; p < nfull; p += 2) {
-        const unsigned char *E = area + p * mat;
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-          const double2 a = *reinterpret_cast<const double2 *>(E + (pk[g][0] & 0xffff));
-          const double2 b0 = *reinterpret_cast<const double2 *>(E + ((unsigned)pk[g][0] >> 16));
-          const double2 b1 = *reinterpret_cast<const double2 *>(E + (pk[g][1] & 0xffff));
-          const double2 b2 = *reinterpret_cast<const double2 *>(E + ((unsigned)pk[g][1] >> 16));
-          const double2 b3 = *reinterpret_cast<const double2 *>(E + pk[g][2]);
-          C[g][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.x, b0.x, C[g][0], 0, 0, 0);
-          C[g][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.x, b1.x, C[g][1], 0, 0, 0);
-          C[g][2] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.x, b2.x, C[g][2], 0, 0, 0);
-          C[g][3] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.x, b3.x, C[g][3], 0, 0, 0);
-          C[g][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.y, b0.y, C[g][0], 0, 0, 0);
-          C[g][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.y, b1.y, C[g][1], 0, 0, 0);
-          C[g][2] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.y, b2.y, C[g][2], 0, 0, 0);
-          C[g][3] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.y, b3.y, C[g][3], 0, 0, 0);
-        }
-      }
-      for (int e = 0; e < nedges; ++e) {
-        const unsigned char *E = area + full_at(nent - 1 - e);
-#pragma unroll
-        for (int i = 0; i < kTriEdges; ++i)
-          if (i < nedge)
-            CE[i] = __builtin_amdgcn_mfma_f64_4x4x4f64(*reinterpret_cast<const double *>(E + (pe_[i] & 0xffff)),
-                                                       *reinterpret_cast<const double *>(E + ((unsigned)pe_[i] >> 16)),
-                                                       CE[i], 0, 0, 0);
-      }
-      __syncthreads();
-      pa = pb;
     }
+    // bundles into the entries
+    for (int q = tid; q < np * 2 * nch; q += nt) {
+      const int id = fast_div(q, inv), ch = q - id * nch;
+      const int4 o = s_off[id];
+      const int *dst = s_dst + ((id & 1) ? 2 * nch : 0) + ch;
+      const double2 v0 = buf_load<double2>(rG, o.x + ch * 16), v1 = buf_load<double2>(rG, o.y + ch * 16);
+      const double2 v2 = buf_load<double2>(rG, o.z + ch * 16), v3 = buf_load<double2>(rG, o.w + ch * 16);
+      const int4 ps = s_pos[id];
+      const int fl = ps.x, mode = ps.w;
+      const double2 wa = s_w[2 * id], wb = s_w[2 * id + 1];
+      const double c = s_c[id];
+      double x = fabs(wa.x) * v0.x;
+      x = fma(fabs(wa.y), v1.x, x);
+      x = fma(fabs(wb.x), v2.x, x);
+      x = fma(fabs(wb.y), v3.x, x);
+      double y = and_sign(wa.x, mask) * v0.y;
+      y = fma(and_sign(wa.y, mask), v1.y, y);
+      y = fma(and_sign(wb.x, mask), v2.y, y);
+      y = fma(and_sign(wb.y, mask), v3.y, y);
+      x *= c;
+      y *= c;
+      const int d = dst[(fl & 1) ? nch : 0];
+      if (mode == kModeMain) {
+        unsigned char *E = area + ps.y;
+        *reinterpret_cast<double *>(E + (d & 0x7fff)) = flip_by(x, ((fl << 30) & xt) ^ (d << 16));
+        *reinterpret_cast<double *>(E + ((d >> 16) & 0x7fff)) = flip_by(y, ((fl << 30) & yt) ^ d);
+      } else {
+        double dg = 0.0;  // l = d component of the diagonal supports
+        if (dens) {
+          dg = fl & 16 ? wa.x * v0.y : 0.0;
+          dg = fma(fl & 32 ? wa.y : 0.0, v1.y, dg);
+          dg = fma(fl & 64 ? wb.x : 0.0, v2.y, dg);
+          dg = fma(fl & 128 ? wb.y : 0.0, v3.y, dg);
+          dg *= c;
+        }
+        unsigned char *E = area + ps.y, *E2 = area + ps.z;
+        *reinterpret_cast<double *>(E + (d & 0x7fff)) = flip_by(x, ((fl << 30) & xt) ^ (d << 16));
+        *reinterpret_cast<double *>(E + ((d >> 16) & 0x7fff)) =
+            flip_by(mode == kModeApart ? y : y - dg, ((fl << 30) & yt) ^ d);
+        if (mode == kModeEdge) {
+          // row d of X', in the exchanged places, and column d of Y', in the plain ones
+          const int de = dst[(id & 1) ? 0 : nch];
+          if (dens) *reinterpret_cast<double *>(E2 + ((de >> 16) & 0x7fff)) = flip_by(-dg, ((fl << 30) & yt) ^ de);
+        } else {
+          const int di = mode == kModeApart ? dst[(fl & 4) ? nch : 0] : d, ti = mode == kModeApart ? fl << 28 : fl << 30;
+          const double x2 = mode == kModeApart ? x : 0.0;
+          const double y2 = mode == kModeApart ? (dens ? fma(2.0, dg, -y) : y) : -dg;
+          *reinterpret_cast<double *>(E2 + (di & 0x7fff)) = flip_by(x2, (ti & xt) ^ (di << 16));
+          *reinterpret_cast<double *>(E2 + ((di >> 16) & 0x7fff)) = flip_by(y2, (ti & yt) ^ di);
+        }
+      }
+    }
+    // an odd number of entries: nothing from the other half of the last pair
+    if (nfull & 1)
+      for (int q = tid; q < mat / 16; q += nt) *reinterpret_cast<double *>(area + full_at(nfull) + q * 16) = 0.0;
+    __syncthreads();
+    e0 += np;
+    if (wave == 0 && e0 < n) describe(e0);  // (the products do not read the descriptors)
+    for (int p = 0; p < nfull; p += 2) {
+      const unsigned char *E = area + p * mat;
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        // (unpacked here: the compiler would otherwise keep the positions apart)
+        asm volatile("" : "+v"(pk[g][0]), "+v"(pk[g][1]), "+v"(pk[g][2]));
+        const double2 a = *reinterpret_cast<const double2 *>(E + (pk[g][0] & 0xffff));
+        const double2 b0 = *reinterpret_cast<const double2 *>(E + ((unsigned)pk[g][0] >> 16));
+        const double2 b1 = *reinterpret_cast<const double2 *>(E + (pk[g][1] & 0xffff));
+        const double2 b2 = *reinterpret_cast<const double2 *>(E + ((unsigned)pk[g][1] >> 16));
+        const double2 b3 = *reinterpret_cast<const double2 *>(E + pk[g][2]);
+        C[g][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.x, b0.x, C[g][0], 0, 0, 0);
+        C[g][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.x, b1.x, C[g][1], 0, 0, 0);
+        C[g][2] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.x, b2.x, C[g][2], 0, 0, 0);
+        C[g][3] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.x, b3.x, C[g][3], 0, 0, 0);
+        C[g][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.y, b0.y, C[g][0], 0, 0, 0);
+        C[g][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.y, b1.y, C[g][1], 0, 0, 0);
+        C[g][2] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.y, b2.y, C[g][2], 0, 0, 0);
+        C[g][3] = __builtin_amdgcn_mfma_f64_4x4x4f64(a.y, b3.y, C[g][3], 0, 0, 0);
+      }
+    }
+    if (nedges)
+#pragma unroll
+      for (int i = 0; i < kTriEdges; ++i) {
+        if (i >= nedge) break;
+        const unsigned q = F.t_edge_ops[(wave * nedge + i) * 64 + lane];
+        for (int e = 0; e < nedges; ++e) {
+          const unsigned char *E = area + full_at(nent - 1 - e);
+          CE[i] = __builtin_amdgcn_mfma_f64_4x4x4f64(*reinterpret_cast<const double *>(E + (q & 0xffff)),
+                                                     *reinterpret_cast<const double *>(E + (q >> 16)), CE[i], 0, 0, 0);
+        }
+      }
+    __syncthreads();
   }
 
   // overlap lists, S and U values, prefactor 1/(2 pi)
@@ -827,7 +822,7 @@ inline TriPlan build_tri_plan(const sp_tri_problem *p) {
         for (int h = 0; h < 2; ++h) {
           const int k = (ch & 7) >> 1, l = 2 * (ch & 1) + h;
           const int s1 = ex ? inv[l] : k, s2 = ex ? inv[k] : l;
-          const unsigned at = side ? tri_el(site, s1, s2) : tri_el(site, s2, s1);
+          const unsigned at = side ? tri_el(L, site, s1, s2) : tri_el(L, site, s2, s1);
           code |= (at | (hat_sign(s1, s2) < 0 ? 0x8000u : 0u)) << (16 * h);
         }
         r.dst[(2 * side + ex) * 8 * L + ch] = (int)code;
@@ -875,6 +870,12 @@ inline TriPlan build_tri_plan(const sp_tri_problem *p) {
     }
   const int groups = (nruns + 3) / 4;
   int waves = 1;
+  // More waves per item shorten the phases between barriers: up to four while a
+  // wave has more than three groups (honeycomb r3, 5 sites, at cutoff 0.02: 0.171 ->
+  // 0.145 ms, kagome r3, 8 sites: 2.17 -> 2.01 ms; fewer groups gain nothing:
+  // kagome r2, 4 sites, 2.14 ms, 2.20 with two waves).  More than five groups do not fit the
+  // registers of four waves per SIMD; then eight waves.
+  while (waves < 4 && (groups + waves - 1) / waves > 3) waves *= 2;
   while (waves < 8 && (groups + waves - 1) / waves > 5) waves *= 2;
   const int ng = (groups + waves - 1) / waves, nt = 64 * waves;
   if (ng > kTriMaxGroups) return r;
@@ -908,7 +909,10 @@ inline TriPlan build_tri_plan(const sp_tri_problem *p) {
           for (int o = 0; o < b; ++o) {
             const Product *x = u.x[perm[z]], *y = order[4 * g + o].x[z];
             if (x && y)
-              for (int k = 0; k < 4; ++k) c += ((x->q[k] + x->right) & 3) == ((y->q[k] + y->right) & 3);
+              for (int k = 0; k < 4; ++k) {
+                const int S = tri_sites(L);
+                c += ((x->q[k] * S + x->right) & 3) == ((y->q[k] * S + y->right) & 3);
+              }
           }
         if (c < cost) {
           cost = c;
@@ -929,8 +933,8 @@ inline TriPlan build_tri_plan(const sp_tri_problem *p) {
       const int k = lane >> 4, b = (lane >> 2) & 3, i = lane & 3;
       const Run &u = order[4 * g + b];
       int o[4];
-      for (int z = 0; z < 4; ++z) o[z] = right0 + (u.x[z] ? tri_el(u.x[z]->right, u.x[z]->q[k], i) : tri_el(L, k, i));
-      r.ops[64 * (size_t)g + lane] = make_int4(tri_el(u.left, k, i) | o[0] << 16, o[1] | o[2] << 16, o[3], 0);
+      for (int z = 0; z < 4; ++z) o[z] = right0 + (u.x[z] ? tri_el(L, u.x[z]->right, u.x[z]->q[k], i) : tri_el(L, L, k, i));
+      r.ops[64 * (size_t)g + lane] = make_int4(tri_el(L, u.left, k, i) | o[0] << 16, o[1] | o[2] << 16, o[3], 0);
     }
   }
   // edge entries: blocks of four left and four right sites, row d of X' and
@@ -965,8 +969,8 @@ inline TriPlan build_tri_plan(const sp_tri_problem *p) {
         const Block x = 4 * z + ((lane >> 2) & 3) < (int)blocks.size() ? blocks[4 * z + ((lane >> 2) & 3)]
                                                                      : Block{-1, -1, {0, 1, 2, 3}};
         const int l = 4 * x.left + i, rt = 4 * x.right + i;
-        const int a = x.left < 0 || l >= L ? tri_el(L, k, i) : tri_el(l, k, 3);
-        const int b = x.right < 0 || rt >= L ? tri_el(L, x.q[k], i) : tri_el(rt, x.q[k], 3);
+        const int a = x.left < 0 || l >= L ? tri_el(L, L, k, i) : tri_el(L, l, k, 3);
+        const int b = x.right < 0 || rt >= L ? tri_el(L, L, x.q[k], i) : tri_el(L, rt, x.q[k], 3);
         r.edge_ops[64 * (size_t)z + lane] = a | (right0 + b) << 16;
       }
   }
