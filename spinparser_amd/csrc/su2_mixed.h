@@ -15,7 +15,9 @@
 // What bounds it: the gathers (8 bytes a lane) and the vector instructions about
 // equally.  Simple cubic J1-J2, 48 frequencies, 23 sites, mean over the cutoffs
 // 100 to 3: 1095 -> 494 us per evaluation (k_su32 238, k_t32 256) against one
-// 256-thread workgroup per item with a producer wave.
+// 256-thread workgroup per item with a producer wave.  Kagome, 26 sites, bonds
+// not equivalent to their reverse, 48 frequencies: 950 -> 590 us at cutoff 20,
+// 2336 -> 1859 us at 0.3.
 #pragma once
 
 // spin and density of an access buffer from its supports v in the order (lo lo),
@@ -390,29 +392,43 @@ __global__ __launch_bounds__(64 * kRhsWaves, FT + HT == 1 ? 4 : 3) void k_t32(co
         __builtin_amdgcn_sched_barrier(0);
         const float c = (float)s_c[e];
         Bundle32 first[2], second[2];
+        // the pair's first buffer: the interpolations in the other order, the
+        // density sign of the other exchange
+        auto image = [&](int p, const float4 &w, const float2 (&x)[4]) {
+          const int2 g = s_fl[2 * e + p];
+          const float m0 = (g.x & 4) ? w.x : -w.x, m1 = (g.x & 8) ? w.y : -w.y;
+          const float m2 = (g.y & 4) ? w.z : -w.z, m3 = (g.y & 8) ? w.w : -w.w;
+          return Bundle32{spin_chain(m0, m2, m1, m3, x[0], x[2], x[1], x[3]),
+                          density_chain(m0, m2, m1, m3, x[0], x[2], x[1], x[3])};
+        };
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
           const float4 w = s_w[2 * e + p];
-          const int2 g = s_fl[2 * e + p];
           second[p] = Bundle32{spin_chain(w.x, w.y, w.z, w.w, v[p][0], v[p][1], v[p][2], v[p][3]),
                                density_chain(w.x, w.y, w.z, w.w, v[p][0], v[p][1], v[p][2], v[p][3])};
-          // the first buffer: the interpolations in the other order, the density
-          // sign of the other exchange
-          const float m0 = (g.x & 4) ? w.x : -w.x, m1 = (g.x & 8) ? w.y : -w.y;
-          const float m2 = (g.y & 4) ? w.z : -w.z, m3 = (g.y & 8) ? w.w : -w.w;
+          first[p] = image(p, w, v[p]);
           if (ASYM) {
-            if (g.x & 2) {
-              // an argument of exactly zero: it exchanges the sites the other way
+            settle(second[p].s, second[p].d);
+            settle(first[p].s, first[p].d);
+          }
+        }
+        if (ASYM) {
+          // an argument of exactly zero: the first buffer exchanges the sites
+          // the other way.  After the rest and as a branch of the whole wave: a
+          // lane's own branch that replaced supports still in use kept both
+          // gathers of every tile in registers (157 spilled at 26 sites)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            const int gx = s_fl[2 * e + p].x;
+            if (__any(gx & 2)) {
               const int4 o = s_off[2 * e + p];
-              const unsigned site = (g.x & 1) ? sr[k] : sx[k];
-              v[p][0] = buf_load<float2>(rG, o.x + site);
-              v[p][1] = buf_load<float2>(rG, o.y + site);
-              v[p][2] = buf_load<float2>(rG, o.z + site);
-              v[p][3] = buf_load<float2>(rG, o.w + site);
+              const unsigned site = (gx & 1) ? sr[k] : sx[k];
+              const float2 x[4] = {buf_load<float2>(rG, o.x + site), buf_load<float2>(rG, o.y + site),
+                                   buf_load<float2>(rG, o.z + site), buf_load<float2>(rG, o.w + site)};
+              const Bundle32 f = image(p, s_w[2 * e + p], x);
+              if (gx & 2) first[p] = f;
             }
           }
-          first[p] = Bundle32{spin_chain(m0, m2, m1, m3, v[p][0], v[p][2], v[p][1], v[p][3]),
-                              density_chain(m0, m2, m1, m3, v[p][0], v[p][2], v[p][1], v[p][3])};
         }
         const float4 l0 = s_loc[2 * e], l1 = s_loc[2 * e + 1];
         rs[k] += (double)(c * fmaf(l0.x, first[0].s, fmaf(l0.z, first[1].s, fmaf(l1.x, second[0].s, l1.z * second[1].s))));

@@ -71,7 +71,7 @@ __device__ __forceinline__ void reread_lds() {
 // computes a and b here: the compiler would otherwise sink their sums to the
 // last use, across the branches between, and hold the gathered supports until
 // then (more than 100 spilled registers)
-__device__ __forceinline__ void settle(double &a, double &b) { asm volatile("" : "+v"(a), "+v"(b)); }
+template <class T> __device__ __forceinline__ void settle(T &a, T &b) { asm volatile("" : "+v"(a), "+v"(b)); }
 
 struct Bracket {
   int lo, step;  // support indices lo and lo + step (step 0: clamped, weight 0)
