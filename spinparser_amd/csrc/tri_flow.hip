@@ -206,6 +206,28 @@ __device__ __forceinline__ void apply_table(double (&acc)[16], const double (&x)
   apply_terms<KIND>(acc, x, y, std::make_integer_sequence<int, 256>{});
 }
 
+// the same with the sixteen terms of an output summed before they are added: one
+// rounding of the accumulator per product
+template <int KIND, int O, int... K>
+__device__ __forceinline__ void add_output(double (&acc)[16], const double (&x)[16], const double (&y)[16],
+                                           std::integer_sequence<int, K...>) {
+  double t[16] = {};
+  t[O] = kTab[KIND].t[16 * O].c > 0 ? x[kTab[KIND].t[16 * O].a] * y[kTab[KIND].t[16 * O].b]
+                                    : -x[kTab[KIND].t[16 * O].a] * y[kTab[KIND].t[16 * O].b];
+  (term<KIND, 16 * O + 1 + K>(t, x, y), ...);
+  acc[O] += t[O];
+}
+template <int KIND, int... O>
+__device__ __forceinline__ void add_outputs(double (&acc)[16], const double (&x)[16], const double (&y)[16],
+                                            std::integer_sequence<int, O...>) {
+  static_assert(((kTab[KIND].t[16 * O].o == O && kTab[KIND].t[16 * O + 15].o == O) && ...), "terms by output");
+  (add_output<KIND, O>(acc, x, y, std::make_integer_sequence<int, 15>{}), ...);
+}
+template <int KIND>
+__device__ __forceinline__ void add_table(double (&acc)[16], const double (&x)[16], const double (&y)[16]) {
+  add_outputs<KIND>(acc, x, y, std::make_integer_sequence<int, 16>{});
+}
+
 __device__ __forceinline__ int zeta(int s) { return s <= 2 ? -1 : 1; }
 
 __device__ __forceinline__ double pick3(double u0, double u1, double u2, int i) {

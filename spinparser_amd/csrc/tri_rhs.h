@@ -13,9 +13,14 @@
 //    This needs site_rid and site_perm to be identities and inv_rid a
 //    permutation, which every lattice of the factory has; other tables, and
 //    lattices of more than kMaxTriRhsL sites, run the general kernel.
-//  * With e = -i sigma the components are those of an element of H (x) H, the
-//    real 4 x 4 matrices: S and U products of 256 terms become 4 x 4 matrix
-//    products of 64 (k_tri_su), and the U integrals are the S ones with the
+//  * S and U add the 256 products of the components of two bundles, each output's
+//    sixteen terms summed first (k_tri_su).  As elements of H (x) H, 4 x 4 real
+//    matrices, the bundles would need 64 products, but sums and differences of
+//    components mix their sizes: on flowed kagome-DM states the error of the
+//    Dzyaloshinskii-Moriya components (1e-5 to 4e-2 of the others) was 1.3 to 2
+//    times that of sums over their own terms, and components 1e-8 as large as
+//    others had 7e-10 of their size.  The matrices were faster (kagome-DM r5 at
+//    cutoff 0.02: k_tri_su 8.2 instead of 9.8 ms).  The U integrals are the S ones with the
 //    sign of the l = d components changed in the buffers and in the result.
 //  * With s(x, y) = -1 for x a spin and y the density, A(r, m) s(r, m) are 4 x 4
 //    matrices whose plain product is the lattice bubble (times s(r, t)), and
@@ -26,9 +31,9 @@
 //    over the points before the overlap lists are applied (k_tri_t).
 //
 // Kagome with DM exchange, 19 sites, 48 frequencies, against one workgroup per
-// item that forms all terms point by point: 12.9 -> 5.2 ms at cutoff 20, 46.3 ->
-// 14.1 ms at 0.7, 81.9 -> 24.1 ms at 0.02 (k_tri_su 8.2 ms, its gathers 70 % of
-// the cache's rate and its vector instructions 64 %; k_tri_t 15.8 ms, which
+// item that forms all terms point by point: 12.9 -> 5.5 ms at cutoff 20, 46.3 ->
+// 15.0 ms at 0.7, 81.9 -> 25.9 ms at 0.02 (k_tri_su 9.8 ms, bound by its gathers
+// and its vector instructions about equally; k_tri_t 15.8 ms, which
 // alternates between gathers, 11 ms by themselves, and matrix products, 13 ms by
 // themselves: the descriptors of the next points are formed beside the products).
 #pragma once
@@ -41,64 +46,6 @@ constexpr int kTriMaxGroups = 10;  // per wave, of at most eight waves
 // label of a component in the group the Pauli products follow: d 0, x 1, y 2, z 3
 constexpr int pauli_label(int k) { return (k + 1) & 3; }
 constexpr int pauli_comp(int label) { return (label + 3) & 3; }
-// sign of e_a e_b (quaternion units; the product is e_(a ^ b))
-constexpr int quat_sign(int a, int b) {
-  if (a == 0 || b == 0) return 1;
-  if (a == b) return -1;
-  return (b - a == 1 || b - a == -2) ? 1 : -1;
-}
-// entry (i, i ^ k ^ l) of the matrix of component c = (k, l): v -> e_k v conj(e_l),
-// negated for all components but the density-density one (sigma = i e)
-constexpr int quat_entry(int c, int i) {
-  const int k = pauli_label(c / 4), l = pauli_label(c % 4), j = i ^ k ^ l;
-  int sg = (k == 0 && l == 0) ? 1 : -1;
-  sg *= l == 0 ? 1 : -1;                      // conj(e_l)
-  sg *= quat_sign(j, l) * quat_sign(k, j ^ l);  // e_k (e_j e_l)
-  return sg;
-}
-constexpr unsigned long long quat_mask() {
-  unsigned long long m = 0;
-  for (int c = 0; c < 16; ++c)
-    for (int i = 0; i < 4; ++i)
-      if (quat_entry(c, i) < 0) m |= 1ull << (c * 4 + i);
-  return m;
-}
-constexpr unsigned long long kQuatMask = quat_mask();
-
-// the four entries (i, i ^ D) from the four components (k, l) with k ^ l = D
-template <int D, int I>
-__device__ __forceinline__ double quat_out(const double (&t)[2], const double (&w)[2]) {
-  constexpr int s0 = quat_entry(4 * pauli_comp(0) + pauli_comp(D), I), s1 = quat_entry(4 * pauli_comp(1) + pauli_comp(1 ^ D), I);
-  constexpr int s2 = quat_entry(4 * pauli_comp(2) + pauli_comp(2 ^ D), I), s3 = quat_entry(4 * pauli_comp(3) + pauli_comp(3 ^ D), I);
-  const double p = t[s0 == s1 ? 0 : 1], q = w[s2 == s3 ? 0 : 1];
-  return (s0 > 0 ? p : -p) + (s2 > 0 ? q : -q);
-}
-// v(c): component c
-template <int D, class V> __device__ __forceinline__ void quat_part(double (&m)[16], V v) {
-  const double a = v(4 * pauli_comp(0) + pauli_comp(D)), b = v(4 * pauli_comp(1) + pauli_comp(1 ^ D));
-  const double c = v(4 * pauli_comp(2) + pauli_comp(2 ^ D)), d = v(4 * pauli_comp(3) + pauli_comp(3 ^ D));
-  const double t[2] = {a + b, a - b}, w[2] = {c + d, c - d};
-  m[D] = quat_out<D, 0>(t, w);
-  m[4 + (1 ^ D)] = quat_out<D, 1>(t, w);
-  m[8 + (2 ^ D)] = quat_out<D, 2>(t, w);
-  m[12 + (3 ^ D)] = quat_out<D, 3>(t, w);
-}
-template <class V> __device__ __forceinline__ void quat_matrix(double (&m)[16], V v) {
-  quat_part<0>(m, v);
-  quat_part<1>(m, v);
-  quat_part<2>(m, v);
-  quat_part<3>(m, v);
-}
-// acc += y x
-__device__ __forceinline__ void add_product(double (&acc)[16], const double (&y)[16], const double (&x)[16]) {
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[4 * i + j] = fma(y[4 * i + k], x[4 * k + j], acc[4 * i + j]);
-}
-
 __device__ __forceinline__ double flip(double v, bool neg) { return neg ? -v : v; }
 // v with the sign bit changed by bit 31 of s
 __device__ __forceinline__ double flip_by(double v, int s) {
@@ -271,7 +218,7 @@ __global__ __launch_bounds__(64 * kRhsWaves, 2) void k_tri_su(TriDev F, long lon
       }
     }
   };
-  // matrix of a buffer's bundle at the lane's site
+  // a buffer's bundle at the lane's site, times c
   auto bundle = [&](const double *raw, bool ex, double c, double (&m)[16]) {
     // (positions formed here, each time: kept in registers over the loops they
     // would take more than 100)
@@ -281,9 +228,8 @@ __global__ __launch_bounds__(64 * kRhsWaves, 2) void k_tri_su(TriDev F, long lon
     const double *b = raw + at;
     const int A[4] = {ex ? q0 : 0, ex ? q1 : 4, ex ? q2 : 8, ex ? 3 : 12};
     const int B[4] = {ex ? 4 * q0 : 0, ex ? 4 * q1 : 1, ex ? 4 * q2 : 2, ex ? 12 : 3};
-    quat_matrix(m, [&](int k) { return b[A[k >> 2] + B[k & 3]]; });
 #pragma unroll
-    for (int k = 0; k < 16; ++k) m[k] *= c;
+    for (int k = 0; k < 16; ++k) m[k] = c * b[A[k >> 2] + B[k & 3]];
   };
 
   double wp_next = pe < n ? Wwp[pe] : 0.0, c_next = pe < n ? Wc[pe] : 0.0;
@@ -346,22 +292,22 @@ __global__ __launch_bounds__(64 * kRhsWaves, 2) void k_tri_su(TriDev F, long lon
         double x[16];
         if (want & 1) {
           bundle(s_v, f.x & 2, 1.0, x);
-          add_product(r1, y3, x);
+          add_table<0>(r1, x, y3);
           bundle(s_v + sh.raw, f.y & 2, 1.0, x);
-          add_product(r1, y2, x);
+          add_table<0>(r1, x, y2);
         }
         if (want & 2) {
           bundle(s_v, f.x & 1, 1.0, x);
-          add_product(r2, y2, x);
+          add_table<0>(r2, x, y2);
           bundle(s_v + sh.raw, f.y & 1, 1.0, x);
-          add_product(r2, y3, x);
+          add_table<0>(r2, x, y3);
         }
         wave_lds_fence();
       }
     }
   }
 
-  // sum over the slots, back to components, one addition to each value of the
+  // sum over the slots, one addition to each value of the
   // item (zeroed before; two additions in all, so their order does not matter)
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
@@ -375,16 +321,9 @@ __global__ __launch_bounds__(64 * kRhsWaves, 2) void k_tri_su(TriDev F, long lon
     const bool urule = un.u_rule(r);
     double *out = F.dG + (size_t)un.item(r, nw) * L * 16;
     for (int q = lane; q < 16 * L; q += 64) {
-      const int st = q >> 4, c = q & 15;
-      const int kl = pauli_label(c >> 2) ^ pauli_label(c & 3);
       double v = 0.0;
-      for (int z = 0; z < sh.slots; ++z) {
-        const double *m = s_v + (z * L + st) * kTriRaw;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v += flip(m[4 * i + (i ^ kl)], (kQuatMask >> (4 * c + i)) & 1);
-      }
-      v *= 0.25;
-      unsafeAtomicAdd(out + q, (urule && (c & 3) == 3) ? -v : v);
+      for (int z = 0; z < sh.slots; ++z) v += s_v[(z * L + (q >> 4)) * kTriRaw + (q & 15)];
+      unsafeAtomicAdd(out + q, (urule && (q & 3) == 3) ? -v : v);
     }
   }
 }
