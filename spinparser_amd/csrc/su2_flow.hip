@@ -1584,22 +1584,22 @@ int sp_ctx_create(const sp_su2_problem *p, sp_ctx **out) {
     SP_HIP(hipMemcpy(oidx, idx.data(), (size_t)O * 2, hipMemcpyHostToDevice));
   }
   if (f.L <= kMaxRhsL) {
-    LanePlan plan;
-    try { build_overlap_plan(plan, f.L, p->ovl_off, p->ovl_rid1, p->ovl_rid2); } catch (...) { return fail(ctx, SP_ENOMEM, "host buffer"); }
     // one table: lane_of (L + 1), count (64), entries (16-byte aligned)
-    const size_t head = (plan.lane_of.size() + plan.count.size() + 3) & ~size_t(3);
+    LanePlan plan;
     std::vector<unsigned> table;
+    size_t head = 0;
     try {
-      table.assign(plan.lane_of.begin(), plan.lane_of.end());
-      table.insert(table.end(), plan.count.begin(), plan.count.end());
-      table.resize(head, 0);
-      table.insert(table.end(), plan.ent.begin(), plan.ent.end());
+      build_overlap_plan(plan, f.L, p->ovl_off, p->ovl_rid1, p->ovl_rid2);
+      head = ((size_t)f.L + 1 + plan.lanes + 3) & ~size_t(3);
+      table.assign(head + plan.entries(), 0);
     } catch (...) { return fail(ctx, SP_ENOMEM, "host buffer"); }
+    std::copy_n(plan.lane_of.begin(), f.L + 1, table.begin());
+    plan.store(table.data() + head, reinterpret_cast<int *>(table.data()) + f.L + 1);
     unsigned *tab = nullptr;
     if ((rc = dalloc(ctx, &tab, table.size()))) return rc;
     SP_HIP(hipMemcpy(tab, table.data(), table.size() * 4, hipMemcpyHostToDevice));
     const unsigned *ent = tab + head;
-    const int *lane = reinterpret_cast<const int *>(tab), *count = lane + plan.lane_of.size();
+    const int *lane = reinterpret_cast<const int *>(tab), *count = lane + f.L + 1;
     f.plan_ent = ent;
     f.plan_lane = lane;
     f.plan_count = count;
@@ -2050,7 +2050,9 @@ constexpr int kNoAllocDevices = 64;
 std::mutex g_noalloc_mu;
 unsigned char *g_noalloc_ptr[kNoAllocDevices] = {};  // device address of scratch, per device
 int g_noalloc_lds[kNoAllocDevices] = {};            // LDS limit per workgroup, per device
-LanePlan g_noalloc_overlap;                         // keeps its host buffers from call to call
+// overlap plan of a call; the general kernel's 10 bytes per overlap entry bound their number
+using NoAllocOverlap = LanePlanOf<FixedPlan<SP_NOALLOC_SCRATCH_BYTES / 10, kMaxRhsL * kMaxRhsL, kMaxRhsL>>;
+NoAllocOverlap g_noalloc_overlap;
 unsigned char g_noalloc_image[SP_NOALLOC_SCRATCH_BYTES];  // host image of the scratch contents
 
 struct NoAllocPlan {
@@ -2059,7 +2061,7 @@ struct NoAllocPlan {
 
 // contents of the scratch for the general dGamma kernel (wave null; its size
 // is what the documented limit is held against) or for the wave kernels
-NoAllocPlan noalloc_plan(const sp_su2_problem *p, const LanePlan *wave) {
+NoAllocPlan noalloc_plan(const sp_su2_problem *p, const NoAllocOverlap *wave) {
   NoAllocPlan q{};
   size_t o = 0;
   auto take = [&](size_t bytes) {
@@ -2076,9 +2078,9 @@ NoAllocPlan noalloc_plan(const sp_su2_problem *p, const LanePlan *wave) {
   q.inv = take((size_t)p->L * 4);
   q.ooff = take(((size_t)p->L + 1) * 4);
   if (wave) {
-    q.pent = take(wave->ent.size() * 4);
-    q.plane = take(wave->lane_of.size() * 4);
-    q.pcount = take(wave->count.size() * 4);
+    q.pent = take(wave->entries() * 4);
+    q.plane = take(((size_t)p->L + 1) * 4);
+    q.pcount = take((size_t)wave->lanes * 4);
   } else {
     q.o1 = take(O * 4);
     q.o2 = take(O * 4);
@@ -2158,7 +2160,7 @@ extern "C" int sp_compute_step_noalloc(const sp_su2_problem *p, double cutoff, c
   if (lds > (size_t)max_lds) return SP_EARG;
   // the wave kernels add to d_dv4 with FP64 atomics of the memory side, which
   // ordinary device memory takes; any other buffer runs the general kernel
-  LanePlan &plan = g_noalloc_overlap;
+  NoAllocOverlap &plan = g_noalloc_overlap;
   bool wave = false;
   if (f.L <= kMaxRhsL) {
     hipPointerAttribute_t at{};
@@ -2166,7 +2168,10 @@ extern "C" int sp_compute_step_noalloc(const sp_su2_problem *p, double cutoff, c
     else (void)hipGetLastError();
   }
   if (wave) {
-    try { build_overlap_plan(plan, f.L, p->ovl_off, p->ovl_rid1, p->ovl_rid2); } catch (...) { return SP_ENOMEM; }
+    // (before the wait below, beside an earlier call's kernels; by itself 0.6 us
+    // for 226 overlap entries, 4 us for 1,488, 15 us for 8,311 on a host core;
+    // merging on vectors, with divisions per entry, took twice that)
+    build_overlap_plan(plan, f.L, p->ovl_off, p->ovl_rid1, p->ovl_rid2);
     const NoAllocPlan qw = noalloc_plan(p, &plan);
     wave = qw.total <= (size_t)SP_NOALLOC_SCRATCH_BYTES;
     if (wave) q = qw;
@@ -2183,9 +2188,8 @@ extern "C" int sp_compute_step_noalloc(const sp_su2_problem *p, double cutoff, c
   std::memcpy(h + q.inv, p->inv_rid, (size_t)f.L * 4);
   std::memcpy(h + q.ooff, p->ovl_off, ((size_t)f.L + 1) * 4);
   if (wave) {
-    std::memcpy(h + q.pent, plan.ent.data(), plan.ent.size() * 4);
-    std::memcpy(h + q.plane, plan.lane_of.data(), plan.lane_of.size() * 4);
-    std::memcpy(h + q.pcount, plan.count.data(), plan.count.size() * 4);
+    plan.store(reinterpret_cast<unsigned *>(h + q.pent), reinterpret_cast<int *>(h + q.pcount));
+    std::memcpy(h + q.plane, plan.lane_of, ((size_t)f.L + 1) * 4);
     f.plan_ent = reinterpret_cast<const unsigned *>(base + q.pent);
     f.plan_lane = reinterpret_cast<const int *>(base + q.plane);
     f.plan_count = reinterpret_cast<const int *>(base + q.pcount);

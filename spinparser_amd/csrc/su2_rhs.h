@@ -342,11 +342,13 @@ __host__ __device__ inline int t_wave_bytes(int L) {
 
 // distinct (rid1, rid2) pairs of every site's overlap list, with their
 // multiplicities, dealt to the lanes of a wave
-inline void build_overlap_plan(LanePlan &plan, int L, const int *off, const int *rid1, const int *rid2) {
+template <class PLAN>
+inline void build_overlap_plan(PLAN &plan, int L, const int *off, const int *rid1, const int *rid2) {
   const int lp = t_shape(L).lp;
-  plan.begin((size_t)lp * lp);
+  plan.begin((size_t)lp * lp, L);
   for (int r = 0; r < L; ++r) {
-    for (int i = off[r]; i < off[r + 1]; ++i) plan.add((unsigned)(rid1[i] * lp + rid2[i]));
+    const int *r1 = rid1 + off[r], *r2 = rid2 + off[r];
+    plan.add_list(off[r + 1] - off[r], [=](size_t i) { return (unsigned)(r1[i] * lp + r2[i]); });
     plan.end_output();
   }
   plan.deal(64);

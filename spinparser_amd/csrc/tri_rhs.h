@@ -931,23 +931,22 @@ inline TriPlan build_tri_plan(const sp_tri_problem *p) {
   auto append = [&](LanePlan &plan) {
     plan.deal(lanes);
     const size_t head = (2 + 16 * (size_t)L + lanes + 3) & ~(size_t)3, at0 = r.plan.size();
-    r.plan.resize(at0 + head + plan.ent.size());
+    r.plan.resize(at0 + head + plan.entries());
     int *o = r.plan.data() + at0;
     o[0] = plan.quads();
-    std::copy(plan.lane_of.begin(), plan.lane_of.end(), o + 1);
-    std::copy(plan.count.begin(), plan.count.end(), o + 2 + 16 * L);
-    for (size_t k = 0; k < plan.ent.size(); ++k) o[head + k] = (int)plan.ent[k];
+    std::copy_n(plan.lane_of.begin(), 16 * L + 1, o + 1);
+    plan.store(reinterpret_cast<unsigned *>(o + head), o + 2 + 16 * L);
   };
   for (int g0 = 0; g0 < ng; g0 += r.pass) {
     LanePlan plan;
-    plan.begin((size_t)waves * r.pass * 256);
+    plan.begin((size_t)waves * r.pass * 256, 16 * L);
     for (int rid = 0; rid < L; ++rid)
       for (int c = 0; c < 16; ++c) {
         auto add = [&](int at, int row, int col, int times) {
           const int g = at >> 4, w = g / ng, gi = g - w * ng;
           if (gi < g0 || gi >= g0 + r.pass) return;
           const unsigned e = ((w * r.pass + gi - g0) * 4 + ((at >> 2) & 3)) * 64 + 16 * row + 4 * (at & 3) + col;
-          for (int z = 0; z < times; ++z) plan.add(e);
+          plan.add(e, times);
         };
         const int s1 = c >> 2, s2 = c & 3;
         add(product(rid, L, none).at, s1, s2, 1);
@@ -963,12 +962,12 @@ inline TriPlan build_tri_plan(const sp_tri_problem *p) {
   }
   if (r.edges) {
     LanePlan plan;
-    plan.begin((size_t)waves * 256);
+    plan.begin((size_t)waves * 256, 16 * L);
     for (int rid = 0; rid < L; ++rid)
       for (int c = 0; c < 16; ++c) {
         auto add = [&](int b, int row, int col, int times) {
           const int z = b >> 2, w = z / r.edges, zi = z - w * r.edges;
-          for (int t = 0; t < times; ++t) plan.add((w * 4 + zi) * 64 + 16 * row + 4 * (b & 3) + col);
+          plan.add((w * 4 + zi) * 64 + 16 * row + 4 * (b & 3) + col, times);
         };
         const int s1 = c >> 2, s2 = c & 3;
         if (s1 == 3) add(block(rid >> 2, -1, none), rid & 3, s2, 1);

@@ -1,13 +1,9 @@
 // Helpers of the dGamma kernels that evaluate their frequency integrals in
 // independent waves (SU(2), XYZ and TRI cores): lane exchanges, wave-private
-// LDS, bracket searches, unit decoding, and the plan that deals the sums over
-// overlap lists to lanes.
+// LDS, bracket searches, unit decoding, and the sums of a LanePlan.
 #pragma once
-#include <algorithm>
-#include <cstddef>
-#include <vector>
-
 #include "frg_common.h"
+#include "lane_plan.h"
 
 namespace frg {
 
@@ -174,66 +170,6 @@ __device__ __forceinline__ SuBuffer su_buffer(const Bracket &t, const Bracket &o
   d.wb = make_double2((1.0 - t.b) * bh, t.b * bh);
   return d;
 }
-
-// Sums over lists of matrix elements, dealt to lanes: lanes lane_of[k] ..
-// lane_of[k + 1] sum output k; entry j of lane l is element j % 4 of the
-// quadruple at [(j / 4) * lanes + l] = index | multiplicity << 16, count[l]
-// entries.  Repeated indices of an output are merged (simple cubic, range 6:
-// 4095 overlap entries -> 1581), and a lane reads four entries per load.
-struct LanePlan {
-  int rows = 0, lanes = 0;
-  std::vector<unsigned> ent;
-  std::vector<int> lane_of, count;
-  std::vector<unsigned> item, mult;
-  std::vector<size_t> first;
-
-  int quads() const { return (rows + 3) / 4; }
-  void begin(size_t elements) {
-    item.clear();
-    mult.assign(elements, 0);
-    first.assign(1, 0);
-  }
-  void add(unsigned k) {
-    if (mult[k]++ == 0) item.push_back(k);
-  }
-  void end_output() {
-    // an entry holds multiplicities up to 0xffff; larger ones take several
-    const size_t end = item.size();
-    for (size_t j = first.back(); j < end; ++j) {
-      const unsigned k = item[j];
-      unsigned left = mult[k];
-      mult[k] = 0;
-      for (; left > 0xffffu; left -= 0xffffu) item.push_back(k | 0xffff0000u);
-      item[j] = k | left << 16;
-    }
-    first.push_back(item.size());
-  }
-  // outputs <= nlanes
-  void deal(int nlanes) {
-    lanes = nlanes;
-    const int n = (int)first.size() - 1;
-    auto need = [&](int k) { return std::max<int>(1, (int)((first[k + 1] - first[k] + rows - 1) / rows)); };
-    for (rows = std::max(1, (int)((item.size() + nlanes - 1) / nlanes));; ++rows) {
-      int used = 0;
-      for (int k = 0; k < n; ++k) used += need(k);
-      if (used <= nlanes) break;
-    }
-    ent.assign((size_t)quads() * 4 * nlanes, 0);
-    count.assign(nlanes, 0);
-    lane_of.assign(n + 1, 0);
-    int lane = 0;
-    for (int k = 0; k < n; ++k) {
-      lane_of[k] = lane;
-      for (size_t j = first[k]; j < first[k + 1]; ++j) {
-        const int l = lane + (int)((j - first[k]) / rows), row = (int)((j - first[k]) % rows);
-        ent[((size_t)(row >> 2) * nlanes + l) * 4 + (row & 3)] = item[j];
-        count[l] = row + 1;
-      }
-      lane += need(k);
-    }
-    lane_of[n] = lane;
-  }
-};
 
 // a lane's sum over its entries of a plan (ent: the lane's first quadruple);
 // the next quadruple is loaded while one is summed

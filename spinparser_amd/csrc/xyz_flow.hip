@@ -1203,7 +1203,7 @@ int xyz_wave_tables(sp_xyz_ctx *ctx, const sp_xyz_problem *p, const XyzOrder &or
     align4();
     plan_at = table.size();
     for (int t0 = 0; t0 < ntiles; t0 += kXyzPassTiles) {
-      plan.begin((size_t)kXyzPassTiles * 256);
+      plan.begin((size_t)kXyzPassTiles * 256, 4 * L);
       for (int k = 0; k < 4 * L; ++k) {  // outputs in the order of a device row
           const int c = 2 * (k / (2 * L)) + (k & 1), r = (k % (2 * L)) / 2;
           for (int i = p->ovl_off[r]; i < p->ovl_off[r + 1]; ++i) {
@@ -1216,10 +1216,13 @@ int xyz_wave_tables(sp_xyz_ctx *ctx, const sp_xyz_problem *p, const XyzOrder &or
         }
       plan.deal(64 * kRhsWaves);
       table.push_back(plan.quads());
-      table.insert(table.end(), plan.lane_of.begin(), plan.lane_of.end());
-      table.insert(table.end(), plan.count.begin(), plan.count.end());
+      table.insert(table.end(), plan.lane_of.begin(), plan.lane_of.begin() + 4 * L + 1);
+      const size_t count_at = table.size();
+      table.resize(count_at + plan.lanes);
       align4();
-      for (unsigned e : plan.ent) table.push_back((int)e);
+      const size_t ent_at = table.size();
+      table.resize(ent_at + plan.entries());
+      plan.store(reinterpret_cast<unsigned *>(table.data() + ent_at), table.data() + count_at);
     }
   } catch (...) { return xfail(ctx, SP_ENOMEM, "host buffer"); }
   const size_t lds = xyz_t_lds(f.nw, L, lps);
