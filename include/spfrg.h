@@ -166,7 +166,10 @@ int sp_ctx_footprint(const sp_su2_problem *problem, long long *bytes);
  * (SpinParser::runCore's isDiverged check); null: fully asynchronous after
  * the upload.  Every call on one GPU shares that GPU's array: calls that
  * overlap on one GPU (other threads, other streams) race.  Results equal
- * sp_compute_step on a context holding the same state. */
+ * sp_compute_step on a context holding the same state: bit for bit where d_dv4
+ * is an ordinary allocation of the current device, to FP64 rounding where it is
+ * other memory the device can write (pinned or managed host memory, fine-grained
+ * memory, another GPU's). */
 #define SP_NOALLOC_SCRATCH_BYTES (4 << 20)
 int sp_compute_step_noalloc(const sp_su2_problem *problem, double cutoff, const double *d_v2, const double *d_v4,
                             double *d_dv2, double *d_dv4, void *stream, int *diverged);

@@ -66,6 +66,7 @@
 #include <vector>
 
 #include "spfrg.h"
+#include "atomic_memory.h"
 #include "frg_common.h"
 #include "wave_rhs.h"
 
@@ -2158,13 +2159,11 @@ extern "C" int sp_compute_step_noalloc(const sp_su2_problem *p, double cutoff, c
   int rc = noalloc_scratch(dev, &base, &max_lds);
   if (rc != SP_OK) return rc;
   if (lds > (size_t)max_lds) return SP_EARG;
-  // the wave kernels add to d_dv4 with FP64 atomics of the memory side, which
-  // ordinary device memory takes; any other buffer runs the general kernel
   NoAllocOverlap &plan = g_noalloc_overlap;
   bool wave = false;
   if (f.L <= kMaxRhsL) {
     hipPointerAttribute_t at{};
-    if (hipPointerGetAttributes(&at, d_dv4) == hipSuccess) wave = at.type == hipMemoryTypeDevice && !at.isManaged;
+    if (hipPointerGetAttributes(&at, d_dv4) == hipSuccess) wave = takes_fp64_atomics(at, dev);
     else (void)hipGetLastError();
   }
   if (wave) {
