@@ -10,8 +10,10 @@ namespace frg {
 constexpr int kRhsWaves = 4;    // waves (independent work units) per workgroup
 constexpr int kRhsPoints = 16;  // points described per production pass: 64 lanes, four per point
 // byte offsets past every vertex (smaller than 2 GiB): buffer loads return 0.
-// Rows of points past the list, and sites past L; their sum stays below 2^32
+// Rows of points past the list, and sites past L.  Nothing is added to the sum
+// of the two; to a row past the list, offsets within a row are
 constexpr unsigned kNoRow = 0x80000000u, kNoSite = 0x7ffffff0u;
+static_assert((unsigned long long)kNoRow + kNoSite + 16 <= 1ull << 32, "a 16-byte load at the sum does not wrap");
 
 // value of the other lane of an even/odd lane pair
 __device__ __forceinline__ int pair_swap(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true); }

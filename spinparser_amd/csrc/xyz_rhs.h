@@ -15,8 +15,8 @@
 // k_xyz_t the alternation of gathers and matrix instructions (26 % of its
 // time) between barriers.  Honeycomb Heisenberg-Kitaev, 23 sites, 64
 // frequencies, against one workgroup per item with a producer wave: 8.78 ->
-// 3.93 ms at cutoff 20, 23.5 -> 10.3 ms at 0.7, 38.3 -> 15.8 ms at 0.02 (k_xyz_su
-// 6.1 ms, k_xyz_t 9.9 ms).
+// 3.86 ms at cutoff 20, 23.5 -> 10.2 ms at 0.7, 38.3 -> 15.6 ms at 0.02 (k_xyz_su
+// 6.1 ms, k_xyz_t 9.6 ms).
 #pragma once
 
 constexpr int kMaxXyzRhsL = 32;
@@ -42,7 +42,9 @@ __host__ __device__ inline XyzShape xyz_shape(int lps) {
 struct Vec4 {
   double x, y, z, d;
 };
-// the four supports of a buffer at one site (components X, Y and Z, D)
+// the four supports of a buffer at one site (components X, Y and Z, D).  Lanes
+// without a point or without a second site read what a neighbour reads and keep
+// nothing of it: an offset past the vertex could wrap with the half row added.
 struct Quad4 {
   double2 a[4], b[4];
 };
@@ -127,7 +129,7 @@ __global__ __launch_bounds__(64 * kRhsWaves, 3) void k_xyz_su(XyzDev F, long lon
   const int slot = active ? slot0 : sh.slots - 1;
   const XyzLane ln = F.lanes[lj];
   const bool cyc = (ln.pb >> 12) & 1;
-  const unsigned sa = active ? (unsigned)ln.a * 16u : kNoSite, sb = active && ln.b >= 0 ? (unsigned)ln.b * 16u : kNoSite;
+  const unsigned sa = (unsigned)ln.a * 16u, sb = ln.b >= 0 ? (unsigned)ln.b * 16u : sa;
   // first result (t = b, o = a), second (t = a, o = b); sites a, b of the lane
   Vec4 r1[2], r2[2];
 #pragma unroll
@@ -278,8 +280,8 @@ __global__ __launch_bounds__(64 * kRhsWaves, 3) void k_xyz_su(XyzDev F, long lon
 // P[a][r1] Q[b][r2] of the pair's bundles (spin components a, b): the waves
 // write P = c A0 and Q = A1 of their points to LDS and accumulate the 16 x 16
 // tiles of the 4 L x 4 L product matrix that the overlap lists refer to, each
-// wave its own tiles, on the matrix cores.  Three waves per SIMD although the
-// largest lattices then spill 30 registers: 2 to 15 % faster than two.
+// wave its own tiles, on the matrix cores.  Three waves per SIMD although up to
+// 28 tiles then spill 23 registers and more 96: 2 to 15 % faster than two.
 // density of a T buffer on its diagonal supports
 __device__ __forceinline__ double diagonal4(int2 fl, double2 wa, double2 wb, const Quad4 &q) {
   const double m0 = (fl.x & 4) ? wa.x : 0.0, m1 = (fl.x & 8) ? wa.y : 0.0;
@@ -346,7 +348,7 @@ __global__ __launch_bounds__(64 * kRhsWaves, 3) void k_xyz_t(XyzDev F) {
   const int slot = active ? slot0 : sh.slots - 1;
   const XyzLane ln = F.lanes[lj];
   const bool cyc = (ln.pb >> 12) & 1;
-  const unsigned sa = active ? (unsigned)ln.a * 16u : kNoSite, sb = active && ln.b >= 0 ? (unsigned)ln.b * 16u : kNoSite;
+  const unsigned sa = (unsigned)ln.a * 16u, sb = ln.b >= 0 ? (unsigned)ln.b * 16u : sa;
   Vec4 acc[2];
   acc[0] = acc[1] = Vec4{0.0, 0.0, 0.0, 0.0};
   d4 C[TPW];
