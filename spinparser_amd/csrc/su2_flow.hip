@@ -1495,7 +1495,7 @@ int sp_ctx_footprint(const sp_su2_problem *p, long long *bytes) {
   if (p->precision == SP_PRECISION_MIXED) b += nf * p->L * 8;  // FP32 shadow
   b += 3LL * p->nw * 8;                                          // Sigma, dSigma, mesh
   b += 2 * (long long)p->nw * emax * 8 + 2 * emax * 8 + (p->nw + 1) * 4;  // weight tables
-  b += emax * p->L * 16 + 2LL * p->B * p->Rb * 8 + 32;                   // correlation scratch / output, flags
+  b += emax * p->L * 16 + 32;                                            // correlation scratch, flags
   b += 4LL * (3 * p->L + 1 + 2 * p->R + p->B * p->Rb);
   b += 2LL * (p->ovl_off ? p->ovl_off[p->L] : 0);                         // packed overlap indices
   if (p->L <= kMaxRhsL)  // overlap plan of k_t: at most two places per entry, and the lane tables
@@ -1558,7 +1558,7 @@ int sp_ctx_create(const sp_su2_problem *p, sp_ctx **out) {
       (rc = dalloc(ctx, &f.Wc, (size_t)f.nw * emax)) || (rc = dalloc(ctx, &f.Wn, f.nw)) ||
       (rc = dalloc(ctx, &f.Cwp, emax)) || (rc = dalloc(ctx, &f.Cw, emax)) || (rc = dalloc(ctx, &f.Cn, 1)) ||
       (rc = dalloc(ctx, &f.corr_partial, (size_t)emax * f.L * 2)) ||
-      (rc = dalloc(ctx, &f.corr_out, (size_t)2 * f.B * f.Rb + 1)) || (rc = dalloc(ctx, &f.flags, 8)) ||
+      (rc = dalloc(ctx, &f.flags, 8)) ||
       (rc = dalloc(ctx, &ctx->d_fd, 1)))
     return rc;
   {

@@ -1226,11 +1226,16 @@ int sp_tri_ctx_footprint(const sp_tri_problem *p, long long *bytes) {
   long long b = 2 * nf * 16 * p->L * 8;                                       // Gamma, dGamma
   b += 3LL * p->nw * 8;                                                       // Sigma, dSigma, mesh
   b += 2 * (long long)p->nw * emax * 8 + 2 * emax * 8 + (p->nw + 1) * 4;      // weight tables
-  b += emax * 10 * p->L * 8 + 10LL * p->B * p->Rb * 8 + 16;                   // correlation scratch, output, flags
+  b += emax * 10 * p->L * 8 + 16;                                             // correlation scratch, flags
   b += 4LL * (10 * p->L + 1 + 5 * O + 2 * p->R + 4 * p->B * p->Rb);           // lattice tables
-  if (p->L <= kMaxTriRhsL)
-    b += std::min<long long>(nf * 16 * p->L * 8, 32ll << 20) + 4LL * 32 * p->L +
-         64LL * 16 * 8 * kTriMaxGroups + 64LL * (32 * p->L + 512 + O);  // staging rows, tables of the T kernel
+  if (check_tri_problem(nullptr, p) == SP_OK) {
+    try {
+      const TriPlan plan = build_tri_plan(p);
+      if (plan.ok)  // staging rows, tables of k_tri_t
+        b += std::min<long long>(nf * 16 * p->L * 8, 32ll << 20) +
+             4LL * (long long)(plan.dst.size() + plan.plan.size() + plan.edge_ops.size()) + 16LL * (long long)plan.ops.size();
+    } catch (...) { return SP_ENOMEM; }
+  }
   *bytes = b;
   return SP_OK;
 }
@@ -1363,7 +1368,7 @@ int sp_tri_ctx_create(const sp_tri_problem *p, sp_tri_ctx **out) {
       (rc = talloc(ctx, &f.Wwp, (size_t)f.nw * emax)) || (rc = talloc(ctx, &f.Wc, (size_t)f.nw * emax)) ||
       (rc = talloc(ctx, &f.Wn, f.nw)) || (rc = talloc(ctx, &f.Cwp, emax)) || (rc = talloc(ctx, &f.Cw, emax)) ||
       (rc = talloc(ctx, &f.Cn, 1)) || (rc = talloc(ctx, &f.corr_partial, (size_t)emax * 10 * f.L)) ||
-      (rc = talloc(ctx, &f.corr_out, 10 * nc + 1)) || (rc = talloc(ctx, &f.flags, 4)) ||
+      (rc = talloc(ctx, &f.flags, 4)) ||
       (f.t_waves && ((rc = talloc(ctx, &tdst, plan.dst.size())) || (rc = talloc(ctx, &tedge, plan.edge_ops.size())) || (rc = talloc(ctx, &tplan, plan.plan.size())) ||
                      (rc = talloc(ctx, &tops, plan.ops.size())) ||
                      (rc = talloc(ctx, &ctx->stage, (size_t)tri_stage_rows(f) * 16 * f.L)))))

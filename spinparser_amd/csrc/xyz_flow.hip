@@ -1159,83 +1159,91 @@ XyzOrder xyz_order(const sp_xyz_problem *p) {
 // Tables of the wave kernels, if the lattice has the form they need: lanes of
 // a point, the tiles of the bubble product matrix that the overlap lists refer
 // to, and the plan of their sums.
-int xyz_wave_tables(sp_xyz_ctx *ctx, const sp_xyz_problem *p, const XyzOrder &order, int max_lds) {
-  XyzDev &f = ctx->fd;
-  const int L = f.L;
-  if (!order.waves) return SP_OK;
-  std::vector<int> table;  // lanes, tiles, then the plans of the passes
-  LanePlan plan;
-  const int lps = (int)order.first.size();
-  int ntiles = 0;
+struct XyzWaves {
+  int lps = 0, ntiles = 0;
   size_t tiles_at = 0, plan_at = 0;
+  std::vector<int> table;  // lanes, tiles, then the plans of the passes; empty: another form
+};
+XyzWaves xyz_wave_tables(const sp_xyz_problem *p, const XyzOrder &order) {
+  XyzWaves w;
+  const int L = p->L;
+  if (!order.waves) return w;
+  std::vector<int> &table = w.table;
+  LanePlan plan;
+  const int lps = w.lps = (int)order.first.size();
+  int &ntiles = w.ntiles;
   auto align4 = [&] { table.resize((table.size() + 3) & ~size_t(3), 0); };
-  try {
-    auto packed = [](const int *q) { return q[0] | q[1] << 2 | q[2] << 4; };
-    auto perms = [&](int r) { return packed(p->site_perm + 3 * r) | packed(p->inv_perm + 3 * r) << 6; };
-    for (int j = 0; j < lps; ++j) {
-      const int a = order.first[j], b = order.second[j];
-      const int cyc = b >= 0 && p->inv_rid[a] == b;
-      const XyzLane ln{a, b, perms(a), b >= 0 ? perms(b) | cyc << 12 : 0};
-      table.insert(table.end(), {ln.a, ln.b, ln.pa, ln.pb});
+  auto packed = [](const int *q) { return q[0] | q[1] << 2 | q[2] << 4; };
+  auto perms = [&](int r) { return packed(p->site_perm + 3 * r) | packed(p->inv_perm + 3 * r) << 6; };
+  for (int j = 0; j < lps; ++j) {
+    const int a = order.first[j], b = order.second[j];
+    const int cyc = b >= 0 && p->inv_rid[a] == b;
+    const XyzLane ln{a, b, perms(a), b >= 0 ? perms(b) | cyc << 12 : 0};
+    table.insert(table.end(), {ln.a, ln.b, ln.pa, ln.pb});
+  }
+  // element (a, r1), (b, r2) of the product matrix
+  const int nt = (4 * L + 15) / 16, O = p->ovl_off[L];
+  std::vector<int> tile((size_t)nt * nt, -1);
+  std::vector<int> list;
+  auto rows_cols = [&](int i, int c, int &row, int &col) {
+    row = (c < 3 ? p->ovl_perm1[3 * i + c] : 3) * L + p->ovl_rid1[i];
+    col = (c < 3 ? p->ovl_perm2[3 * i + c] : 3) * L + p->ovl_rid2[i];
+  };
+  for (int i = 0; i < O; ++i)
+    for (int c = 0; c < 4; ++c) {
+      int row, col;
+      rows_cols(i, c, row, col);
+      tile[(row >> 4) * nt + (col >> 4)] = 0;
     }
-    // element (a, r1), (b, r2) of the product matrix
-    const int nt = (4 * L + 15) / 16, O = p->ovl_off[L];
-    std::vector<int> tile((size_t)nt * nt, -1);
-    std::vector<int> list;
-    auto rows_cols = [&](int i, int c, int &row, int &col) {
-      row = (c < 3 ? p->ovl_perm1[3 * i + c] : 3) * L + p->ovl_rid1[i];
-      col = (c < 3 ? p->ovl_perm2[3 * i + c] : 3) * L + p->ovl_rid2[i];
-    };
-    for (int i = 0; i < O; ++i)
-      for (int c = 0; c < 4; ++c) {
-        int row, col;
-        rows_cols(i, c, row, col);
-        tile[(row >> 4) * nt + (col >> 4)] = 0;
-      }
-    for (int k = 0; k < nt * nt; ++k)
-      if (tile[k] == 0) {
-        tile[k] = ntiles++;
-        list.push_back((k / nt) * 16 | (k % nt) * 16 << 16);
-      }
-    if (ntiles > kXyzMaxTiles * kRhsWaves) return SP_OK;
-    tiles_at = table.size();
-    table.insert(table.end(), list.begin(), list.end());
-    align4();
-    plan_at = table.size();
-    for (int t0 = 0; t0 < ntiles; t0 += kXyzPassTiles) {
-      plan.begin((size_t)kXyzPassTiles * 256, 4 * L);
-      for (int k = 0; k < 4 * L; ++k) {  // outputs in the order of a device row
-          const int c = 2 * (k / (2 * L)) + (k & 1), r = (k % (2 * L)) / 2;
-          for (int i = p->ovl_off[r]; i < p->ovl_off[r + 1]; ++i) {
-            int row, col;
-            rows_cols(i, c, row, col);
-            const int t = tile[(row >> 4) * nt + (col >> 4)] - t0;
-            if (t >= 0 && t < kXyzPassTiles) plan.add((unsigned)(t * 256 + (row & 15) * 16 + (col & 15)));
-          }
-          plan.end_output();
+  for (int k = 0; k < nt * nt; ++k)
+    if (tile[k] == 0) {
+      tile[k] = ntiles++;
+      list.push_back((k / nt) * 16 | (k % nt) * 16 << 16);
+    }
+  if (ntiles > kXyzMaxTiles * kRhsWaves) return XyzWaves{};
+  w.tiles_at = table.size();
+  table.insert(table.end(), list.begin(), list.end());
+  align4();
+  w.plan_at = table.size();
+  for (int t0 = 0; t0 < ntiles; t0 += kXyzPassTiles) {
+    plan.begin((size_t)kXyzPassTiles * 256, 4 * L);
+    for (int k = 0; k < 4 * L; ++k) {  // outputs in the order of a device row
+        const int c = 2 * (k / (2 * L)) + (k & 1), r = (k % (2 * L)) / 2;
+        for (int i = p->ovl_off[r]; i < p->ovl_off[r + 1]; ++i) {
+          int row, col;
+          rows_cols(i, c, row, col);
+          const int t = tile[(row >> 4) * nt + (col >> 4)] - t0;
+          if (t >= 0 && t < kXyzPassTiles) plan.add((unsigned)(t * 256 + (row & 15) * 16 + (col & 15)));
         }
-      plan.deal(64 * kRhsWaves);
-      table.push_back(plan.quads());
-      table.insert(table.end(), plan.lane_of.begin(), plan.lane_of.begin() + 4 * L + 1);
-      const size_t count_at = table.size();
-      table.resize(count_at + plan.lanes);
-      align4();
-      const size_t ent_at = table.size();
-      table.resize(ent_at + plan.entries());
-      plan.store(reinterpret_cast<unsigned *>(table.data() + ent_at), table.data() + count_at);
-    }
-  } catch (...) { return xfail(ctx, SP_ENOMEM, "host buffer"); }
-  const size_t lds = xyz_t_lds(f.nw, L, lps);
-  if (lds > (size_t)max_lds) return SP_OK;
+        plan.end_output();
+      }
+    plan.deal(64 * kRhsWaves);
+    table.push_back(plan.quads());
+    table.insert(table.end(), plan.lane_of.begin(), plan.lane_of.begin() + 4 * L + 1);
+    const size_t count_at = table.size();
+    table.resize(count_at + plan.lanes);
+    align4();
+    const size_t ent_at = table.size();
+    table.resize(ent_at + plan.entries());
+    plan.store(reinterpret_cast<unsigned *>(table.data() + ent_at), table.data() + count_at);
+  }
+  return w;
+}
+// the wave kernels for a context, if its lattice has their form
+int xyz_use_waves(sp_xyz_ctx *ctx, const sp_xyz_problem *p, const XyzOrder &order, int max_lds) {
+  XyzDev &f = ctx->fd;
+  XyzWaves w;
+  try { w = xyz_wave_tables(p, order); } catch (...) { return xfail(ctx, SP_ENOMEM, "host buffer"); }
+  if (w.table.empty() || xyz_t_lds(f.nw, f.L, w.lps) > max_lds) return SP_OK;
   int *d = nullptr;
-  int rc = xalloc(ctx, &d, table.size());
+  int rc = xalloc(ctx, &d, w.table.size());
   if (rc) return rc;
-  SP_XHIP(hipMemcpy(d, table.data(), table.size() * 4, hipMemcpyHostToDevice));
-  f.lps = lps;
-  f.ntiles = ntiles;
+  SP_XHIP(hipMemcpy(d, w.table.data(), w.table.size() * 4, hipMemcpyHostToDevice));
+  f.lps = w.lps;
+  f.ntiles = w.ntiles;
   f.lanes = reinterpret_cast<const XyzLane *>(d);
-  f.tiles = d + tiles_at;
-  f.plan = d + plan_at;
+  f.tiles = d + w.tiles_at;
+  f.plan = d + w.plan_at;
   SP_XHIP(hipFuncSetAttribute((const void *)k_xyz_t<4>, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
   SP_XHIP(hipFuncSetAttribute((const void *)k_xyz_t<7>, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
   SP_XHIP(hipFuncSetAttribute((const void *)k_xyz_t<kXyzMaxTiles>, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds));
@@ -1330,10 +1338,17 @@ int sp_xyz_ctx_footprint(const sp_xyz_problem *p, long long *bytes) {
   long long b = 2 * nf * 4 * p->L * 8;                                        // Gamma, dGamma
   b += 3LL * p->nw * 8;                                                       // Sigma, dSigma, mesh
   b += 2 * (long long)p->nw * emax * 8 + 2 * emax * 8 + (p->nw + 1) * 4;      // weight tables
-  b += emax * 4 * p->L * 8 + 4LL * p->B * p->Rb * 8 + 16;                     // correlation scratch, output, flags
-  b += 4LL * (8 * p->L + 1 + 8 * O + 2 * p->R + 4 * p->B * p->Rb);            // lattice tables
+  b += emax * 4 * p->L * 8 + 16;                                              // correlation scratch, flags
+  b += 4LL * (9 * p->L + 1 + 8 * O + 2 * p->R + 4 * p->B * p->Rb);            // lattice tables
   b += 16LL * O;                                                              // bubble-matrix indices
   b += std::min<long long>(nf * 4 * p->L * 8, 32ll << 20) + 16LL * p->L;      // staging rows, their order
+  if (check_xyz_problem(nullptr, p) == SP_OK) {
+    try {
+      const XyzOrder order = xyz_order(p);
+      const XyzTables tables(p, order.order);
+      b += 4LL * (long long)xyz_wave_tables(&tables.q, order).table.size();     // tables of the wave kernels
+    } catch (...) { return SP_ENOMEM; }
+  }
   *bytes = b;
   return SP_OK;
 }
@@ -1432,7 +1447,7 @@ static int xyz_ctx_init(sp_xyz_ctx *ctx, const sp_xyz_problem *p, const XyzOrder
       (rc = xalloc(ctx, &f.Wwp, (size_t)f.nw * emax)) || (rc = xalloc(ctx, &f.Wc, (size_t)f.nw * emax)) ||
       (rc = xalloc(ctx, &f.Wn, f.nw)) || (rc = xalloc(ctx, &f.Cwp, emax)) || (rc = xalloc(ctx, &f.Cw, emax)) ||
       (rc = xalloc(ctx, &f.Cn, 1)) || (rc = xalloc(ctx, &f.corr_partial, (size_t)emax * 4 * f.L)) ||
-      (rc = xalloc(ctx, &f.corr_out, 4 * nc + 1)) || (rc = xalloc(ctx, &f.flags, 4)))
+      (rc = xalloc(ctx, &f.flags, 4)))
     return rc;
   int4 *midx_d = nullptr;
   if ((rc = xalloc(ctx, &midx_d, midx.size()))) return rc;
@@ -1476,7 +1491,7 @@ static int xyz_ctx_init(sp_xyz_ctx *ctx, const sp_xyz_problem *p, const XyzOrder
   SP_XHIP(hipMemcpy(ri, p->range_inv, (size_t)f.R * 4, hipMemcpyHostToDevice));
   SP_XHIP(hipMemcpy(corr, p->corr_rid, nc * 4, hipMemcpyHostToDevice));
   SP_XHIP(hipMemcpy(corrp, p->corr_perm, 3 * nc * 4, hipMemcpyHostToDevice));
-  if (!(force && std::strcmp(force, "direct") == 0) && (rc = xyz_wave_tables(ctx, p, order, max_lds))) return rc;
+  if (!(force && std::strcmp(force, "direct") == 0) && (rc = xyz_use_waves(ctx, p, order, max_lds))) return rc;
   SP_XHIP(hipMemset(f.G, 0, nv * 8));
   SP_XHIP(hipMemset(f.dG, 0, nv * 8));
   SP_XHIP(hipMemset(f.v2, 0, f.nw * 8));
