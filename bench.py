@@ -22,11 +22,13 @@ dGamma/dLambda evaluations per second (``value``, FP64 form).  Beside it:
   derivative on a common state;
 * ``fixed_cutoff``: evals/s at the first, middle and last cutoff with the
   algorithmic work F(cutoff) of one evaluation;
-* ``roofline``: the dGamma kernel timed with HIP events on the context's
-  stream; achieved = algorithmic FLOP of the timed evaluations (exact
-  integrand-call counts x per-call work model) / summed kernel time, against
-  the MI355X FP64 peak; ``traffic`` = HBM bytes per launch from rocprofv3
-  FETCH_SIZE / WRITE_SIZE (table below);
+* ``roofline``: the dGamma kernels timed with HIP events on the context's
+  stream; achieved = the operations the timed evaluations cannot do without
+  (necessary_flops: exact point counts, each symmetric image and each product of
+  sites once) / summed kernel time, against the MI355X FP64 peak;
+  ``reference_tflops`` is the same with the operations of the reference's kernels
+  (``algorithmic_tflop_total``), which the kernels do not execute; ``traffic`` =
+  HBM bytes per evaluation from rocprofv3 FETCH_SIZE / WRITE_SIZE (table below);
 * ``cpu_baseline``: the reference-arithmetic CPU oracle with OpenMP over items
   on a bounded sample of the same workload, extrapolated by integrand-call
   counts over the schedule.
@@ -63,7 +65,7 @@ from spinparser_amd.capi import (KERNEL_DGAMMA, SP_PRECISION_FP64, SP_PRECISION_
                                  FlowContext, TriFlowContext, XyzFlowContext, footprint_bytes)
 from spinparser_amd.problem import su2_problem, tri_problem, xyz_problem  # noqa: E402
 from spinparser_amd.task import make_task_xml, parse_task  # noqa: E402
-from spinparser_amd.workload import compulsory_bytes, evaluation_flops  # noqa: E402
+from spinparser_amd.workload import compulsory_bytes, evaluation_flops, necessary_flops  # noqa: E402
 
 FP64_PEAK_TFLOPS = 78.6
 HBM_PEAK_GBS = 8000.0
@@ -90,27 +92,33 @@ XYZ_WORKLOAD = dict(lattice="honeycomb", lattice_range=8, model="honeycomb-kitae
                     freq_min=0.005, freq_max=50.0, freq_count=64, cutoff_max=50.0, cutoff_min=0.01, cutoff_step=0.98)
 
 # the cores measured beside the SU(2) flow: workload, problem builder, context,
-# oracle class name and dGamma kernel name
+# oracle class name and the kernels that the dGamma timer brackets (dGamma is
+# cleared in k_tri_clear, in the SU(2) and XYZ cores by k_weights and k_xyz_weights
+# outside the bracket)
+DGAMMA_KERNELS = "k_su + k_t"
 CORES = {
     "tri": dict(label="TRI", workload="kagome-dm-r5-nw48", spec=TRI_WORKLOAD, symmetry="TRI", build=tri_problem,
-                context=TriFlowContext, oracle="TriOracle", kernel="k_tri_dgamma"),
+                context=TriFlowContext, oracle="TriOracle", kernel="k_tri_clear + k_tri_su + k_tri_t"),
     "xyz": dict(label="XYZ", workload="honeycomb-kitaev-r8-nw64", spec=XYZ_WORKLOAD, symmetry="XYZ",
-                build=xyz_problem, context=XyzFlowContext, oracle="XyzOracle", kernel="k_xyz_dgamma"),
+                build=xyz_problem, context=XyzFlowContext, oracle="XyzOracle", kernel="k_xyz_su + k_xyz_t"),
 }
 
-# HBM bytes of the dGamma kernels (k_su and k_t) per evaluation over the full
-# flow, from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (KiB, averaged over the
-# evaluations of the full flow).  Each counter is multiplied by the ratio of known
-# bytes to counter reading for a plain streaming kernel of known size (k_euler
-# reads Gamma and dGamma, writes Gamma: FETCH_SIZE reads half the known bytes,
-# scale 2.00; WRITE_SIZE reads them exactly, scale 1.00).  The profile summaries
-# under profiles/ hold the runs and the commands; workloads without an entry have
-# not been counted with these kernels.
+# HBM bytes of the dGamma kernels (those the timer brackets) per evaluation over
+# the full flow, from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (KiB, averaged over
+# the evaluations of the full flow).  Each counter is multiplied by the ratio of
+# known bytes to counter reading for a plain streaming kernel of known size (the
+# Euler kernel reads Gamma and dGamma, writes Gamma: FETCH_SIZE reads half the
+# known bytes, scale 2.00; WRITE_SIZE reads them exactly, scale 1.00).  The profile
+# summaries under profiles/ hold the runs and the commands.
 TRAFFIC_KIB = {
-    ("cubic-j1j2-r6-nw64", "f64"): {"fetch_kib": 263184.1, "write_kib": 149068.4,
+    ("cubic-j1j2-r6-nw64", "f64"): {"fetch_kib": 263179.4, "write_kib": 149068.7,
                                     "fetch_scale": 2.00, "write_scale": 1.00},
-    ("square-r4-nw32", "f64"): {"fetch_kib": 9547.1, "write_kib": 7720.0,
+    ("square-r4-nw32", "f64"): {"fetch_kib": 9547.6, "write_kib": 7720.0,
                                 "fetch_scale": 2.00, "write_scale": 1.00},
+    ("kagome-dm-r5-nw48", "f64"): {"fetch_kib": 990083.6, "write_kib": 3593973.7,
+                                   "fetch_scale": 2.00, "write_scale": 1.00},
+    ("honeycomb-kitaev-r8-nw64", "f64"): {"fetch_kib": 719914.5, "write_kib": 2830006.2,
+                                          "fetch_scale": 2.00, "write_scale": 1.00},
 }
 
 
@@ -213,9 +221,10 @@ def flow_leg(prob, precision, steps, warmup, label, queued=True):
     ctx.set_state(float(prob.cutoffs[0]), *init)
     # algorithmic FLOP per evaluation, counted before the timed region
     step_flops = [evaluation_flops(prob, prob.cutoffs[k]) for k in range(nsteps_flow)]
+    step_work = [necessary_flops(prob, prob.cutoffs[k]) for k in range(nsteps_flow)]
     ctx.synchronize()
     ctx.profile(True)
-    flops = 0.0
+    flops = work = 0.0
     records = []
     t0 = time.perf_counter()
     if queued:
@@ -229,6 +238,7 @@ def flow_leg(prob, precision, steps, warmup, label, queued=True):
                 raise RuntimeError("flow diverged at cutoff index %d" % (len(recs) - 1))
             records = recs
             flops += sum(step_flops[:n])
+            work += sum(step_work[:n])
             done += n
             print("# %s step %d / %d  %.1f s" % (label, done, steps, time.perf_counter() - t0), file=sys.stderr,
                   flush=True)
@@ -240,6 +250,7 @@ def flow_leg(prob, precision, steps, warmup, label, queued=True):
                 records = []
             run_step(ctx, prob, k, records)
             flops += step_flops[k]
+            work += step_work[k]
             if (i + 1) % 100 == 0:
                 print("# %s step %d / %d  cutoff %.5g  %.1f s" % (label, i + 1, steps, prob.cutoffs[k],
                                                                  time.perf_counter() - t0), file=sys.stderr, flush=True)
@@ -249,7 +260,7 @@ def flow_leg(prob, precision, steps, warmup, label, queued=True):
     ctx.profile(False)
     final = ctx.get_state() if steps % nsteps_flow == 0 else None
     ctx.close()
-    return dict(elapsed=elapsed, dg_ms=dg_ms, dg_n=dg_n, flops=flops, records=records, final=final)
+    return dict(elapsed=elapsed, dg_ms=dg_ms, dg_n=dg_n, flops=flops, work=work, records=records, final=final)
 
 
 def fixed_cutoff(prob, precision, reps=5):
@@ -276,7 +287,8 @@ def fixed_cutoff(prob, precision, reps=5):
         f = evaluation_flops(prob, prob.cutoffs[k])
         kern = (ms1 - ms0) * 1e-3 / max(n1 - n0, 1)
         out.append({"cutoff": float(prob.cutoffs[k]), "gflop_per_eval": f / 1e9, "evals_per_s": 1.0 / wall,
-                    "k_dgamma_ms": kern * 1e3, "tflops_k_dgamma": f / kern / 1e12})
+                    "dgamma_ms": kern * 1e3,
+                    "tflops_dgamma": necessary_flops(prob, prob.cutoffs[k]) / kern / 1e12})
     ctx.close()
     return out
 
@@ -313,8 +325,6 @@ def core_leg(core, samples=5, reps=2):
     ks = [int(round(x)) for x in np.linspace(0, ncut - 2, samples)]
     v2, v4 = p.initial_state(np.float64)
     ctx = c["context"](p)
-    kkey = c["kernel"] + "_ms"
-    tkey = "tflops_" + c["kernel"]
     pts = []
     for k in ks:
         ctx.set_state(float(p.cutoffs[k]), v2, v4)
@@ -332,7 +342,7 @@ def core_leg(core, samples=5, reps=2):
         f = evaluation_flops(p, p.cutoffs[k])
         kern = (ms1 - ms0) * 1e-3 / max(1, n1 - n0)
         pts.append({"cutoff": float(p.cutoffs[k]), "index": k, "gflop_per_eval": f / 1e9, "evals_per_s": 1.0 / wall,
-                    kkey: kern * 1e3, tkey: f / kern / 1e12})
+                    "dgamma_ms": kern * 1e3, "tflops_dgamma": necessary_flops(p, p.cutoffs[k]) / kern / 1e12})
     ctx.close()
     # seconds per FLOP, piecewise linear in the cutoff index between samples
     idx = np.array([q["index"] for q in pts], dtype=float)
@@ -340,7 +350,7 @@ def core_leg(core, samples=5, reps=2):
     flops = np.array([evaluation_flops(p, p.cutoffs[k]) for k in range(ncut - 1)])
     est = float(np.sum(flops * np.interp(np.arange(ncut - 1), idx, spf)))
     return {"workload": c["workload"], "L": p.L, "nw": p.nw, "overlap_terms": p.overlap_total,
-            "n_freq_triples": p.n_freq, "cutoffs": ncut, "samples": pts,
+            "n_freq_triples": p.n_freq, "cutoffs": ncut, "kernel": c["kernel"], "samples": pts,
             "full_flow_algorithmic_tflop": float(flops.sum()) / 1e12,
             "est_full_flow_s": est, "est_evals_per_s": (ncut - 1) / est,
             "method": "%d evaluations at each of %d cutoffs, integrated over the schedule by algorithmic FLOP"
@@ -398,7 +408,9 @@ def mode_core_flow(args, core):
         ctx.measure_correlation()
         ctx.finalize_step(float(p.cutoffs[w + 1]))
     ctx.set_state(float(p.cutoffs[0]), v2, v4)
-    flops = sum(evaluation_flops(p, p.cutoffs[k]) for k in range(steps))  # counted before the timed region
+    # counted before the timed region
+    flops = sum(evaluation_flops(p, p.cutoffs[k]) for k in range(steps))
+    work = sum(necessary_flops(p, p.cutoffs[k]) for k in range(steps))
     ctx.synchronize()
     ctx.profile(True)
     t0 = time.perf_counter()
@@ -415,7 +427,7 @@ def mode_core_flow(args, core):
     elapsed = time.perf_counter() - t0
     dg_ms, dg_n = ctx.profile_get(KERNEL_DGAMMA)
     ctx.close()
-    achieved = flops / (dg_ms * 1e-3) / 1e12
+    achieved = work / (dg_ms * 1e-3) / 1e12
     out = {"metric": "%s dGamma/dLambda evals/s (full-schedule average, FP64 flow)" % c["label"],
            "value": steps / elapsed,
            "unit": "evals/s", "n_gpus": 1, "steps": steps, "warmup": args.warmup,
@@ -427,7 +439,8 @@ def mode_core_flow(args, core):
                         "frac": achieved / FP64_PEAK_TFLOPS, "traffic": traffic_entry(c["workload"], "f64"),
                         "kernel": c["kernel"],
                         "launches": dg_n, "avg_launch_ms": dg_ms / max(dg_n, 1),
-                        "algorithmic_tflop_total": flops / 1e12},
+                        "work_tflop_total": work / 1e12, "algorithmic_tflop_total": flops / 1e12,
+                        "reference_tflops": flops / (dg_ms * 1e-3) / 1e12},
            "cpu_baseline": None}
     if not args.no_cpu_baseline:
         out["cpu_baseline"] = core_cpu_baseline(core, args.cpu_seconds)
@@ -505,7 +518,7 @@ def stratified_leg(prob, precision, steps, warmup, label):
     print("# %s: %d stratified steps %.3f s" % (label, steps, elapsed), file=sys.stderr, flush=True)
     est = full_schedule_seconds(step_flops, ks, t_steps)
     return dict(elapsed=elapsed, dg_ms=dg_ms, dg_n=dg_n, flops=float(sum(step_flops[k] for k in ks)),
-                est_full_s=est, indices=ks)
+                work=float(sum(necessary_flops(prob, prob.cutoffs[k]) for k in ks)), est_full_s=est, indices=ks)
 
 
 def cpu_model():
@@ -536,8 +549,8 @@ def square_leg(args):
     r = flow_leg(prob, SP_PRECISION_FP64, nsteps, 2, "square fp64")
     out = {"workload": "square-r4-nw32", "L": prob.L, "nw": prob.nw, "n_freq_triples": prob.n_freq,
            "cutoffs": len(prob.cutoffs), "gpu_evals_per_s": nsteps / r["elapsed"], "gpu_flow_s": r["elapsed"],
-           "gpu_k_dgamma_avg_ms": r["dg_ms"] / max(r["dg_n"], 1),
-           "gpu_tflops_k_dgamma": r["flops"] / (r["dg_ms"] * 1e-3) / 1e12}
+           "gpu_dgamma_avg_ms": r["dg_ms"] / max(r["dg_n"], 1),
+           "gpu_tflops_dgamma": r["work"] / (r["dg_ms"] * 1e-3) / 1e12}
     if not args.no_cpu_baseline:
         sys.path.insert(0, os.path.join(ROOT, "oracle"))
         from oracle import Oracle
@@ -572,10 +585,10 @@ def mode_flow(args):
         how = "whole flows from the first cutoff, %d evaluations timed" % args.steps
     elapsed = r64["elapsed"]
     # the whole FP64 flow through sp_run_flow, beside the headline; the roofline
-    # describes the dGamma kernel over this whole flow (the launches a profile of
+    # describes the dGamma kernels over this whole flow (the launches a profile of
     # the full-flow command averages over)
     full = r64 if not stratified else flow_leg(prob, SP_PRECISION_FP64, nsteps_flow, 0, "fp64 full flow")
-    achieved = full["flops"] / (full["dg_ms"] * 1e-3) / 1e12
+    achieved = full["work"] / (full["dg_ms"] * 1e-3) / 1e12
     traffic = traffic_entry(args.workload, "f64")
     avg_ms = full["dg_ms"] / max(full["dg_n"], 1)
     out = {
@@ -598,26 +611,27 @@ def mode_flow(args):
         "hbm_gbs_compulsory": compulsory_bytes(prob) / (avg_ms * 1e-3) / 1e9,
         "roofline": {"bound": "valu_fp64", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS, "traffic": traffic,
-                     "kernel": "k_su + k_t (dGamma)", "launches": full["dg_n"], "avg_launch_ms": avg_ms,
-                     "algorithmic_tflop_total": full["flops"] / 1e12,
+                     "kernel": DGAMMA_KERNELS, "launches": full["dg_n"], "avg_launch_ms": avg_ms,
+                     "work_tflop_total": full["work"] / 1e12, "algorithmic_tflop_total": full["flops"] / 1e12,
+                     "reference_tflops": full["flops"] / (full["dg_ms"] * 1e-3) / 1e12,
                      "peak_note": "MI355X FP64 vector FMA peak (equal to the FP64 matrix peak); the kernels are "
                                   "bound by their gathers, the lattice bubble runs on the matrix cores",
                      "window": "the whole flow (%d evaluations, HIP events on the context stream); traffic = "
-                               "mean HBM bytes per launch of the same flow (rocprofv3 FETCH_SIZE + WRITE_SIZE, "
-                               "scaled)" % nsteps_flow},
+                               "mean HBM bytes per evaluation of the same flow (rocprofv3 FETCH_SIZE + "
+                               "WRITE_SIZE, scaled)" % nsteps_flow},
         "cpu_baseline": None,
     }
     if traffic is not None:
         out["roofline"]["traffic_gbs"] = traffic / (avg_ms * 1e-3) / 1e9
     out["full_flow"] = {"evals_per_s": nsteps_flow / full["elapsed"] if stratified else value,
-                        "flow_s": full["elapsed"], "k_dgamma_avg_ms": avg_ms,
-                        "tflops_k_dgamma": achieved, "frac": achieved / FP64_PEAK_TFLOPS,
+                        "flow_s": full["elapsed"], "dgamma_avg_ms": avg_ms,
+                        "tflops_dgamma": achieved, "frac": achieved / FP64_PEAK_TFLOPS,
                         "loop": "sp_run_flow (steps queued, records read back every step, divergence checked "
                                 "on the device)"}
     if stratified:
         w_ms = r64["dg_ms"] / max(r64["dg_n"], 1)
-        out["timed_window"] = {"k_dgamma_avg_ms": w_ms, "launches": r64["dg_n"],
-                               "tflops_k_dgamma": r64["flops"] / (r64["dg_ms"] * 1e-3) / 1e12,
+        out["timed_window"] = {"dgamma_avg_ms": w_ms, "launches": r64["dg_n"],
+                               "tflops_dgamma": r64["work"] / (r64["dg_ms"] * 1e-3) / 1e12,
                                "cutoff_indices": r64["indices"]}
     if not args.no_step_api and not stratified:
         # the same flow with one ABI call per stage and step (the FrgCore call pattern)
@@ -637,7 +651,7 @@ def mode_flow(args):
             m = flow_leg(prob, SP_PRECISION_MIXED, args.steps, 0, "mixed")
             mrate = args.steps / m["elapsed"]
         r32 = m if not stratified else flow_leg(prob, SP_PRECISION_MIXED, nsteps_flow, 0, "mixed full flow")
-        mixed = {"evals_per_s": mrate, "k_dgamma_avg_ms": m["dg_ms"] / max(m["dg_n"], 1),
+        mixed = {"evals_per_s": mrate, "dgamma_avg_ms": m["dg_ms"] / max(m["dg_n"], 1),
                  "speedup_vs_fp64": mrate / value,
                  "full_flow_evals_per_s": nsteps_flow / r32["elapsed"] if stratified else mrate}
         if full["records"] and len(full["records"]) == len(r32["records"]):

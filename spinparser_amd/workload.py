@@ -84,6 +84,27 @@ def evaluation_flops(prob, cut: float) -> float:
     return prob.flops_per_evaluation(cs, ct, cu)
 
 
+def necessary_flops(prob, cut: float) -> float:
+    """Operations one evaluation cannot do without, for the rate a kernel reaches.
+
+    ``evaluation_flops`` counts what the reference's kernels do per integrand
+    call; the symmetries of the vertex leave less.  The S and U channels are images
+    of each other under the exchange of s and u, so one evaluation of the pair is
+    counted, and the two buffers of a T pair are images as well.  The lattice bubble
+    is linear in the products of site pairs: once per point as those products,
+    once per frequency triple as the sum over overlap entries."""
+    nw, L, overlap = len(prob.mesh), prob.L, prob.overlap_total
+    components = getattr(prob, "components", 2)
+    calls = float(channel_calls(prob.mesh, float(cut)).sum())
+    triples = nw * nw * (nw + 1) / 2.0
+    per_su = {2: 64.0 + 28.0, 4: 128.0 + 64.0, 16: 512.0 + 1024.0}[components] * L
+    per_t = {2: 32.0 + 16.0, 4: 64.0 + 64.0, 16: 256.0 + 1024.0}[components] * L
+    bubble = {2: 4.0 * L * L, 4: 20.0 * L * L, 16: min(128.0 * overlap, 512.0 * L * L)}[components]
+    t_points = calls * nw * (nw + 1) / 2.0
+    su_points = calls * nw * (nw + 1)
+    return su_points * per_su + t_points * (per_t + bubble) + triples * 2.0 * components * overlap
+
+
 def compulsory_bytes(prob, value_bytes: int = 8) -> int:
     """Read Gamma and Sigma, write dGamma and dSigma once per evaluation."""
     return 2 * (2 * prob.vertex_size + prob.nw) * value_bytes
