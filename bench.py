@@ -16,7 +16,7 @@ start; K = 655 is the full flow and yields the full-schedule average of
 dGamma/dLambda evaluations per second (``value``, FP64 form).  Beside it:
 
 * ``mixed``: the same flow in the mixed-precision form (FP32 frequency
-  integrals with compensated sums; FP64 state, Euler, self-energy and
+  integrals, their terms summed in FP64; FP64 state, Euler, self-energy and
   correlations), timed the same way, with the max-relative error against the
   FP64 flow of every output: correlations (every record), final state, and the
   derivative on a common state;

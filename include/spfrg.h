@@ -34,8 +34,9 @@ extern "C" {
 #define SP_ESTATE 4    /* call out of order (e.g. flow read before a step)     */
 
 #define SP_PRECISION_FP64 0   /* plain FP64 form                              */
-#define SP_PRECISION_MIXED 1  /* FP32 frequency integrals with compensated sums;
-                                 FP64 state, Euler step, self-energy, measurement */
+#define SP_PRECISION_MIXED 1  /* FP32 frequency integrals, their terms summed in FP64
+                                 (above 32 sites: compensated FP32 sums); FP64 state,
+                                 Euler step, self-energy, measurement            */
 
 /* Problem descriptor: the flattened lattice / mesh tables of one SU(2) flow.
  * Built host-side by the lattice factory; replaces what the reference reads

@@ -20,11 +20,16 @@
 //           kernel takes an array of them, so one launch serves one flow or a
 //           batch of resident flows of different sizes (the served sweep).
 //
-// Kernels (one derivative evaluation = k_dsigma, k_weights, k_dgamma):
-//   k_dsigma   one wavefront per (flow, mesh point); lanes split the range sum.
-//   k_weights  one thread per (flow, exact index): window points, coefficients.
-//   k_dgamma   one workgroup per (flow, frequency triple (s,t,u)): 256 threads,
-//              128 for lattices of at most 16 representative sites;
+// Kernels (one derivative evaluation = k_dsigma, k_weights, then k_su and k_t, or
+// k_dgamma):
+//   k_dsigma   one workgroup per (flow, mesh point): four waves split the range
+//              sum, a fifth evaluates the site-local values beside it.
+//   k_weights  one wave per (flow, exact index): window points, coefficients.
+//   k_su, k_t  (su2_rhs.h) dGamma of lattices of at most kMaxRhsL sites by
+//              independent waves; k_su32, k_t32 (su2_mixed.h) in the mixed form.
+//   k_dgamma   dGamma of larger lattices, and of sp_compute_step_noalloc calls into
+//              memory that takes no atomics: one workgroup per (flow, frequency
+//              triple (s,t,u)) of 256 threads (FP64, at most 16 sites: 128);
 //              blocks mapped to XCDs in contiguous item ranges.  The evaluation
 //              points of the three channels form one sequence of chunks; per chunk:
 //              (A) producer wave (the last wave), one lane per (point, pair of access
@@ -294,8 +299,8 @@ __global__ __launch_bounds__(kSigmaThreads) void k_dsigma(const FlowDev *__restr
 #include "su2_mixed.h"
 
 // ---------------------------------------------------------------------------
-// dGamma/dLambda, general kernel: the mixed form, and lattices of more than
-// kMaxRhsL sites
+// dGamma/dLambda, general kernel: lattices of more than kMaxRhsL sites in both
+// forms, and FP64 calls into memory that takes no atomics
 // ---------------------------------------------------------------------------
 // LDS carve-up (bytes), computed identically on host and device.  Lp = L
 // rounded up to a multiple of 4 (register tiles of the lattice-bubble update); vs =

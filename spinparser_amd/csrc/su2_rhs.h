@@ -31,14 +31,15 @@
 // Frequency arguments: the sums s +- t +- u of float mesh values are exact in
 // FP64, so regrouping them does not change any argument or bracket.
 //
-// What bounds it: a 16-byte gather of a wave costs the vector cache 16 to 17
-// cycles of its CU whatever its lanes and however near the data (measured, 1 to
-// 64 distinct rows, L1 or L2 hits), so the work was arranged to issue few of
+// What bounds it: a 16-byte gather of a wave costs the vector cache 16.8 cycles of
+// its CU where the lanes read whole cache lines, 21 with 19 neighbouring sites of
+// three rows, however near the data, so the work was arranged to issue few of
 // them with full lanes.  Every wave evaluates a unit of its own and describes
 // its own points, without barriers: no producer wave to wait for, and a unit's
 // points fill the wave.  Simple cubic J1-J2, 64 frequencies, 23 sites: one
 // evaluation 2.28 -> 0.99 ms at cutoff 60 and 9.80 -> 4.83 ms at cutoff 0.02
-// (k_su 2.56 ms, 84 % of the gather rate; k_t 2.15 ms) against one 256-thread
+// (k_su 2.56 ms, k_t 2.15 ms; over the whole flow the gathers of k_su take 94 % of
+// its time at 16.5 cycles each) against one 256-thread
 // workgroup per item with a producer wave; 31 sites, 45 frequencies at cutoff
 // 0.05: 3.0 -> 1.5 ms; square, 9 sites, 32 frequencies, whole flow 142 -> 87 ms.
 #pragma once

@@ -12,7 +12,9 @@
 //    raw(P l, P k) at the site inv_rid with the spin permutation P of inv_perm.
 //    This needs site_rid and site_perm to be identities and inv_rid a
 //    permutation, which every lattice of the factory has; other tables, and
-//    lattices of more than kMaxTriRhsL sites, run the general kernel.
+//    lattices of more than kMaxTriRhsL sites, run the general kernel.  So do
+//    lattices with more than 16 kTriMaxGroups products for each of eight waves
+//    (1,280; honeycomb-Kitaev at range 8 and 9, of 23 and 28 sites).
 //  * S and U add the 256 products of the components of two bundles, each output's
 //    sixteen terms summed first (k_tri_su).  As elements of H (x) H, 4 x 4 real
 //    matrices, the bundles would need 64 products, but sums and differences of
@@ -32,8 +34,8 @@
 //
 // Kagome with DM exchange, 19 sites, 48 frequencies, against one workgroup per
 // item that forms all terms point by point: 12.9 -> 5.5 ms at cutoff 20, 46.3 ->
-// 15.0 ms at 0.7, 81.9 -> 25.9 ms at 0.02 (k_tri_su 9.8 ms, bound by its gathers
-// and its vector instructions about equally; k_tri_t 15.8 ms, which
+// 15.0 ms at 0.7, 81.9 -> 25.9 ms at 0.02 (k_tri_su 9.8 ms, its vector instructions
+// 70 and its gathers 64 % of the cycles; k_tri_t 15.8 ms, which
 // alternates between gathers, 11 ms by themselves, and matrix products, 13 ms by
 // themselves: the descriptors of the next points are formed beside the products).
 #pragma once

@@ -94,7 +94,7 @@ using d4 = __attribute__((ext_vector_type(4))) double;
 // Update of a 16 x 16 matrix by four points: lane 16 k + r of a and b holds rows
 // (columns) r at point k.  Done by 4 x 4 x 4 matrix instructions, four blocks
 // each, b rotated by blocks: 17 cycles of a SIMD each where the 16 x 16 x 4
-// instruction takes 129 (measured 73 against 38 TFLOP/s).  c[z] of lane
+// instruction takes some 130 (measured 73 against 38 TFLOP/s).  c[z] of lane
 // 16 i + 4 b + j is the element (4 b + i, 4 ((b + z) % 4) + j).
 __device__ __forceinline__ double mfma_blocks(double a, double b, double c) {
   return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);

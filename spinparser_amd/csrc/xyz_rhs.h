@@ -11,12 +11,12 @@
 // This needs site_rid[r] = r and inv_rid to be an involution, which every
 // lattice of the factory has; other tables run the general kernels.
 //
-// What bounds it: the gathers (k_xyz_su: address unit 93 % busy), and in
-// k_xyz_t the alternation of gathers and matrix instructions (26 % of its
+// What bounds it: the gathers (k_xyz_su: 86 % of its time at 16.5 cycles each), and
+// in k_xyz_t the alternation of gathers (44 %) and matrix instructions (28 % of its
 // time) between barriers.  Honeycomb Heisenberg-Kitaev, 23 sites, 64
 // frequencies, against one workgroup per item with a producer wave: 8.78 ->
 // 3.86 ms at cutoff 20, 23.5 -> 10.2 ms at 0.7, 38.3 -> 15.6 ms at 0.02 (k_xyz_su
-// 6.1 ms, k_xyz_t 9.6 ms).
+// 6.1 ms, k_xyz_t 9.4 ms).
 #pragma once
 
 constexpr int kMaxXyzRhsL = 32;
