@@ -2101,7 +2101,7 @@ NoAllocPlan noalloc_plan(const sp_su2_problem *p, const NoAllocOverlap *wave) {
     q.plane = take(((size_t)p->L + 1) * 4);
     q.pcount = take((size_t)wave->lanes * 4);
   } else {
-    q.o1 = take(O * 4);
+    q.o1 = take(O * 4);  // (not filled: the documented limit counts them)
     q.o2 = take(O * 4);
     q.oidx = take(O * 2);
   }
